@@ -233,7 +233,7 @@ enum { NISE_HOST = 0, NISE_DEVICE = 1 };
  * polarisations, un-normalised, exactly what the reference accumulates.
  * kernel: 0 = frame-major batched kernel (default), 1 = plain
  * one-sample-per-launch kernel (baseline).  propagation 0 (exact
- * exponential, N <= 64) runs the DIA conveyor of nise_absorption_multi. */
+ * exponential, N <= 64) runs the dense-propagator kernel of nise_absorption_multi. */
 int nise_absorption_batched(const t_non *non, const float *H_rec,
                             int64_t H_stride, const float *mu_rec,
                             int64_t mu_stride, int64_t nframes,
@@ -406,7 +406,7 @@ typedef struct {
 /* Absorption of nsys independent systems of uneven size (no counterpart in
  * the reference; each system is what nise_absorption_batched computes).
  * Systems with propagation 1 share one row-conveyor launch; systems with
- * propagation 0 (exact exponential) and N <= 64 share one DIA-conveyor
+ * propagation 0 (exact exponential) and N <= 64 share one dense-propagator
  * launch fed by per-frame propagators from the batched Jacobi solver.
  * re_S / im_S (host) receive each system's tmax1 values, systems one after
  * another.  done_ms (host, nsys, optional) receives each system's

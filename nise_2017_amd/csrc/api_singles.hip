@@ -642,7 +642,7 @@ extern "C" int nise_absorption_batched(const t_non *non, const float *H_rec, int
                                        const float *mu_rec, int64_t mu_stride, int64_t nframes,
                                        const float *coupling_rec, int where, int kernel,
                                        float *re_S, float *im_S) {
-  if (non && non->propagation == 0) {  // exact exponential: the DIA conveyor
+  if (non && non->propagation == 0) {  // exact exponential: the dense propagators
     nise_system y{non, H_rec, H_stride, mu_rec, mu_stride, nframes, coupling_rec};
     return nise_absorption_multi(&y, 1, where, re_S, im_S, nullptr);
   }

@@ -3,11 +3,10 @@
 // Systems with propagation 1 (Trotter coupling scheme) run on the row
 // conveyor in one launch: every workgroup reads its own system descriptor,
 // so waves of different N share the launch.  Systems with propagation 0
-// (exact exponential, src/propagate.c:60-125) and N <= 64 run on the DIA
-// conveyor in a second launch: per frame U = exp(-i H f) is formed once
-// (FP64 Taylor series with scaling and squaring, rounded to FP32) and each
-// workgroup applies its frame's U, staged in LDS, to all its live vectors at
-// that frame.
+// (exact exponential, src/propagate.c:60-125) and N <= 64 run in a second
+// launch: per frame U = exp(-i H f) is formed once (FP64 Taylor series with
+// scaling and squaring, rounded to FP32) and dense_vectors_kernel applies it,
+// one wave per vector.
 //
 // Each workgroup records its start and end on the device wall clock; a
 // system's completion latency is the end of its last workgroup measured from
@@ -187,8 +186,8 @@ __device__ void trig_poly(const double Bv[4][4], const double *B2, double *X, co
 }
 
 // pairs = 0: U[m][a][b] row-major; pairs = 1: U[m][b / 2][a] as float4
-// (U_a,b, U_a,b+1), the second half zero past the last column (the DIA
-// conveyor's layout: one 16-byte read gives a site two columns).
+// (U_a,b, U_a,b+1), the second half zero past the last column (the layout
+// of dense.hip: one 16-byte read gives a site two columns).
 // One system's frames for expm_jobs_kernel; b is set by launch_expm_jobs.
 struct ExpmJob {
   FrameSource src;
@@ -440,179 +439,15 @@ int launch_dia_tables(const FrameSource &src, int N, int64_t f_first, int64_t nf
   return NISE_OK;
 }
 
-// One workgroup (256 threads): vectors v0 .. v0+vp-1 of one system (vp a
-// multiple of 3, so that the three polarisations of a sample share it).
-// Thread (site a, group sg) holds site a of vectors sg + j * (256 / Np),
-// j < kDiaVec, in registers while it applies U; each 16-byte LDS read gives
-// it two columns of U or two entries of one vector.  At frame f only the
-// vectors whose window [fs, fs + tmax) holds f do any work.
-constexpr int kDiaVec = 8;
-// vector rows of Np + 2 (even: 16-byte aligned) entries, so that the rows
-// read at once by the groups of a wave start in different banks
-__host__ __device__ inline int dia_pitch(int Np) { return (Np + 3) & ~1; }
-
-// psB[v] = U psA[v] at site a for the C vectors v = vb, vb + vs, ...: one
-// 16-byte read of U (two columns) serves all C of them.
-template <int C>
-__device__ __forceinline__ void dia_apply(const float4 *Ut, const float2 *psA, float2 *psB, int N, int Pr, int Ps,
-                                          int a, int vb, int vs) {
-  float2 y[C];
-#pragma unroll
-  for (int j = 0; j < C; ++j) y[j] = make_float2(0.f, 0.f);
-  for (int bp = 0; bp < Pr; ++bp) {
-    const float4 u = Ut[bp * N + a];
-#pragma unroll
-    for (int j = 0; j < C; ++j) {
-      const float4 c = *reinterpret_cast<const float4 *>(psA + (vb + j * vs) * Ps + 2 * bp);
-      y[j].x = fmaf(u.x, c.x, y[j].x);
-      y[j].x = fmaf(-u.y, c.y, y[j].x);
-      y[j].x = fmaf(u.z, c.z, y[j].x);
-      y[j].x = fmaf(-u.w, c.w, y[j].x);
-      y[j].y = fmaf(u.x, c.y, y[j].y);
-      y[j].y = fmaf(u.y, c.x, y[j].y);
-      y[j].y = fmaf(u.z, c.w, y[j].y);
-      y[j].y = fmaf(u.w, c.z, y[j].y);
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < C; ++j) psB[(vb + j * vs) * Ps + a] = y[j];
-}
-
-__global__ void __launch_bounds__(256) dia_conveyor_kernel(const DiaSys *sys, const int2 *wmap,
-                                                           unsigned long long *times) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const unsigned long long t_start = __builtin_amdgcn_s_memrealtime();
-  const int2 wm = wmap[blockIdx.x];
-  const DiaSys &S = sys[wm.x];
-  const int N = S.N, Np = S.Np, T = S.tmax, v0 = wm.y, Pr = (N + 1) >> 1, Ps = dia_pitch(Np);
-  const int nv = min(S.vp, S.nvec - v0);
-  const int groups = 256 / Np;
-  float4 *Ut = reinterpret_cast<float4 *>(smem);                // [Pr][N]
-  float2 *psA = reinterpret_cast<float2 *>(Ut + (size_t)Pr * N); // [vp][Np + 2]
-  float2 *psB = psA + (size_t)S.vp * Ps;                         // [vp][Np + 2]
-  double2 *acc = reinterpret_cast<double2 *>(psB + (size_t)S.vp * Ps);  // [T]
-  float2 *red = reinterpret_cast<float2 *>(acc + T);             // [vp]
-  const int t = threadIdx.x, a = t % Np, sg = t / Np;
-  for (int i = t; i < T; i += 256) acc[i] = make_double2(0.0, 0.0);
-  // entries past N stay zero: U's pad column meets a zero, never garbage
-  for (int i = t; i < 2 * S.vp * Ps; i += 256) psA[i] = make_float2(0.f, 0.f);
-  const int64_t s0 = S.begin + v0 / 3;  // first sample of the workgroup
-  const int nsamp = (nv + 2) / 3;
-  const int64_t F0 = s0 * S.sample, F1 = (s0 + nsamp - 1) * S.sample + T;
-  // U and the dipoles of the next frame in flight in registers while this
-  // frame works
-  const int nU = Pr * N;
-  constexpr int kUPer = (32 * 64 + 255) / 256;
-  float4 ureg[kUPer];
-  float mreg[3] = {0.f, 0.f, 0.f};
-  auto load_u = [&](int64_t f) {
-    const float4 *Uf = reinterpret_cast<const float4 *>(S.U) + (f - S.f_lo) * nU;
-#pragma unroll
-    for (int u = 0; u < kUPer; ++u)
-      if (t + u * 256 < nU) ureg[u] = gld(Uf + t + u * 256);
-    const float *mu = S.mu_rec + (S.mu_stride ? f * S.mu_stride : 0) + 1;
-    if (a < N)
-#pragma unroll
-      for (int x = 0; x < 3; ++x) mreg[x] = gld(mu + x * N + a);
-  };
-  load_u(F0);
-  __syncthreads();
-  for (int64_t f = F0; f < F1; ++f) {
-#pragma unroll
-    for (int u = 0; u < kUPer; ++u)
-      if (t + u * 256 < nU) Ut[t + u * 256] = ureg[u];
-    const float m3[3] = {mreg[0], mreg[1], mreg[2]};
-    if (f + 1 < F1) load_u(f + 1);
-    // vectors live at f: samples s0 + k with 0 <= f - (s0 + k) sample < T
-    const int64_t kf = (f - F0) / S.sample;  // last sample started
-    const int64_t klo = f - F0 - T < 0 ? 0 : (f - F0 - T) / S.sample + 1;
-    const int vlo = (int)(3 * klo), vhi = (int)min<int64_t>(nv, 3 * (kf + 1));
-    // this thread's live vectors: j in [jl, jh)
-    int jl = kDiaVec, jh = 0;
-#pragma unroll
-    for (int j = 0; j < kDiaVec; ++j) {
-      const int v = sg + j * groups;
-      if (v >= vlo && v < vhi) jl = min(jl, j), jh = j + 1;
-    }
-    // responses of the live vectors (and the dipole start of new ones); the
-    // site sums of all of them go through the lane butterfly together
-    float r[kDiaVec], q[kDiaVec];
-#pragma unroll
-    for (int j = 0; j < kDiaVec; ++j) {
-      r[j] = q[j] = 0.f;
-      const int v = sg + j * groups;
-      if (j < jl || j >= jh || a >= N) continue;
-      const float m = m3[v % 3];
-      float2 p;
-      if (f == (s0 + v / 3) * S.sample) {
-        p = make_float2(m, 0.f);
-        psA[v * Ps + a] = p;
-      } else {
-        p = psA[v * Ps + a];
-      }
-      r[j] = m * p.x, q[j] = m * p.y;
-    }
-    for (int off = 1; off < Np; off <<= 1)
-#pragma unroll
-      for (int j = 0; j < kDiaVec; ++j)
-        if (j >= jl && j < jh) r[j] += __shfl_xor(r[j], off), q[j] += __shfl_xor(q[j], off);
-    if (a == 0)
-#pragma unroll
-      for (int j = 0; j < kDiaVec; ++j)
-        if (j >= jl && j < jh) red[sg + j * groups] = make_float2(r[j], q[j]);
-    lds_barrier();
-    // responses into the accumulator, one thread per sample in polarisation
-    // order (samples of one workgroup sit at different delays at any frame)
-    if (t < nsamp) {
-      const int64_t rel = f - (s0 + t) * S.sample;
-      if (rel >= 0 && rel < T)
-        for (int x = 0; x < 3; ++x) {
-          const int v = 3 * t + x;
-          if (v < nv) acc[rel].x += (double)red[v].x, acc[rel].y += (double)red[v].y;
-        }
-    }
-    // psi <- U psi for the live vectors that go on (src/propagate.c:109-119)
-    int jlo = kDiaVec, jhi = 0;
-#pragma unroll
-    for (int j = 0; j < kDiaVec; ++j) {
-      const int v = sg + j * groups;
-      const bool go = v >= vlo && v < vhi && f - (s0 + v / 3) * S.sample < T - 1;
-      if (go) jlo = min(jlo, j), jhi = j + 1;
-    }
-    if (a < N && jlo < jhi) {
-      const int vb = sg + jlo * groups;
-      switch (jhi - jlo) {
-        case 1: dia_apply<1>(Ut, psA, psB, N, Pr, Ps, a, vb, groups); break;
-        case 2: dia_apply<2>(Ut, psA, psB, N, Pr, Ps, a, vb, groups); break;
-        case 3: dia_apply<3>(Ut, psA, psB, N, Pr, Ps, a, vb, groups); break;
-        case 4: dia_apply<4>(Ut, psA, psB, N, Pr, Ps, a, vb, groups); break;
-        case 5: dia_apply<5>(Ut, psA, psB, N, Pr, Ps, a, vb, groups); break;
-        case 6: dia_apply<6>(Ut, psA, psB, N, Pr, Ps, a, vb, groups); break;
-        case 7: dia_apply<7>(Ut, psA, psB, N, Pr, Ps, a, vb, groups); break;
-        default: dia_apply<8>(Ut, psA, psB, N, Pr, Ps, a, vb, groups); break;
-      }
-    }
-    lds_barrier();
-    float2 *tmp = psA;
-    psA = psB, psB = tmp;
-  }
-  const int w = v0 / S.vp;
-  for (int i = t; i < T; i += 256) gst(S.partial + (int64_t)w * T + i, acc[i]);
-  if (t == 0 && times) {
-    times[2 * blockIdx.x] = t_start;
-    times[2 * blockIdx.x + 1] = __builtin_amdgcn_s_memrealtime();
-  }
-}
-
-size_t dia_conveyor_smem(int N, int Np, int vp, int T) {
-  return (size_t)((N + 1) / 2) * N * 16 + (size_t)2 * vp * dia_pitch(Np) * 8 + (size_t)T * 16 + (size_t)vp * 8;
-}
-
-// Vectors per workgroup: kDiaVec per thread, whole samples, at most one
-// sample per thread (the accumulation step).
-int dia_vectors_per_group(int Np, int nvec) {
-  const int v = std::min(3 * 256, 3 * ((kDiaVec * (256 / Np)) / 3));
-  return std::max(3, std::min(v, 3 * ((nvec + 2) / 3)));
+// The longest window of a DIA system: the limit of the batch's earlier DIA
+// kernel, which held a sample's response and up to 24 vectors of Np rows in
+// 160 KB of LDS, kept as the entry point's range.
+static bool dia_window_fits(int N, int T, int nvec) {
+  int Np = 1;
+  while (Np < N) Np <<= 1;
+  const int v = std::min(3 * 256, 3 * ((8 * (256 / Np)) / 3)), vp = std::max(3, std::min(v, 3 * ((nvec + 2) / 3)));
+  return (size_t)((N + 1) / 2) * N * 16 + (size_t)2 * vp * ((Np + 3) & ~1) * 8 + (size_t)T * 16 + (size_t)vp * 8 <=
+         160 * 1024;
 }
 
 namespace {
@@ -786,12 +621,10 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
       J.U = s.U.as<float2>();
       jobs.push_back(J);
       DiaSys d;
-      d.N = N, d.Np = 1;
-      while (d.Np < N) d.Np <<= 1;
-      d.vp = dia_vectors_per_group(d.Np, s.nvec);
+      d.N = N;
       d.tmax = s.T, d.begin = non->begin, d.sample = non->sample, d.nvec = s.nvec, d.f_lo = s.f_lo;
       d.U = s.U.as<float2>(), d.mu_rec = s.mu_dev, d.mu_stride = s.mu_stride;
-      s.nwg = (s.nvec + d.vp - 1) / d.vp;
+      s.nwg = s.nvec;  // partial rows: one per vector
       if ((rc = s.partial.alloc((size_t)s.nwg * s.T * sizeof(double2)))) return rc;
       d.partial = s.partial.as<double2>();
       dias.push_back(d);
@@ -875,10 +708,10 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
       rows.push_back(r);
       rows_of.push_back(k);
   }
-  // 5. the two launches (row conveyor for all Trotter systems, DIA conveyor
+  // 5. the two launches (row conveyor for all Trotter systems, dense vectors
   //    for all DIA systems), timed on the device clock
   std::vector<int2> rmap, dmap;
-  size_t rsmem = 0, dsmem = 0;
+  size_t rsmem = 0;
   bool rpf = false;
   if (!rows.empty() && (rc = rows_prepare(rows.data(), (int)rows.size(), R, rmap, rsmem, rpf))) return rc;
   // longest workgroups first (layers x steps x Trotter substeps of their
@@ -888,10 +721,10 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
     return (int64_t)a.nlayers * a.tmax * a.m > (int64_t)b.nlayers * b.tmax * b.m;
   });
   for (size_t i = 0; i < dias.size(); ++i) {
-    dsmem = std::max(dsmem, dia_conveyor_smem(dias[i].N, dias[i].Np, dias[i].vp, dias[i].tmax));
-    for (int v = 0; v < dias[i].nvec; v += dias[i].vp) dmap.push_back(make_int2((int)i, v));
+    if (!dia_window_fits(dias[i].N, dias[i].tmax, dias[i].nvec))
+      return set_error("multi: DIA window of %d steps is too long for N=%d", dias[i].tmax, dias[i].N), NISE_ERR_ARG;
+    for (int v = 0; v < dias[i].nvec; v += 3) dmap.push_back(make_int2((int)i, v));
   }
-  if (dsmem > 160 * 1024) return set_error("multi: DIA conveyor needs %zu B of LDS", dsmem), NISE_ERR_ARG;
   DevBuf &rsys = cache.rsys, &rwm = cache.rwm, &dsys = cache.dsys, &dwm = cache.dwm, &times = cache.times;
   const size_t nt = rmap.size() + dmap.size();
   if ((rc = up(rsys, rows.data(), rows.size() * sizeof(RowsArgs))) ||
@@ -913,13 +746,7 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
   }
   if (!rmap.empty() && (rc = launch_rows(rsys.as<RowsArgs>(), rwm.as<int2>(), (int)rmap.size(), R, rpf, rsmem, st, tm)))
     return rc;
-  if (!dmap.empty()) {
-    NISE_HIP_CHECK(hipFuncSetAttribute((const void *)dia_conveyor_kernel,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)dsmem));
-    hipLaunchKernelGGL(dia_conveyor_kernel, dim3((unsigned)dmap.size()), dim3(256), dsmem, sd,
-                       dsys.as<DiaSys>(), dwm.as<int2>(), tm + 2 * rmap.size());
-    NISE_HIP_CHECK(hipGetLastError());
-  }
+  if ((rc = launch_dense_vectors(dsys.as<DiaSys>(), dwm.as<int2>(), (int)dmap.size(), sd, tm + 2 * rmap.size()))) return rc;
   // the reductions and copies below wait for the DIA stream
   {
     hipEvent_t ev;

@@ -423,16 +423,17 @@ int rows_prepare(const RowsArgs *sys, int nsys, int R, std::vector<int2> &wmap, 
 int launch_rows(const RowsArgs *sys, const int2 *wmap, int nwg, int R, bool pf, size_t smem, hipStream_t st,
                 unsigned long long *times = nullptr);
 
-// DIA conveyor (multi.hip): one descriptor per system, vp consecutive
-// vectors per 256-thread workgroup, Np = N rounded up to a power of two.
+// Dense-propagator vectors (dense.hip): one descriptor per system, one wave
+// per vector (vector v = 3 s + x as in RowsArgs).
 struct DiaSys {
-  int N = 0, Np = 1, vp = 1, tmax = 0, begin = 0, sample = 1, nvec = 0;
+  int N = 0, tmax = 0, begin = 0, sample = 1, nvec = 0;
   int64_t f_lo = 0;
-  const float2 *U = nullptr;     // [rows][N][N] per-frame propagators
+  const float2 *U = nullptr;     // [rows][(N + 1) / 2][N] column pairs (expm_per)
   const float *mu_rec = nullptr;
   int64_t mu_stride = 0;
-  double2 *partial = nullptr;    // [workgroups][tmax]
+  double2 *partial = nullptr;    // [vectors][tmax]
 };
+int launch_dense_vectors(const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t st, unsigned long long *times);
 // U = V exp(-i E f) V^T for nmat eigensystems (multi.hip); thres > 0 drops
 // the elements with FP32 |U_ab|^2 <= thres (the sparse scheme).
 int launch_dia_u(const double *w, const double *V, int N, int64_t nmat, float fac, float thres, float2 *U,
