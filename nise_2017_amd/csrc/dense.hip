@@ -76,7 +76,7 @@ __device__ __forceinline__ void dense_run(const DiaSys &S, int v, float2 *psi) {
       if ((i & 7) == 7) __builtin_amdgcn_sched_barrier(0);
     }
     p = make_float2(y0.x + y1.x, y0.y + y1.y);
-    if constexpr (G > 1) p = make_float2(stride_sum<(NP < 8 ? 8 : NP)>(p.x), stride_sum<(NP < 8 ? 8 : NP)>(p.y));
+    if constexpr (G > 1) p = make_float2(stride_sum<NP>(p.x), stride_sum<NP>(p.y));
   }
 }
 

@@ -33,10 +33,14 @@ __device__ __forceinline__ float group_sum(float x) {
   if constexpr (W > 32) x = add_xor32(x);
   return x;
 }
-// Sum over the lanes with the same lane % W (W a power of two >= 8), in every lane.
+// Sum over the lanes with the same lane % W (W a power of two), in every
+// lane: rotations of 8 and 4 lanes within a row keep lane % 4, then quads.
 template <int W>
 __device__ __forceinline__ float stride_sum(float x) {
   if constexpr (W <= 8) x += dpp_move<0x128>(x);  // row_ror:8
+  if constexpr (W <= 4) x += dpp_move<0x124>(x);  // row_ror:4
+  if constexpr (W <= 2) x += dpp_move<0x4E>(x);   // lane ^ 2
+  if constexpr (W <= 1) x += dpp_move<0xB1>(x);   // lane ^ 1
   if constexpr (W <= 16) x = add_xor16(x);
   if constexpr (W <= 32) x = add_xor32(x);
   return x;

@@ -35,6 +35,7 @@
 #include "nise_internal.h"
 #include "doubles_dev.h"
 #include "persist_dev.h"
+#include "twodir_basis.h"
 
 namespace nise {
 
@@ -969,6 +970,14 @@ extern "C" int nise_2dir_batched(const t_non *non, const float *H_rec, int64_t H
     for (int a = 0; a < N; ++a)
       for (int b = a + 1; b < N; ++b, ++p)
         if (mask[p]) lex.push_back((uint32_t)a | ((uint32_t)b << 16));
+  }
+  if (basis_path(non, (int)lex.size(), do_ea)) {
+    BasisCall c;
+    c.non = non, c.src = src, c.mask = mask, c.lex = lex;
+    c.end = end, c.do_gb = do_gb, c.do_se = do_se, c.do_ea = do_ea, c.es = es;
+    c.f_lo = f_lo, c.f_hi = f_hi, c.mu_rec = mud, c.mu_stride = ctype ? 0 : mu_stride;
+    c.anh_rec = Ad, c.over_rec = Od, c.st = st;
+    return run_basis(c, R12);
   }
   const float fac = trotter_factor(non->deltat, 1, non->ts);
   DevBuf &ab = B.ab, &lay = B.lay, &diag = B.diag, &cs = B.cs, &ab2 = B.ab2, &D2 = B.D2, &cs2 = B.cs2, &stp = B.stp;
