@@ -39,6 +39,10 @@ struct nise_abs_plan {
   int rows = 0;                // rows of the row conveyor, 0: slot conveyor
   DevBuf ab, layer_off, diag, cs, slots, wg_begin, partial, out, steps, row_steps, row_sys, row_wmap;
   size_t row_smem = 0;
+  bool packed = false;  // sch_rows is the packed schedule (pack_schedule_rows)
+  bool dense = false;   // per-frame propagators instead of the row conveyor (dense.hip)
+  RowsArgs row_desc;    // the uploaded descriptor
+  DevBuf U, dsys, dmap;
   bool row_pf = false;  // the row conveyor prefetches each frame's first site batch
   int nsteps = 0;
   DevBuf ws_cs, resp_plain;
@@ -80,6 +84,24 @@ int upload(DevBuf &dst, const void *src, size_t bytes, hipStream_t st) {
 
 bool is_coupling_type(const t_non *non) { return std::strcmp(non->hamiltonian, "Coupling") == 0; }
 
+// Descriptor, workgroup map and U of the dense propagators.
+int upload_dense(nise_abs_plan *P) {
+  const RowsArgs &r = P->row_desc;
+  DiaSys d;
+  d.N = r.N, d.tmax = r.tmax, d.begin = r.begin, d.sample = r.sample, d.nvec = r.nvec, d.f_lo = r.f_lo;
+  d.mu_rec = r.mu_rec, d.mu_stride = r.mu_stride, d.partial = r.partial;
+  d.hist = r.hist, d.hist_every = r.hist_every, d.nck = r.nck;
+  int rc;
+  if ((rc = P->U.alloc(dense_u_bytes(r.N, P->f_hi - P->f_lo)))) return rc;
+  d.U = P->U.as<float2>();
+  const int ns = P->end - P->begin;
+  P->nwg = ns, P->npart = r.N <= 64 ? 3 * ns : ns;
+  std::vector<int2> map(ns);
+  for (int s = 0; s < ns; ++s) map[s] = make_int2(0, r.N <= 64 ? 3 * s : s);
+  if ((rc = upload(P->dsys, &d, sizeof(d), P->st))) return rc;
+  return upload(P->dmap, map.data(), map.size() * sizeof(int2), P->st);
+}
+
 // Descriptor of the plan's single system for the row conveyor (device
 // copy and workgroup map; refreshed when checkpoints are switched on).
 int upload_rows_desc(nise_abs_plan *P) {
@@ -92,6 +114,8 @@ int upload_rows_desc(nise_abs_plan *P) {
   std::vector<int2> wmap;
   int rc = rows_prepare(&r, 1, P->rows, wmap, P->row_smem, P->row_pf);
   if (rc) return rc;
+  P->row_desc = r;
+  if (P->dense) return upload_dense(P);
   if ((rc = upload(P->row_sys, &r, sizeof(r), P->st))) return rc;
   return upload(P->row_wmap, wmap.data(), wmap.size() * sizeof(int2), P->st);
 }
@@ -158,6 +182,12 @@ int run_tables(nise_abs_plan *P) {
 }
 
 int run_conveyor(nise_abs_plan *P) {
+  if (P->dense) {
+    int rc = launch_rows_u(P->row_desc, P->rows, P->f_hi - P->f_lo, P->U.as<float2>(), P->st);
+    if (rc) return rc;
+    return (P->N <= 64 ? launch_dense_vectors : launch_dense_wide)(P->dsys.as<DiaSys>(), P->dmap.as<int2>(), P->nwg,
+                                                                   P->st, nullptr);
+  }
   if (P->rows)
     return launch_rows(P->row_sys.as<RowsArgs>(), P->row_wmap.as<int2>(), P->nwg, P->rows, P->row_pf, P->row_smem,
                        P->st);
@@ -338,8 +368,10 @@ static int plan_create(nise_abs_plan **out, const t_non *non, const float *H_rec
     // slot conveyor's shape (set_shape) stays available
     P->vp = 16, P->spw = 5;
     P->rows = rows_for(N, P->sch_asap.Kreal, P->sch_asap.nlayers());
-    build_schedule_rows(N, mask, P->rows, P->sch_rows);
     P->mask = mask;
+    P->dense = P->packed = dense_pays(N, P->tmax, P->end - P->begin, nfr, P->sch_asap.Kreal, P->sch_asap.nlayers(), P->m);
+    if (P->dense) pack_schedule_rows(P->sch_asap, P->rows, P->sch_rows);
+    else build_schedule_rows(N, mask, P->rows, P->sch_rows);
     if ((rc = build_slots(P))) return rc;
   }
   NISE_HIP_CHECK(hipStreamSynchronize(P->st));
@@ -375,7 +407,7 @@ extern "C" int nise_abs_plan_set_shape(nise_abs_plan *P, int vp, int samples_per
       !(block == 64 || block == 256 || block == 512 || block == -2 || block == -4) ||
       (block > 0 && vp > block))
     return set_error("bad shape vp=%d spw=%d block=%d", vp, samples_per_wg, block), NISE_ERR_ARG;
-  P->vp = vp, P->spw = samples_per_wg, P->block = block, P->rows = 0;
+  P->vp = vp, P->spw = samples_per_wg, P->block = block, P->rows = 0, P->dense = false;
   if (P->graph_ready) {
     (void)hipGraphExecDestroy(P->exec), (void)hipGraphDestroy(P->graph);
     P->exec = nullptr, P->graph = nullptr, P->graph_ready = false;
@@ -393,8 +425,8 @@ extern "C" int nise_abs_plan_set_rows(nise_abs_plan *P, int R) {
     return set_error("rows must be 1, 2, 4, 8, 16, 32 or 64, got %d", R), NISE_ERR_ARG;
   if (rows_smem(P->N, R) > 160 * 1024)
     return set_error("N=%d does not fit the row conveyor with %d rows", P->N, R), NISE_ERR_ARG;
-  if (R != P->rows || P->sch_rows.ab.empty()) build_schedule_rows(P->N, P->mask, R, P->sch_rows);
-  P->rows = R;
+  if (R != P->rows || P->packed || P->sch_rows.ab.empty()) build_schedule_rows(P->N, P->mask, R, P->sch_rows);
+  P->rows = R, P->dense = P->packed = false;
   if (P->graph_ready) {
     (void)hipGraphExecDestroy(P->exec), (void)hipGraphDestroy(P->graph);
     P->exec = nullptr, P->graph = nullptr, P->graph_ready = false;
@@ -561,6 +593,10 @@ extern "C" int nise_abs_plan_enable_adjoint(nise_abs_plan *P, int every) {
   if ((rc = P->ck.alloc((size_t)nslot * nck * N * sizeof(float2)))) return rc;
   if ((rc = P->jf.alloc((size_t)(P->f_hi - P->f_lo) * std::max(P->sch.K, 1) * 4))) return rc;
   P->every = every, P->nck = nck;
+  if (P->packed && P->rows) {  // the backward sweeps take the list schedule
+    build_schedule_rows(N, P->mask, P->rows, P->sch_rows);
+    P->packed = false;
+  }
   // backward grouping: consecutive slots, adj_vp per single-wave workgroup
   P->adj_vp = adjoint_vp(P->sch, N, T);
   std::vector<SlotDesc> sl;

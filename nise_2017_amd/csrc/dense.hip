@@ -1,5 +1,7 @@
-// Absorption vectors through dense per-frame propagators U (the exact
-// exponential, src/propagate.c:60-125): one wave per vector.
+// Absorption vectors through dense per-frame propagators U: the exact
+// exponential (src/propagate.c:60-125), and the Trotter scheme where a run has
+// too few vectors to fill the chip with sweeps (dense_pays).  N <= 64: one
+// wave per vector.
 //
 // What bounds it is the chain of tmax dependent steps: a batch has a few
 // hundred vectors, far fewer than the chip has wave slots, so a step's
@@ -14,6 +16,7 @@
 // earlier kernel, whose 256-thread workgroups walked the frames of 21 samples
 // with two barriers a frame (9 us each), 0.154 ms here.
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "lanes.h"
@@ -52,6 +55,10 @@ __device__ __forceinline__ void dense_run(const DiaSys &S, int v, float2 *psi) {
   float2 p = make_float2(m, 0.f);
   double2 *out = S.partial + (int64_t)v * T;
   for (int t = 0; t < T; ++t) {
+    if (S.hist) {  // checkpoint rows as the conveyor writes them (RowsArgs)
+      const int hr = t % S.hist_every == 0 ? t / S.hist_every : t == T - 1 ? t / S.hist_every + 1 : -1;
+      if (hr >= 0 && row && g == 0) gst(S.hist + ((int64_t)v * S.nck + hr) * N + a, p);
+    }
     // response mu(f).psi (src/absorption.c:205-212), summed over the rows
     const float rr = group_sum<NP>(row ? m * p.x : 0.f), ri = group_sum<NP>(row ? m * p.y : 0.f);
     if (lane == 0) gst(out + t, make_double2((double)rr, (double)ri));
@@ -109,12 +116,179 @@ dense_vectors_kernel(const DiaSys *sys, const int2 *wmap,
   }
 }
 
+// ---------------------------------------------------------------------------
+// N = 65 .. 128: one workgroup of eight waves per sample.  Lane (h, r) =
+// (lane / 32, lane % 32) of wave w holds rows r, r + 32, ... of the column
+// pairs 2 w + h, + 16, ... in registers and applies them to the sample's
+// three vectors, so each entry of U is loaded once per sample and step (a
+// wave per vector loads it three times: at N = 110 the L1 alone would take
+// 4,500 cycles a step).  The waves' partial sums meet in LDS, thread (x, a)
+// adds them and forms its part of the next response: two barriers a step.
+// ---------------------------------------------------------------------------
+constexpr int kWideWaves = 8, kWideSlices = 2 * kWideWaves;
+template <int RPL, int PPL>
+struct WideLds {
+  float2 psi[3][2 * kWideSlices * PPL];
+  float2 part[kWideWaves][3][32 * RPL];
+  float2 red[2][kWideWaves];
+};
+template <int RPL, int PPL>
+__device__ __forceinline__ void wide_run(const DiaSys &S, int s, unsigned char *smem) {
+  WideLds<RPL, PPL> &L = *reinterpret_cast<WideLds<RPL, PPL> *>(smem);
+  constexpr int NR = 32 * RPL;
+  const int N = S.N, T = S.tmax, Pr = (N + 1) >> 1, nU = Pr * N, tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, h = lane >> 5, r = lane & 31;
+  const int64_t fs = (int64_t)(S.begin + s) * S.sample;
+  // entries past N stay zero: U's pad column and the clamped pairs meet a zero
+  for (int i = tid; i < 3 * 2 * kWideSlices * PPL; i += 64 * kWideWaves) (&L.psi[0][0])[i] = make_float2(0.f, 0.f);
+  const float4 *U = reinterpret_cast<const float4 *>(S.U) + (fs - S.f_lo) * nU;
+  uint32_t po[PPL], ro[RPL];
+#pragma unroll
+  for (int i = 0; i < PPL; ++i) po[i] = (uint32_t)(min(2 * wave + h + kWideSlices * i, Pr - 1) * N);
+#pragma unroll
+  for (int k = 0; k < RPL; ++k) ro[k] = (uint32_t)min(r + 32 * k, N - 1);
+  float4 u[PPL][RPL];
+#pragma unroll
+  for (int i = 0; i < PPL; ++i)
+#pragma unroll
+    for (int k = 0; k < RPL; ++k) u[i][k] = gld(U + po[i] + ro[k]);
+  // thread (x, a): site a of polarisation x
+  const int x = tid / NR, a = tid - x * NR;
+  const bool own = x < 3 && a < N;
+  const float *mu = S.mu_rec + (S.mu_stride ? fs * S.mu_stride : 0) + 1 + (own ? (int64_t)x * N + a : 0);
+  float m = gld(mu);
+  float2 p = make_float2(own ? m : 0.f, 0.f);
+  __syncthreads();
+  double2 *out = S.partial + (int64_t)s * T;
+  for (int t = 0;; ++t) {
+    if (S.hist) {
+      const int hr = t % S.hist_every == 0 ? t / S.hist_every : t == T - 1 ? t / S.hist_every + 1 : -1;
+      if (hr >= 0 && own) gst(S.hist + ((int64_t)(3 * s + x) * S.nck + hr) * N + a, p);
+    }
+    // publish psi(t) and this wave's part of the response mu(f).psi
+    if (own) L.psi[x][a] = p;
+    const float rr = group_sum<64>(own ? m * p.x : 0.f), ri = group_sum<64>(own ? m * p.y : 0.f);
+    if (lane == 0) L.red[t & 1][wave] = make_float2(rr, ri);
+    __syncthreads();
+    if (tid == 0) {
+      double2 z = make_double2(0.0, 0.0);
+      for (int w = 0; w < kWideWaves; ++w) z.x += (double)L.red[t & 1][w].x, z.y += (double)L.red[t & 1][w].y;
+      gst(out + t, z);
+    }
+    if (t == T - 1) break;
+    mu += S.mu_stride;
+    m = gld(mu);
+    U += nU;  // the refills: frame fs + t + 1 <= fs + T - 1
+    float2 y[3][RPL];
+#pragma unroll
+    for (int v = 0; v < 3; ++v)
+#pragma unroll
+      for (int k = 0; k < RPL; ++k) y[v][k] = make_float2(0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < PPL; ++i) {
+      float4 c[3];
+#pragma unroll
+      for (int v = 0; v < 3; ++v)
+        c[v] = *reinterpret_cast<const float4 *>(&L.psi[v][2 * (2 * wave + h + kWideSlices * i)]);
+#pragma unroll
+      for (int k = 0; k < RPL; ++k) {
+        const float4 w = u[i][k];
+        u[i][k] = gld(U + po[i] + ro[k]);
+#pragma unroll
+        for (int v = 0; v < 3; ++v) {
+          float2 &z = y[v][k];
+          z.x = fmaf(w.x, c[v].x, z.x), z.y = fmaf(w.x, c[v].y, z.y);
+          z.x = fmaf(-w.y, c[v].y, z.x), z.y = fmaf(w.y, c[v].x, z.y);
+          z.x = fmaf(w.z, c[v].z, z.x), z.y = fmaf(w.z, c[v].w, z.y);
+          z.x = fmaf(-w.w, c[v].w, z.x), z.y = fmaf(w.w, c[v].z, z.y);
+        }
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 3; ++v)
+#pragma unroll
+      for (int k = 0; k < RPL; ++k) {
+        const float2 z = make_float2(add_xor32(y[v][k].x), add_xor32(y[v][k].y));
+        if (h == 0) L.part[wave][v][r + 32 * k] = z;
+      }
+    __syncthreads();
+    if (own) {
+      float2 q[kWideWaves];
+#pragma unroll
+      for (int w = 0; w < kWideWaves; ++w) q[w] = L.part[w][x][a];
+#pragma unroll
+      for (int st = 1; st < kWideWaves; st <<= 1)
+#pragma unroll
+        for (int w = 0; w < kWideWaves; w += 2 * st) q[w].x += q[w + st].x, q[w].y += q[w + st].y;
+      p = q[0];
+    }
+  }
+}
+
+// Workgroup: sample wmap.y of system wmap.x (N <= 128; N <= 64 pads).
+__global__ void __launch_bounds__(64 * kWideWaves) __attribute__((amdgpu_waves_per_eu(2)))
+dense_wide_kernel(const DiaSys *sys, const int2 *wmap, unsigned long long *times) {
+  __shared__ __align__(16) unsigned char smem[sizeof(WideLds<4, 4>)];
+  const unsigned long long t_start = __builtin_amdgcn_s_memrealtime();
+  const int2 wm = wmap[blockIdx.x];
+  const DiaSys S = sys[__builtin_amdgcn_readfirstlane(wm.x)];
+  const int s = __builtin_amdgcn_readfirstlane(wm.y);
+  if (S.N <= 64) wide_run<2, 2>(S, s, smem);
+  else if (S.N <= 96) wide_run<3, 3>(S, s, smem);
+  else wide_run<4, 4>(S, s, smem);
+  if (threadIdx.x == 0 && times) {
+    times[2 * blockIdx.x] = t_start;
+    times[2 * blockIdx.x + 1] = __builtin_amdgcn_s_memrealtime();
+  }
+}
+
 // sys / wmap: device copies, one workgroup per (system, sample), N <= 64.
 int launch_dense_vectors(const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t st, unsigned long long *times) {
   if (nwg == 0) return NISE_OK;
   hipLaunchKernelGGL(dense_vectors_kernel, dim3((unsigned)nwg), dim3(192), 0, st, sys, wmap, times);
   NISE_HIP_CHECK(hipGetLastError());
   return NISE_OK;
+}
+
+// sys / wmap: device copies, one workgroup per (system, sample), N <= 128;
+// partial holds one row per sample.
+int launch_dense_wide(const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t st, unsigned long long *times) {
+  if (nwg == 0) return NISE_OK;
+  hipLaunchKernelGGL(dense_wide_kernel, dim3((unsigned)nwg), dim3(64 * kWideWaves), 0, st, sys, wmap, times);
+  NISE_HIP_CHECK(hipGetLastError());
+  return NISE_OK;
+}
+
+// Whether a Trotter run goes through per-frame propagators instead of the row
+// conveyor: rotation sweeps on the N columns of every frame (independent of
+// each other) and one product per vector step, against rotation sweeps on
+// every vector step.  A conveyor wave walks tmax frames of nlayers dependent
+// LDS round trips, so runs with few waves are far from its throughput.  The
+// cycle counts are fits: measured (conveyor and this, ms) N = 16 chain, 200
+// samples 0.45 and 0.14; N = 77 lattice, 333 samples 2.66 and 1.09; N = 121
+// lattice, 600 samples 4.14 and 3.31; N = 64 lattice, 1,500 samples 2.74 and
+// 3.37 (conveyor); N = 100 lattice, 1,500 samples 4.12 (conveyor).
+// Kreal, nasap: rotations and layers of the layered schedule; m: Trotter
+// substeps; F: frames; S: samples.
+bool dense_pays(int N, int T, int64_t S, int64_t F, int Kreal, int nasap, int m) {
+  if (T > kDenseMaxT) return false;
+  if (N > kDenseMaxN || F >= (1 << 30) || (double)dense_u_bytes(N, F) > kDenseMaxBytes) return false;
+  const int R = rows_for(N, Kreal, nasap);
+  const double G = 64.0 / R, sweep = std::max({(double)nasap, (double)Kreal / R, 8.0}) * m;
+  // conveyor: a wave's frame is a chain of LDS round trips and its share of
+  // the sites; all waves together are bound by LDS instructions
+  const double site = 12.0 * N / R + 600.0, waves = 3.0 * S / G;
+  const double rows = T * std::max(sweep * 170.0 + site, waves / 256.0 * (sweep * 22.5 + site * 0.25));
+  const double build = F * std::ceil((N + (N & 1)) / G) / 256.0 * (sweep * 22.5 + 400.0) + 20000.0;
+  const double apply = N <= 64 ? T * std::max(700.0 + 20.0 * N, 3.0 * S / 1024.0 * (300.0 + 30.0 * N))
+                               : T * std::ceil(S / 256.0) * (1800.0 + 36.0 * N);
+  if (!(build + apply < 0.85 * rows)) return false;
+  // nise_absorption_batched_noalloc follows the same choice in windows of
+  // samples: a run that its array held with the conveyor's tables must hold
+  // one sample's window
+  const double K = std::max((double)nasap, (double)Kreal / R) * R * 1.1 + 8.0 * R;
+  const double part = 3.0 * S * T * 16 + K * 12 + S * 8 + 65536;
+  return F * (N + K) * 8 + part > kScratchBytes * 1.2 || T * ((N + K) * 8 + dense_u_bytes(N, 1)) + part < kScratchBytes * 0.9;
 }
 
 }  // namespace nise

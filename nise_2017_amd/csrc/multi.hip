@@ -460,6 +460,7 @@ int up(DevBuf &d, const void *s, size_t n) {
 
 struct SysState {
   int N = 0, T = 0, dia = 0, nvec = 0, nwg = 0;  // nwg: rows of partial responses
+  bool dense = false;  // Trotter system through per-frame propagators
   float thres = 0.f;  // sparse DIA threshold (0: full DIA)
   int64_t f_lo = 0, f_hi = 0;
   FrameSource src;
@@ -472,10 +473,12 @@ struct SysState {
   // (the row schedule's step table and frame-table order stay on the device)
   std::vector<uint8_t> asap_mask, rows_mask;
   int asap_N = 0, rows_R = 0, rows_N = 0;
+  bool rows_packed = false;
   // everything but the device buffers and the cached schedules, which the
   // next call reuses
   void reset() {
     N = T = dia = nvec = nwg = 0;
+    dense = false;
     thres = 0.f;
     f_lo = f_hi = 0;
     src = FrameSource();
@@ -665,13 +668,14 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
   // many couplings per layer take wide layers, which shortens the chain of
   // layers each of their workgroups walks)
   int R = 0, cap = kMultiRowCap;
+  bool own = R_force == 0 || R_force == -1;  // the default: systems that pay for it take the dense propagators
   std::vector<int64_t> sig;
   if (R_force == 0 && cache.tune_R != 0) batch_signature(systems, nsys, sig);
   if (R_force > 0) R = R_force;
   else if (R_force < -1) cap = -R_force;
   else if (R_force == 0 && cache.tune_R != 0 && sig == cache.tune_sig) {
-    if (cache.tune_R > 0) R = cache.tune_R;
-    else if (cache.tune_R < -1) cap = -cache.tune_R;
+    if (cache.tune_R > 0) R = cache.tune_R, own = false;
+    else if (cache.tune_R < -1) cap = -cache.tune_R, own = false;
   }
   // 4. tables of the Trotter systems
   for (int k = 0; k < nsys; ++k) {
@@ -681,9 +685,11 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
     const int64_t nfr = s.f_hi - s.f_lo;
     if (s.dia) continue;
       const int Rk = R > 0 ? R : rows_for(N, s.sch_asap.Kreal, s.sch_asap.nlayers(), cap);
-      if (s.rows_N != N || s.rows_R != Rk || s.rows_mask != s.mask) {
+      s.dense = own && dense_pays(N, s.T, s.nvec / 3, nfr, s.sch_asap.Kreal, s.sch_asap.nlayers(), non->ts);
+      if (s.rows_N != N || s.rows_R != Rk || s.rows_packed != s.dense || s.rows_mask != s.mask) {
         s.rows_N = 0;  // until the tables below are on the device
-        build_schedule_rows(N, s.mask, Rk, s.sch);
+        if (s.dense) pack_schedule_rows(s.sch_asap, Rk, s.sch);
+        else build_schedule_rows(N, s.mask, Rk, s.sch);
         std::vector<uint2> tab;
         rows_step_table(s.sch, Rk, tab);
         std::vector<uint32_t> abd;  // the frame tables follow the step table's order
@@ -691,13 +697,13 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
         if ((rc = up(s.ab, abd.data(), abd.size() * 4)) ||
             (rc = up(s.steps, tab.data(), tab.size() * sizeof(uint2))))
           return rc;
-        s.rows_mask = s.mask, s.rows_R = Rk, s.rows_N = N;
+        s.rows_mask = s.mask, s.rows_R = Rk, s.rows_N = N, s.rows_packed = s.dense;
       }
       if ((rc = s.diag.alloc((size_t)nfr * N * 8)) || (rc = s.cs.alloc((size_t)nfr * s.sch.K * 8))) return rc;
       if ((rc = launch_frame_tables(s.src, N, s.sch, s.ab.as<uint32_t>(), trotter_factor(non->deltat, 1, non->ts),
                                     s.f_lo, nfr, s.diag.as<float2>(), s.cs.as<float2>(), st)))
         return rc;
-      s.nwg = s.nvec;  // partial rows: one per vector
+      s.nwg = s.dense && N > 64 ? s.nvec / 3 : s.nvec;  // partial rows: one per vector or sample
       if ((rc = s.partial.alloc((size_t)s.nwg * s.T * sizeof(double2)))) return rc;
       RowsArgs r;
       r.N = N, r.tmax = s.T, r.m = non->ts, r.nlayers = s.sch.nlayers(), r.K = s.sch.K, r.f_lo = s.f_lo;
@@ -705,6 +711,15 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
       r.nvec = s.nvec, r.begin = non->begin, r.sample = non->sample;
       r.steps = s.steps.as<uint2>(), r.cs = s.cs.as<float2>(), r.diag = s.diag.as<float2>();
       r.mu_rec = s.mu_dev, r.mu_stride = s.mu_stride, r.partial = s.partial.as<double2>();
+      if (s.dense) {  // U of every frame now, the vectors with step 5
+        if ((rc = s.U.alloc(dense_u_bytes(N, nfr))) || (rc = launch_rows_u(r, Rk, nfr, s.U.as<float2>(), st))) return rc;
+        DiaSys d;
+        d.N = N, d.tmax = s.T, d.begin = non->begin, d.sample = non->sample, d.nvec = s.nvec, d.f_lo = s.f_lo;
+        d.U = s.U.as<float2>(), d.mu_rec = s.mu_dev, d.mu_stride = s.mu_stride, d.partial = r.partial;
+        dias.push_back(d);
+        dia_of.push_back(k);
+        continue;
+      }
       rows.push_back(r);
       rows_of.push_back(k);
   }
@@ -720,10 +735,23 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
     const RowsArgs &a = rows[x.x], &b = rows[y.x];
     return (int64_t)a.nlayers * a.tmax * a.m > (int64_t)b.nlayers * b.tmax * b.m;
   });
+  // dmap: vectors of the DIA systems (second stream), then of the Trotter
+  // systems' propagators up to 64 sites and above (first stream)
+  size_t dend[3];
+  for (int kind = 0; kind < 3; ++kind) {
+    for (size_t i = 0; i < dias.size(); ++i) {
+      const SysState &s = *S[dia_of[i]];
+      if (kind != (!s.dense ? 0 : s.N <= 64 ? 1 : 2)) continue;
+      if (kind == 2)
+        for (int v = 0; v < s.nvec / 3; ++v) dmap.push_back(make_int2((int)i, v));
+      else
+        for (int v = 0; v < s.nvec; v += 3) dmap.push_back(make_int2((int)i, v));
+    }
+    dend[kind] = dmap.size();
+  }
   for (size_t i = 0; i < dias.size(); ++i) {
-    if (!dia_window_fits(dias[i].N, dias[i].tmax, dias[i].nvec))
+    if (!S[dia_of[i]]->dense && !dia_window_fits(dias[i].N, dias[i].tmax, dias[i].nvec))
       return set_error("multi: DIA window of %d steps is too long for N=%d", dias[i].tmax, dias[i].N), NISE_ERR_ARG;
-    for (int v = 0; v < dias[i].nvec; v += 3) dmap.push_back(make_int2((int)i, v));
   }
   DevBuf &rsys = cache.rsys, &rwm = cache.rwm, &dsys = cache.dsys, &dwm = cache.dwm, &times = cache.times;
   const size_t nt = rmap.size() + dmap.size();
@@ -746,7 +774,13 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
   }
   if (!rmap.empty() && (rc = launch_rows(rsys.as<RowsArgs>(), rwm.as<int2>(), (int)rmap.size(), R, rpf, rsmem, st, tm)))
     return rc;
-  if ((rc = launch_dense_vectors(dsys.as<DiaSys>(), dwm.as<int2>(), (int)dmap.size(), sd, tm + 2 * rmap.size()))) return rc;
+  const DiaSys *dsp = dsys.as<DiaSys>();
+  const int2 *dmp = dwm.as<int2>();
+  unsigned long long *td = tm + 2 * rmap.size();
+  if ((rc = launch_dense_vectors(dsp, dmp, (int)dend[0], sd, td)) ||
+      (rc = launch_dense_vectors(dsp, dmp + dend[0], (int)(dend[1] - dend[0]), st, td + 2 * dend[0])) ||
+      (rc = launch_dense_wide(dsp, dmp + dend[1], (int)(dend[2] - dend[1]), st, td + 2 * dend[1])))
+    return rc;
   // the reductions and copies below wait for the DIA stream
   {
     hipEvent_t ev;

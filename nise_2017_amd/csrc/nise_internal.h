@@ -73,6 +73,10 @@ void build_schedule(int N, const std::vector<uint8_t> &mask, Schedule &s);
 // Row schedule: layers of exactly R entries (rotations, then dummy pairs
 // (N+q, N+q) in the unused rows q), for the row conveyor.
 void build_schedule_rows(int N, const std::vector<uint8_t> &mask, int R, Schedule &s);
+// A row schedule straight from the layered one (each of its layers cut into
+// rows of R): more layers, no list scheduling on the host; for sweeps that
+// are a small part of their run (the dense propagators).
+void pack_schedule_rows(const Schedule &asap, int R, Schedule &s);
 
 // Singles parameters shared by the frame-table kernels.
 struct FrameSource {
@@ -419,6 +423,8 @@ struct RowsArgs {
   int hist_every = 1, nck = 0;
 };
 int rows_prepare(const RowsArgs *sys, int nsys, int R, std::vector<int2> &wmap, size_t &smem, bool &pf);
+// U of every frame of the row tables (Trotter step propagators, DiaSys layout).
+int launch_rows_u(const RowsArgs &a, int R, int64_t nfr, float2 *U, hipStream_t st);
 // times (optional): per workgroup (start, end) on the device wall clock.
 int launch_rows(const RowsArgs *sys, const int2 *wmap, int nwg, int R, bool pf, size_t smem, hipStream_t st,
                 unsigned long long *times = nullptr);
@@ -431,8 +437,23 @@ struct DiaSys {
   const float2 *U = nullptr;     // [rows][(N + 1) / 2][N] column pairs (expm_per)
   const float *mu_rec = nullptr;
   int64_t mu_stride = 0;
-  double2 *partial = nullptr;    // [vectors][tmax]
+  double2 *partial = nullptr;    // [vectors][tmax] (N > 64: [samples][tmax])
+  float2 *hist = nullptr;        // checkpoints, as RowsArgs
+  int hist_every = 1, nck = 0;
 };
+// Trotter runs through propagators keep the reference's rounded rotation
+// coefficients but not its rounding of every product, which is biased where a
+// cosine is 1 - k 2^-24 (weak couplings): 0.4 to 1.2e-5 relative L2 apart after
+// 256 steps (closer to the 64-bit result), 2e-5 after 512, where the results are
+// to agree with the reference to 1e-5; longer windows keep the conveyor.
+constexpr int kDenseMaxN = 128, kDenseMaxT = 256;
+constexpr double kDenseMaxBytes = 1 << 30;  // of U
+constexpr size_t kScratchBytes = (size_t)32 << 20;  // noalloc.hip's array, per GPU
+bool dense_pays(int N, int T, int64_t S, int64_t F, int Kreal, int nasap, int m);
+inline size_t dense_u_bytes(int N, int64_t F) { return (size_t)F * 2 * ((N + 1) / 2) * N * 8; }
+// Workgroups: wmap entry (system, 3 * sample) for N <= 64 (launch_dense_vectors),
+// (system, sample) above (launch_dense_wide).
+int launch_dense_wide(const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t st, unsigned long long *times);
 int launch_dense_vectors(const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t st, unsigned long long *times);
 // U = V exp(-i E f) V^T for nmat eigensystems (multi.hip); thres > 0 drops
 // the elements with FP32 |U_ab|^2 <= thres (the sparse scheme).

@@ -18,6 +18,7 @@
 // vector's partial row and the reduction every output.  Calls on one GPU are
 // serialised by a per-device lock inside this process; launches of other
 // code that reuse the array concurrently would race with it.
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -30,7 +31,6 @@ int onfly_scheme(const t_non *non);  // api_singles.hip
 
 namespace {
 
-constexpr size_t kScratchBytes = (size_t)32 << 20;  // per GPU
 constexpr int kMaxDevices = 64;
 
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -84,6 +84,67 @@ int too_big(size_t need) {
             "(use nise_absorption_batched)",
             need, kScratchBytes);
   return NISE_ERR_RANGE;
+}
+
+// The run through per-frame propagators (dense.hip, the choice and kernels of
+// nise_abs_plan_create) in windows of as many samples as the array holds; a
+// sample's response depends on its own frames only, so the windows give the
+// plan's partial rows bit for bit.  r: the conveyor's descriptor (sizes and
+// inputs); the array is free from `used` on.
+int run_dense(unsigned char *base, size_t used, const FrameSource &src, RowsArgs r, const Schedule &asap, int R, int ns,
+              float fac, float *re_S, float *im_S) {
+  int rc;
+  const hipStream_t st = nullptr;
+  const int N = r.N, T = r.tmax, npart = N <= 64 ? 3 * ns : ns;
+  Schedule sch;
+  pack_schedule_rows(asap, R, sch);
+  std::vector<uint2> tab;
+  rows_step_table(sch, R, tab);
+  std::vector<uint32_t> ab;
+  rows_device_order(sch, R, ab);
+  Arena ar{base, used};
+  uint2 *steps = ar.take<uint2>(tab.size());
+  uint32_t *abd = ar.take<uint32_t>(ab.size());
+  double2 *partial = ar.take<double2>((size_t)npart * T);
+  float *out = ar.take<float>(2 * (size_t)T);
+  DiaSys *sysd = ar.take<DiaSys>(1);
+  int2 *mapd = ar.take<int2>(ns);
+  if (!steps || !abd || !partial || !out || !sysd || !mapd) return too_big(kScratchBytes + 1);
+  // samples per window: their frames' phases, rotations and U
+  auto frames = [&](int n) { return (int64_t)(n - 1) * r.sample + T; };
+  auto bytes = [&](int n) {
+    const size_t f = (size_t)frames(n);
+    return Arena::bytes_of(f * N, 8) + Arena::bytes_of(f * sch.K, 8) + Arena::bytes_of(dense_u_bytes(N, f), 1);
+  };
+  int per = ns;
+  while (per > 1 && ar.used + bytes(per) > kScratchBytes) per = per > 16 ? per * 7 / 8 : per - 1;
+  if (ar.used + bytes(per) > kScratchBytes) return too_big(ar.used + bytes(per));
+  NISE_HIP_CHECK(hipMemcpy(steps, tab.data(), tab.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  NISE_HIP_CHECK(hipMemcpy(abd, ab.data(), ab.size() * 4, hipMemcpyHostToDevice));
+  std::vector<int2> map(ns);
+  for (int s = 0; s < ns; ++s) map[s] = make_int2(0, N <= 64 ? 3 * s : s);
+  NISE_HIP_CHECK(hipMemcpy(mapd, map.data(), map.size() * sizeof(int2), hipMemcpyHostToDevice));
+  r.nlayers = sch.nlayers(), r.K = sch.K, r.steps = steps;
+  for (int s0 = 0; s0 < ns; s0 += per) {
+    const int n = std::min(per, ns - s0);
+    const int64_t f0 = (int64_t)(r.begin + s0) * r.sample, nf = frames(n);
+    Arena w{base, ar.used};
+    float2 *diag = w.take<float2>((size_t)nf * N), *cs = w.take<float2>((size_t)nf * sch.K);
+    float2 *U = reinterpret_cast<float2 *>(w.take<unsigned char>(dense_u_bytes(N, nf)));
+    if (!diag || !cs || !U) return too_big(kScratchBytes + 1);
+    if ((rc = launch_frame_tables(src, N, sch, abd, fac, f0, nf, diag, cs, st, nullptr))) return rc;
+    r.diag = diag, r.cs = cs, r.f_lo = f0;
+    if ((rc = launch_rows_u(r, R, nf, U, st))) return rc;
+    DiaSys d;
+    d.N = N, d.tmax = T, d.begin = r.begin + s0, d.sample = r.sample, d.nvec = 3 * n, d.f_lo = f0, d.U = U;
+    d.mu_rec = r.mu_rec, d.mu_stride = r.mu_stride, d.partial = partial + (size_t)(N <= 64 ? 3 * s0 : s0) * T;
+    NISE_HIP_CHECK(hipMemcpy(sysd, &d, sizeof(d), hipMemcpyHostToDevice));  // waits for the previous window
+    if ((rc = (N <= 64 ? launch_dense_vectors : launch_dense_wide)(sysd, mapd, n, st, nullptr))) return rc;
+  }
+  if ((rc = launch_reduce_partials(partial, npart, T, out, out + T, st))) return rc;
+  NISE_HIP_CHECK(hipMemcpy(re_S, out, T * sizeof(float), hipMemcpyDeviceToHost));
+  NISE_HIP_CHECK(hipMemcpy(im_S, out + T, T * sizeof(float), hipMemcpyDeviceToHost));
+  return NISE_OK;
 }
 
 }  // namespace
@@ -150,6 +211,7 @@ extern "C" int nise_absorption_batched_noalloc(const t_non *non, const float *H_
     ar.used = mark;  // the mask is on the host now
   }
 
+  const size_t ar0 = ar.used;  // the array from here on is the run's
   // the default row conveyor of nise_abs_plan_create
   Schedule asap, sch;
   build_schedule(N, mask, asap);
@@ -177,12 +239,6 @@ extern "C" int nise_absorption_batched_noalloc(const t_non *non, const float *H_
   RowsArgs *sysd = ar.take<RowsArgs>(1);
   int2 *wmapd = ar.take<int2>(nwg);
   if (!steps || !abd || !diag || !cs || !partial || !out || !sysd || !wmapd) return too_big(need);
-  if (!tab.empty()) NISE_HIP_CHECK(hipMemcpy(steps, tab.data(), tab.size() * sizeof(uint2), hipMemcpyHostToDevice));
-  if (!ab.empty()) NISE_HIP_CHECK(hipMemcpy(abd, ab.data(), ab.size() * 4, hipMemcpyHostToDevice));
-
-  // per-frame half-step phases and rotation tables (every entry written)
-  if ((rc = launch_frame_tables(src, N, sch, abd, trotter_factor(non->deltat, 1, m), f_lo, nfr, diag, cs, st, nullptr)))
-    return rc;
 
   RowsArgs r;
   r.N = N, r.tmax = T, r.m = m, r.nlayers = sch.nlayers(), r.K = sch.K, r.rows = R;
@@ -194,6 +250,14 @@ extern "C" int nise_absorption_batched_noalloc(const t_non *non, const float *H_
   bool pf = false;
   if ((rc = rows_prepare(&r, 1, R, wmap, smem, pf))) return rc;
   if ((int)wmap.size() != nwg) return set_error("row conveyor: workgroup map mismatch"), NISE_ERR_ARG;
+  if (dense_pays(N, T, end - begin, nfr, asap.Kreal, asap.nlayers(), m))
+    return run_dense(ds->ptr, ar0, src, r, asap, R, end - begin, trotter_factor(non->deltat, 1, m), re_S, im_S);
+  if (!tab.empty()) NISE_HIP_CHECK(hipMemcpy(steps, tab.data(), tab.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  if (!ab.empty()) NISE_HIP_CHECK(hipMemcpy(abd, ab.data(), ab.size() * 4, hipMemcpyHostToDevice));
+  // per-frame half-step phases and rotation tables (every entry written)
+  if ((rc = launch_frame_tables(src, N, sch, abd, trotter_factor(non->deltat, 1, m), f_lo, nfr, diag, cs, st, nullptr)))
+    return rc;
+
   NISE_HIP_CHECK(hipMemcpy(sysd, &r, sizeof(r), hipMemcpyHostToDevice));
   NISE_HIP_CHECK(hipMemcpy(wmapd, wmap.data(), wmap.size() * sizeof(int2), hipMemcpyHostToDevice));
   if ((rc = launch_rows(sysd, wmapd, nwg, R, pf, smem, st))) return rc;

@@ -409,6 +409,85 @@ __global__ void __launch_bounds__(64) rows_mixed_kernel(const RowsArgs *__restri
   }
 }
 
+// The Trotter step propagator U of one frame, G = 64 / R columns per wave
+// (the unit vectors through the frame's sweeps, all at the same frame), in the
+// column-pair layout of dense.hip.  Frames are independent, so unlike the
+// vectors' chains these fill the chip.  The rotations round as the
+// reference's: with a cosine of 1 - k 2^-24 (weak couplings, short steps) its
+// rounded product is biased, a drift of 2e-5 over 512 steps that fused
+// products do not have, and results are compared with the reference's.  Bound
+// by LDS instructions as the conveyor.
+template <int R>
+__global__ void __launch_bounds__(64) rows_u_kernel(RowsArgs A, float2 *U) {
+  constexpr int G = 64 / R, B = G < 4 ? G : 4, kRingS = kRingL / B;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int N = A.N, nl = A.nlayers, lane = threadIdx.x, q = lane / G, g = lane % G;
+  const int64_t row = blockIdx.x;
+  const int c = blockIdx.y * G + g;
+  const uint32_t gofs = (uint32_t)g * 8u;
+  const float2 *D = A.diag + row * N;
+  for (int i = lane; i < (N + R) * G; i += 64) reinterpret_cast<float2 *>(smem)[i] = make_float2(0.f, 0.f);
+  if (q == 0 && c < N) *reinterpret_cast<float2 *>(smem + ((uint32_t)c * G * 8u + gofs)) = gld(D + c);
+  const uint32_t loff = (uint32_t)(B * q + (lane & (B - 1)));
+  const float2 *csf = A.cs + row * A.K + loff;
+  const uint2 *stp = A.steps + loff;
+  auto rot = [&](uint2 e, float2 cc) { rot_step(smem, gofs, e, cc); };
+  for (int sub = 0; sub < A.m; ++sub) {
+    if (sub)
+      for (int i = q; i < N; i += R) {
+        const float2 d = gld(D + i);
+        float2 *pp = reinterpret_cast<float2 *>(smem + ((uint32_t)i * G * 8u + gofs));
+        *pp = cmul_diag(cmul_diag(*pp, d), d);
+      }
+    uint2 re[kRingS];
+    float2 rc[kRingS];
+#pragma unroll
+    for (int k = 0; k < kRingS; ++k) re[k] = gld(stp + B * k * R), rc[k] = gld(csf + B * k * R);
+    for (int b0 = 0; b0 < nl; b0 += kRingL) {
+      const int nx = b0 + kRingL < nl ? (b0 + kRingL) * R : 0;  // (the last block reads the first again)
+#pragma unroll
+      for (int k = 0; k < kRingS; ++k) {
+        const uint2 e = re[k];
+        const float2 cc = rc[k];
+        re[k] = gld(stp + nx + B * k * R), rc[k] = gld(csf + nx + B * k * R);
+        rot(make_uint2(grp_bcast<B, 0>(e.x), grp_bcast<B, 0>(e.y)), make_float2(grp_bcast<B, 0>(cc.x), grp_bcast<B, 0>(cc.y)));
+        if constexpr (B > 1)
+          rot(make_uint2(grp_bcast<B, 1>(e.x), grp_bcast<B, 1>(e.y)), make_float2(grp_bcast<B, 1>(cc.x), grp_bcast<B, 1>(cc.y)));
+        if constexpr (B > 2) {
+          rot(make_uint2(grp_bcast<B, 2>(e.x), grp_bcast<B, 2>(e.y)), make_float2(grp_bcast<B, 2>(cc.x), grp_bcast<B, 2>(cc.y)));
+          rot(make_uint2(grp_bcast<B, 3>(e.x), grp_bcast<B, 3>(e.y)), make_float2(grp_bcast<B, 3>(cc.x), grp_bcast<B, 3>(cc.y)));
+        }
+      }
+    }
+  }
+  const int Pr = (N + 1) >> 1;
+  float2 *Um = U + row * 2 * Pr * N;
+  if (c < 2 * Pr)  // an odd N's pad column holds zeros
+    for (int i = q; i < N; i += R) {
+      const float2 p = *reinterpret_cast<const float2 *>(smem + ((uint32_t)i * G * 8u + gofs));
+      gst(Um + ((int64_t)(c >> 1) * N + i) * 2 + (c & 1), cmul_diag(p, gld(D + i)));
+    }
+}
+
+int launch_rows_u(const RowsArgs &a, int R, int64_t nfr, float2 *U, hipStream_t st) {
+  const void *fn = R == 1 ? (const void *)rows_u_kernel<1> : R == 2 ? (const void *)rows_u_kernel<2>
+                 : R == 4 ? (const void *)rows_u_kernel<4> : R == 8 ? (const void *)rows_u_kernel<8>
+                 : R == 16 ? (const void *)rows_u_kernel<16> : R == 32 ? (const void *)rows_u_kernel<32>
+                 : R == 64 ? (const void *)rows_u_kernel<64> : nullptr;
+  if (!fn) return set_error("row propagators: unsupported row count %d", R), NISE_ERR_ARG;
+  if (a.nlayers < kRingL || a.nlayers % kRingL || a.K != (int64_t)a.nlayers * R)
+    return set_error("row propagators: schedule built for other rows"), NISE_ERR_ARG;
+  const size_t smem = rows_smem(a.N, R);
+  if (smem > 160 * 1024) return set_error("row propagators: %zu B of LDS needed", smem), NISE_ERR_ARG;
+  NISE_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+  RowsArgs A = a;
+  void *kargs[] = {&A, &U};
+  const int G = 64 / R;
+  NISE_HIP_CHECK(hipLaunchKernel(fn, dim3((unsigned)nfr, (unsigned)((a.N + (a.N & 1) + G - 1) / G)), dim3(64), kargs, smem,
+                                 st));
+  return NISE_OK;
+}
+
 size_t rows_smem(int N, int R) { return (size_t)(N + R) * (64 / R) * 8; }
 
 template <bool PF>

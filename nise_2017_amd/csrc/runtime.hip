@@ -215,6 +215,25 @@ void build_schedule_rows(int N, const std::vector<uint8_t> &mask, int R, Schedul
   }
 }
 
+void pack_schedule_rows(const Schedule &asap, int R, Schedule &s) {
+  constexpr int kMinLayers = 8;
+  const int N = asap.N;
+  s.N = N, s.Kreal = asap.Kreal;
+  s.ab.clear();
+  s.layer_off.assign(1, 0);
+  auto pad = [&]() {
+    for (int q = (int)s.ab.size() % R; q && q < R; ++q) s.ab.push_back((uint32_t)(N + q) | ((uint32_t)(N + q) << 16));
+  };
+  for (int l = 0; l < asap.nlayers(); ++l) {
+    s.ab.insert(s.ab.end(), asap.ab.begin() + asap.layer_off[l], asap.ab.begin() + asap.layer_off[l + 1]);
+    pad();
+  }
+  while (s.ab.empty() || s.ab.size() % ((size_t)R * kMinLayers))
+    for (int q = 0; q < R; ++q) s.ab.push_back((uint32_t)(N + q) | ((uint32_t)(N + q) << 16));
+  s.K = (int)s.ab.size();
+  for (int k = R; k <= s.K; k += R) s.layer_off.push_back(k);
+}
+
 static std::once_flag g_dev_once;
 static int g_dev_status = NISE_OK;
 

@@ -1,4 +1,4 @@
-"""The dense-propagator kernel (one wave per vector, exact exponential) at
+"""The dense-propagator kernels: the exact exponential (one wave per vector) at
 the edges of its row and column classes, against the oracle: site counts on
 both sides of every class boundary, windows of one and two steps, one sample
 and a sample count that leaves no full workgroup pattern.  Tolerance 1e-5
@@ -7,7 +7,7 @@ exponential)."""
 import numpy as np
 import pytest
 
-from nise_2017_amd import abi
+from nise_2017_amd import abi, synth
 
 from test_gpu_multi import rel, system
 
@@ -25,3 +25,111 @@ def test_class_edges(orc, T, ns, sr):
         e = rel(re + 1j * im, o_re + 1j * o_im)
         assert e < 1e-5, (non.singles, e)
     assert np.isfinite(out[-1][0]).all()
+
+
+def lattice_case(N, T, ns, sr, seed, ts=1, begin=0, **kw):
+    """N sites of a dipole lattice, Full records."""
+    L = int(np.ceil(np.sqrt(N)))
+    rng, mus, coup = synth.lattice_static(L, seed=seed)
+    nfr = (begin + ns - 1) * sr + T + 2
+    H = synth.full_records(synth.lattice_diag(rng, nfr, L * L), coup)
+    a, b = np.triu_indices(L * L)
+    keep = (a < N) & (b < N)
+    H = np.ascontiguousarray(np.concatenate([H[:, :1], H[:, 1:][:, keep]], axis=1))
+    mu = synth.dipole_records(mus[:N], nfr)
+    lo, hi = synth.shifted_center(H, N)
+    non = abi.make_non(singles=N, tmax1=T, sample=sr, begin=begin, end=begin + ns, ts=ts, propagation=1, deltat=2.0,
+                       min1=lo, max1=hi, **kw)
+    non.shifte = np.float32((np.float32(hi) + np.float32(lo)) / np.float32(2))
+    return non, H, mu
+
+
+def both(non, H, mu, C=None):
+    """The default plan (checked to run one workgroup per sample) and the row
+    conveyor on the same records."""
+    p = abi.AbsPlan(non, H, H.shape[1], mu, mu.shape[1], H.shape[0], C)
+    try:
+        assert p.info()["nwg"] == non.end - non.begin
+        dense = p.execute()
+        graph = [p.execute(flags=2) for _ in range(3)]
+        p.set_rows(0)
+        rows = p.execute()
+    finally:
+        p.close()
+    for g in graph:
+        assert np.array_equal(g[0], dense[0]) and np.array_equal(g[1], dense[1])
+    return dense[0] + 1j * dense[1], rows[0] + 1j * rows[1]
+
+
+@pytest.mark.parametrize("N,T,ns,sr,ts,begin", [
+    (65, 40, 9, 3, 1, 0), (95, 33, 4, 5, 2, 1), (96, 24, 5, 30, 1, 0), (97, 40, 7, 4, 1, 2), (127, 30, 3, 2, 1, 0),
+    (128, 41, 8, 3, 2, 0), (64, 64, 10, 4, 1, 3), (33, 50, 7, 5, 2, 0), (5, 64, 6, 7, 1, 0), (66, 2, 3, 1, 1, 0)])
+def test_trotter_propagators_against_conveyor(orc, N, T, ns, sr, ts, begin):
+    """The Trotter scheme through per-frame propagators against the row
+    conveyor and the oracle: both sides of every row class, odd N, Trotter
+    substeps, samples that do not start at frame 0, windows with gaps, graph
+    replays.  1e-5 as for the conveyor (the propagators' own rounding is far
+    below over these windows)."""
+    non, H, mu = lattice_case(N, T, ns, sr, seed=800 + N, ts=ts, begin=begin)
+    print(f"[dense] Trotter N={N} T={T}", flush=True)
+    d, r = both(non, H, mu)
+    assert rel(d, r) < 1e-5
+    o_re, o_im = orc.absorption(non, H, mu)
+    assert rel(d, o_re + 1j * o_im) < 1e-5
+
+
+def test_trotter_propagators_coupling_type_and_shifts():
+    """Coupling type with static dipoles, single-site shifts, host and device records."""
+    import torch
+    N, T, ns = 70, 30, 6
+    non, H, mu = lattice_case(N, T, ns, 4, seed=870, hamiltonian="Coupling", couplingcut=0.2,
+                              single_shift=[(3, 1.0, 25.0), (69, 0.9, -4.0)])
+    a, b = np.triu_indices(N)
+    Hc = np.ascontiguousarray(np.concatenate([H[:, :1], H[:, 1:][:, a == b]], axis=1))
+    Cr, muc = np.ascontiguousarray(H[0]), np.ascontiguousarray(mu[:1])
+    d, r = both(non, Hc, muc, Cr)
+    assert rel(d, r) < 1e-5
+    x = [torch.from_numpy(v).cuda() for v in (Hc, muc, Cr)]
+    torch.cuda.synchronize()
+    p = abi.AbsPlan(non, x[0], Hc.shape[1], x[1], muc.shape[1], Hc.shape[0], x[2], where=abi.NISE_DEVICE)
+    re, im = p.execute()
+    p.close()
+    assert np.array_equal(re + 1j * im, d)
+
+
+@pytest.mark.parametrize("N", [40, 90])
+def test_noalloc_windows_match_plan(N):
+    """A run whose propagators exceed the fixed scratch array: windows of
+    samples, bit for bit the plan's result."""
+    import ctypes as C
+
+    import torch
+    T, ns, sr = 60, 90 if N == 90 else 200, 14
+    non, H, mu = lattice_case(N, T, ns, sr, seed=880 + N)
+    Hd, mud = torch.from_numpy(H).cuda(), torch.from_numpy(mu).cuda()
+    torch.cuda.synchronize()
+    p = abi.AbsPlan(non, Hd, H.shape[1], mud, mu.shape[1], H.shape[0], where=abi.NISE_DEVICE)
+    assert p.info()["nwg"] == ns
+    re, im = p.execute()
+    p.close()
+    r1, i1 = np.zeros(T, np.float32), np.zeros(T, np.float32)
+    abi.check(abi.lib().nise_absorption_batched_noalloc(C.byref(non), abi.ptr(Hd), H.shape[1], abi.ptr(mud), mu.shape[1],
+                                                        H.shape[0], None, r1, i1))
+    assert np.array_equal(re, r1) and np.array_equal(im, i1)
+
+
+def test_gradient_from_propagator_checkpoints(orc):
+    """The adjoint from checkpoints that the propagator kernels wrote (N <= 64
+    and above), against the conveyor's."""
+    from nise_2017_amd import adjoint
+    for N in (20, 70):
+        non, H, mu = lattice_case(N, 40, 6, 5, seed=890 + N)
+        g = np.linspace(1.0, -0.5, 40)
+        got = []
+        for rows in (None, 4):
+            m = adjoint.AdjointAbsorption(non, H, mu, every=7, rows=rows)
+            m.forward(np.full(N, 0.5, np.float32), 1.02)
+            gd, gc = m.backward(g, g[::-1].copy())
+            got.append(np.concatenate([gd, [gc]]))
+            m.close()
+        assert rel(got[0], got[1]) < 1e-4
