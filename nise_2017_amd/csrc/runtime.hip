@@ -70,67 +70,124 @@ void build_schedule(int N, const std::vector<uint8_t> &mask, Schedule &s) {
     s.ab[fill[lay[k]]++] = (uint32_t)la[k] | ((uint32_t)lb[k] << 16);
 }
 
-// LDS bank cost of a layer's row order e[0..R) (padding rows ~0u stand for
-// the row's scratch site N + q): a row's G vectors occupy 2G consecutive
+// LDS bank cost of a layer's row order: a row's G vectors occupy 2G consecutive
 // dwords, so in B banks its run falls in block slot mod (B / 2G); per group
 // of lanes the busiest block bounds the passes of an access.  The grouping
 // the hardware uses for 8-byte accesses is not pinned here, so the cost is
 // summed over 32-lane groups on 64 banks and 16-lane groups on 32 banks
 // (a grouping of all 64 lanes does not depend on the row order).
 struct BankModel {
-  int nblk, rpg;  // blocks, rows per lane group
+  int nblk = 0, rpg = 0;  // blocks, rows per lane group
 };
-static int group_cost(const uint32_t *e, int g0, int rpg, int nblk, int N, int R) {
-  int cost = 0;
-  for (int side = 0; side < 2; ++side) {
-    int cnt[64], mx = 0;
-    for (int k = 0; k < nblk; ++k) cnt[k] = 0;
-    for (int q = g0; q < std::min(R, g0 + rpg); ++q) {
-      const int slot = e[q] == ~0u ? N + q : side ? (int)(e[q] >> 16) : (int)(e[q] & 0xffffu);
-      mx = std::max(mx, ++cnt[slot & (nblk - 1)]);
-    }
-    cost += mx;
-  }
-  return cost;
-}
 
 // Rotations of one layer touch disjoint sites, so their order across the R
-// rows is free: passes of pairwise swaps between lane groups lower the
-// layer's bank cost (a swap changes only the two groups it touches).
-static void assign_rows(std::vector<uint32_t> &e, int R, int N) {
-  const int G = 64 / R;
+// rows is free.  Each of the layer's n rotations goes to the lane group (of
+// the finer model; a coarser group holds whole finer ones) where it raises the
+// busiest blocks least, ties to the emptiest group; then one pass of swaps
+// between groups lowers the cost, only of entries in a busiest block and with
+// each swap's gain read from the block counts.  (Four passes over all pairs,
+// each swap evaluated over its groups' rows, took 90% of a schedule's time for
+// a cost 1% lower: N = 256 lattice, R = 16, 22 ms against 5 and cost 5,795
+// against 5,855; N = 384, R = 32, 94 ms against 13 and 4,663 against 4,675.)
+struct LayerBanks {
+  int nm = 0, fine = 1, R = 1;
   BankModel bm[2];
-  int nm = 0;
-  for (const auto &m : {std::make_pair(64, 32), std::make_pair(32, 16)}) {
-    const int span = 2 * G, rpg = std::max(1, m.second / G);
-    if (span <= m.first && rpg < R) bm[nm++] = BankModel{m.first / span, rpg};
+  uint8_t cnt[2][2][64][64];  // [model][side][group][block] entries
+  uint8_t hist[2][2][64][66]; // [..][count] blocks that hold so many
+  uint8_t top[2][2][64];      // the busiest block's count
+  int group(int k, int row) const { return row / bm[k].rpg; }
+  int block(int k, int d, uint32_t e) const { return (int)(d ? e >> 16 : e & 0xffffu) & (bm[k].nblk - 1); }
+  void init(int R_) {
+    R = R_, nm = 0;
+    const int G = 64 / R;
+    for (const auto &m : {std::make_pair(64, 32), std::make_pair(32, 16)}) {
+      const int span = 2 * G, rpg = std::max(1, m.second / G);
+      if (span <= m.first && rpg < R) bm[nm].nblk = m.first / span, bm[nm++].rpg = rpg;
+    }
+    if (nm) fine = bm[nm - 1].rpg;
   }
-  if (!nm) return;
-  for (int pass = 0; pass < 4; ++pass) {
-    bool improved = false;
-    for (int i = 0; i < R; ++i)
-      for (int j = i + 1; j < R; ++j) {
-        if (e[i] == ~0u && e[j] == ~0u) continue;
-        int before = 0, after = 0;
-        for (int k = 0; k < nm; ++k) {
-          const int gi = i / bm[k].rpg * bm[k].rpg, gj = j / bm[k].rpg * bm[k].rpg;
-          if (gi != gj)
-            before += group_cost(e.data(), gi, bm[k].rpg, bm[k].nblk, N, R) +
-                      group_cost(e.data(), gj, bm[k].rpg, bm[k].nblk, N, R);
+  void clear() {
+    for (int k = 0; k < nm; ++k)
+      for (int d = 0; d < 2; ++d)
+        for (int g = 0; g < R / bm[k].rpg; ++g) {
+          std::memset(cnt[k][d][g], 0, bm[k].nblk);
+          std::memset(hist[k][d][g], 0, sizeof(hist[k][d][g]));
+          hist[k][d][g][0] = (uint8_t)bm[k].nblk, top[k][d][g] = 0;
         }
-        if (!before) continue;
-        std::swap(e[i], e[j]);
-        for (int k = 0; k < nm; ++k) {
-          const int gi = i / bm[k].rpg * bm[k].rpg, gj = j / bm[k].rpg * bm[k].rpg;
-          if (gi != gj)
-            after += group_cost(e.data(), gi, bm[k].rpg, bm[k].nblk, N, R) +
-                     group_cost(e.data(), gj, bm[k].rpg, bm[k].nblk, N, R);
-        }
-        if (after < before) improved = true;
-        else std::swap(e[i], e[j]);
+  }
+  void add(int row, uint32_t e, int by) {
+    for (int k = 0; k < nm; ++k)
+      for (int d = 0; d < 2; ++d) {
+        const int g = group(k, row);
+        uint8_t &c = cnt[k][d][g][block(k, d, e)], *h = hist[k][d][g];
+        --h[c], c = (uint8_t)(c + by), ++h[c];
+        uint8_t &t = top[k][d][g];
+        if (c > t) t = c;
+        while (t && !h[t]) --t;
       }
-    if (!improved) break;
   }
+  // the group's top with entry `out` replaced by `in` (~0u: none)
+  int top_after(int k, int d, int g, uint32_t out, uint32_t in) const {
+    int t = top[k][d][g];
+    const uint8_t *c = cnt[k][d][g];
+    const int bo = out == ~0u ? -1 : block(k, d, out), bi = in == ~0u ? -1 : block(k, d, in);
+    if (bo == bi) return t;
+    if (bo >= 0 && c[bo] == t && hist[k][d][g][t] == 1) --t;
+    return bi >= 0 ? std::max(t, c[bi] + 1) : t;
+  }
+  bool hot(int row, uint32_t e) const {
+    for (int k = 0; k < nm; ++k)
+      for (int d = 0; d < 2; ++d) {
+        const int g = group(k, row), t = top[k][d][g];
+        if (t > 1 && cnt[k][d][g][block(k, d, e)] == t) return true;
+      }
+    return false;
+  }
+};
+static void assign_rows(LayerBanks &B, std::vector<uint32_t> &e, int n) {
+  if (!B.nm) return;
+  const int R = B.R, ng = R / B.fine;
+  int used[64] = {};
+  uint32_t out[64];
+  for (int q = 0; q < R; ++q) out[q] = ~0u;
+  B.clear();
+  for (int i = 0; i < n; ++i) {
+    int best = -1, bc = 0;
+    for (int f = 0; f < ng; ++f) {
+      if (used[f] == B.fine) continue;
+      int c = 0;
+      for (int k = 0; k < B.nm; ++k) {
+        const int g = B.group(k, f * B.fine);
+        for (int d = 0; d < 2; ++d) c += B.cnt[k][d][g][B.block(k, d, e[i])] >= B.top[k][d][g];
+      }
+      c = c * 64 + used[f];
+      if (best < 0 || c < bc) best = f, bc = c;
+    }
+    const int row = best * B.fine + used[best]++;
+    out[row] = e[i];
+    B.add(row, e[i], 1);
+  }
+  for (int i = 0; i < R; ++i) {
+    if (out[i] == ~0u || !B.hot(i, out[i])) continue;
+    for (int j = 0; j < R; ++j) {
+      if (j / B.fine == i / B.fine) continue;
+      int gain = 0;
+      for (int k = 0; k < B.nm; ++k) {
+        const int gi = B.group(k, i), gj = B.group(k, j);
+        if (gi == gj) continue;
+        for (int d = 0; d < 2; ++d)
+          gain += B.top[k][d][gi] + B.top[k][d][gj] - B.top_after(k, d, gi, out[i], out[j]) -
+                  B.top_after(k, d, gj, out[j], out[i]);
+      }
+      if (gain <= 0) continue;
+      B.add(i, out[i], -1);
+      if (out[j] != ~0u) B.add(j, out[j], -1), B.add(i, out[j], 1);
+      B.add(j, out[i], 1);
+      std::swap(out[i], out[j]);
+      break;
+    }
+  }
+  e.assign(out, out + R);
 }
 
 // Layers of at most R rotations by list scheduling on the dependency graph
@@ -206,9 +263,11 @@ void build_schedule_rows(int N, const std::vector<uint8_t> &mask, int R, Schedul
   s.ab.clear();
   s.layer_off.assign(1, 0);
   std::vector<uint32_t> e(R);
+  static thread_local LayerBanks banks;
+  if (R >= 4 && R <= 64) banks.init(R);
   for (auto &L : layers) {
     for (int q = 0; q < R; ++q) e[q] = q < (int)L.size() ? L[q] : ~0u;
-    if (R >= 4 && R <= 64) assign_rows(e, R, N);
+    if (R >= 4 && R <= 64) assign_rows(banks, e, (int)L.size());
     for (int q = 0; q < R; ++q)
       s.ab.push_back(e[q] != ~0u ? e[q] : (uint32_t)(N + q) | ((uint32_t)(N + q) << 16));
     s.layer_off.push_back((int)s.ab.size());
