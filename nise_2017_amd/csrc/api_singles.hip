@@ -95,9 +95,9 @@ int upload_dense(nise_abs_plan *P) {
   if ((rc = P->U.alloc(dense_u_bytes(r.N, P->f_hi - P->f_lo)))) return rc;
   d.U = P->U.as<float2>();
   const int ns = P->end - P->begin;
-  P->nwg = ns, P->npart = r.N <= 64 ? 3 * ns : ns;
+  P->nwg = ns, P->npart = dense_parts(r.N, ns);
   std::vector<int2> map(ns);
-  for (int s = 0; s < ns; ++s) map[s] = make_int2(0, r.N <= 64 ? 3 * s : s);
+  for (int s = 0; s < ns; ++s) map[s] = make_int2(0, s);
   if ((rc = upload(P->dsys, &d, sizeof(d), P->st))) return rc;
   return upload(P->dmap, map.data(), map.size() * sizeof(int2), P->st);
 }
@@ -185,8 +185,7 @@ int run_conveyor(nise_abs_plan *P) {
   if (P->dense) {
     int rc = launch_rows_u(P->row_desc, P->rows, P->f_hi - P->f_lo, P->U.as<float2>(), P->st);
     if (rc) return rc;
-    return (P->N <= 64 ? launch_dense_vectors : launch_dense_wide)(P->dsys.as<DiaSys>(), P->dmap.as<int2>(), P->nwg,
-                                                                   P->st, nullptr);
+    return launch_dense(dense_class(P->N), P->dsys.as<DiaSys>(), P->dmap.as<int2>(), P->nwg, P->st, nullptr);
   }
   if (P->rows)
     return launch_rows(P->row_sys.as<RowsArgs>(), P->row_wmap.as<int2>(), P->nwg, P->rows, P->row_pf, P->row_smem,
@@ -251,11 +250,13 @@ int onfly_scheme(const t_non *non) {
   return 0;
 }
 
-// Plan set-up shared by nise_abs_plan_create and nise_abs_plan_create_onfly
-// (pos_rec: position records for on-the-fly couplings, else null).
+// Plan set-up shared by nise_abs_plan_create, nise_abs_plan_create_onfly
+// (pos_rec: position records for on-the-fly couplings, else null) and
+// nise_absorption_batched (one_run).
 static int plan_create(nise_abs_plan **out, const t_non *non, const float *H_rec, int64_t H_stride,
                        const float *mu_rec, int64_t mu_stride, int64_t nframes, const float *coupling_rec,
-                       const float *pos_rec, int64_t pos_stride, const float *box_rec, int where, int kernel) {
+                       const float *pos_rec, int64_t pos_stride, const float *box_rec, int where, int kernel,
+                       bool one_run = false) {
   *out = nullptr;
   int rc = ensure_device();
   if (rc) return rc;
@@ -369,8 +370,9 @@ static int plan_create(nise_abs_plan **out, const t_non *non, const float *H_rec
     P->vp = 16, P->spw = 5;
     P->rows = rows_for(N, P->sch_asap.Kreal, P->sch_asap.nlayers());
     P->mask = mask;
-    P->dense = P->packed = dense_pays(N, P->tmax, P->end - P->begin, nfr, P->sch_asap.Kreal, P->sch_asap.nlayers(), P->m);
-    if (P->dense) pack_schedule_rows(P->sch_asap, P->rows, P->sch_rows);
+    P->dense = dense_pays(N, P->tmax, P->end - P->begin, nfr, P->sch_asap.Kreal, P->sch_asap.nlayers(), P->m);
+    P->packed = P->dense && one_run;  // a run made once does not pay for the list schedule
+    if (P->packed) pack_schedule_rows(P->sch_asap, P->rows, P->sch_rows);
     else build_schedule_rows(N, mask, P->rows, P->sch_rows);
     if ((rc = build_slots(P))) return rc;
   }
@@ -683,8 +685,8 @@ extern "C" int nise_absorption_batched(const t_non *non, const float *H_rec, int
     return nise_absorption_multi(&y, 1, where, re_S, im_S, nullptr);
   }
   nise_abs_plan *P = nullptr;
-  int rc = nise_abs_plan_create(&P, non, H_rec, H_stride, mu_rec, mu_stride, nframes, coupling_rec,
-                                where, kernel);
+  int rc = plan_create(&P, non, H_rec, H_stride, mu_rec, mu_stride, nframes, coupling_rec, nullptr, 0, nullptr, where,
+                       kernel, true);
   if (rc) return rc;
   rc = nise_abs_plan_execute(P, re_S, im_S, 0);
   nise_abs_plan_destroy(P);

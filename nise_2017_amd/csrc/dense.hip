@@ -1,6 +1,6 @@
 // Absorption vectors through dense per-frame propagators U: the exact
 // exponential (src/propagate.c:60-125), and the Trotter scheme where a run has
-// too few vectors to fill the chip with sweeps (dense_pays).  N <= 64: one
+// too few vectors to fill the chip with sweeps (dense_pays).  N <= 32: one
 // wave per vector.
 //
 // What bounds it is the chain of tmax dependent steps: a batch has a few
@@ -24,14 +24,14 @@
 
 namespace nise {
 
-// NP: rows (a power of two >= N, at most 64); PPL: column pairs per lane.
+// NP: rows (a power of two >= N, at most 32); PPL: column pairs per lane.
 template <int NP, int PPL>
 __device__ __forceinline__ void dense_run(const DiaSys &S, int v, float2 *psi) {
   constexpr int G = 64 / NP;
   const int N = S.N, T = S.tmax, Pr = (N + 1) >> 1, nU = Pr * N;
   const int lane = threadIdx.x & 63, a = lane % NP, g = lane / NP;
   const bool row = a < N;
-  const int64_t fs = (int64_t)(S.begin + v / 3) * S.sample;
+  const int64_t fs = (int64_t)(S.begin + v / 3) * S.sample + S.t0;  // frame of step t0
   // entries past N stay zero: U's pad column and the clamped pairs below
   // meet a zero
   for (int i = lane; i < 2 * G * PPL; i += 64) psi[i] = make_float2(0.f, 0.f);
@@ -53,8 +53,9 @@ __device__ __forceinline__ void dense_run(const DiaSys &S, int v, float2 *psi) {
   for (int i = 0; i < PPL; ++i) u[i] = load(U, i);
   float m = gld(mu);
   float2 p = make_float2(m, 0.f);
+  if (S.t0) p = gld(S.state + (int64_t)v * N + min(a, N - 1));
   double2 *out = S.partial + (int64_t)v * T;
-  for (int t = 0; t < T; ++t) {
+  for (int t = S.t0;; ++t) {
     if (S.hist) {  // checkpoint rows as the conveyor writes them (RowsArgs)
       const int hr = t % S.hist_every == 0 ? t / S.hist_every : t == T - 1 ? t / S.hist_every + 1 : -1;
       if (hr >= 0 && row && g == 0) gst(S.hist + ((int64_t)v * S.nck + hr) * N + a, p);
@@ -63,12 +64,14 @@ __device__ __forceinline__ void dense_run(const DiaSys &S, int v, float2 *psi) {
     const float rr = group_sum<NP>(row ? m * p.x : 0.f), ri = group_sum<NP>(row ? m * p.y : 0.f);
     if (lane == 0) gst(out + t, make_double2((double)rr, (double)ri));
     if (t == T - 1) break;
-    mu += S.mu_stride;
+    const bool more = t + 1 < S.t1;
+    mu += more ? S.mu_stride : 0;
     m = gld(mu);
     if (row && g == 0) psi[a] = p;
-    // psi <- U psi (src/propagate.c:109-119); the refills read frame fs + t
-    // + 1 <= fs + T - 1, which the tables hold
-    U += nU;
+    // psi <- psi + (U - I) psi (src/propagate.c:109-119); the refills read the frame of
+    // step t + 1 < t1, which the tables hold (at the end of a segment the same
+    // frame again, not used)
+    U += more ? nU : 0;
     float2 y0 = make_float2(0.f, 0.f), y1 = make_float2(0.f, 0.f);
 #pragma unroll
     for (int i = 0; i < PPL; ++i) {
@@ -79,36 +82,32 @@ __device__ __forceinline__ void dense_run(const DiaSys &S, int v, float2 *psi) {
       y1.x = fmaf(w.z, c.z, y1.x), y1.y = fmaf(w.z, c.w, y1.y);
       y0.x = fmaf(-w.y, c.y, y0.x), y0.y = fmaf(w.y, c.x, y0.y);
       y1.x = fmaf(-w.w, c.w, y1.x), y1.y = fmaf(w.w, c.z, y1.y);
-      // eight state reads in flight: hoisting all 32 of an N = 64 row spills
-      if ((i & 7) == 7) __builtin_amdgcn_sched_barrier(0);
     }
-    p = make_float2(y0.x + y1.x, y0.y + y1.y);
-    if constexpr (G > 1) p = make_float2(stride_sum<NP>(p.x), stride_sum<NP>(p.y));
+    p = make_float2(p.x + stride_sum<NP>(y0.x + y1.x), p.y + stride_sum<NP>(y0.y + y1.y));
+    if (!more) {  // the segment's end: its state
+      if (row && g == 0) gst(S.state + (int64_t)v * N + a, p);
+      break;
+    }
   }
 }
 
-// Workgroup: the three polarisations of sample wmap.y / 3 of system wmap.x,
+// Workgroup: the three polarisations of sample wmap.y of system wmap.x,
 // one wave each (they read the same U at about the same time, through the
-// same L1).  Row classes of 8, 16, 32 and 64; a lane's pairs cover N.
-constexpr int kDensePsi = 64;  // LDS state entries per wave
-__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(2)))
-dense_vectors_kernel(const DiaSys *sys, const int2 *wmap,
-                                                            unsigned long long *times) {
+// same L1).  Row classes of 8, 16 and 32; a lane's pairs cover N.
+constexpr int kDensePsi = 32;  // LDS state entries per wave
+__global__ void __launch_bounds__(192)
+dense_vectors_kernel(const DiaSys *sys, const int2 *wmap, unsigned long long *times) {
   __shared__ __align__(16) float2 psi[3][kDensePsi];
   const unsigned long long t_start = __builtin_amdgcn_s_memrealtime();
   const int2 wm0 = wmap[blockIdx.x];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const DiaSys S = sys[__builtin_amdgcn_readfirstlane(wm0.x)];
-  const int v = __builtin_amdgcn_readfirstlane(wm0.y) + wave;
+  const int v = 3 * __builtin_amdgcn_readfirstlane(wm0.y) + wave;
   const int N = S.N;
   if (N <= 8) dense_run<8, 1>(S, v, psi[wave]);
   else if (N <= 16) dense_run<16, 2>(S, v, psi[wave]);
   else if (N <= 24) dense_run<32, 6>(S, v, psi[wave]);
-  else if (N <= 32) dense_run<32, 8>(S, v, psi[wave]);
-  else if (N <= 40) dense_run<64, 20>(S, v, psi[wave]);
-  else if (N <= 48) dense_run<64, 24>(S, v, psi[wave]);
-  else if (N <= 56) dense_run<64, 28>(S, v, psi[wave]);
-  else dense_run<64, 32>(S, v, psi[wave]);
+  else dense_run<32, 8>(S, v, psi[wave]);
   __syncthreads();
   if (threadIdx.x == 0 && times) {
     times[2 * blockIdx.x] = t_start;
@@ -117,7 +116,7 @@ dense_vectors_kernel(const DiaSys *sys, const int2 *wmap,
 }
 
 // ---------------------------------------------------------------------------
-// N = 65 .. 128: one workgroup of eight waves per sample.  Lane (h, r) =
+// N = 33 .. 128: one workgroup of eight waves per sample.  Lane (h, r) =
 // (lane / 32, lane % 32) of wave w holds rows r, r + 32, ... of the column
 // pairs 2 w + h, + 16, ... in registers and applies them to the sample's
 // three vectors, so each entry of U is loaded once per sample and step (a
@@ -138,7 +137,7 @@ __device__ __forceinline__ void wide_run(const DiaSys &S, int s, unsigned char *
   constexpr int NR = 32 * RPL;
   const int N = S.N, T = S.tmax, Pr = (N + 1) >> 1, nU = Pr * N, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, h = lane >> 5, r = lane & 31;
-  const int64_t fs = (int64_t)(S.begin + s) * S.sample;
+  const int64_t fs = (int64_t)(S.begin + s) * S.sample + S.t0;  // frame of step t0
   // entries past N stay zero: U's pad column and the clamped pairs meet a zero
   for (int i = tid; i < 3 * 2 * kWideSlices * PPL; i += 64 * kWideWaves) (&L.psi[0][0])[i] = make_float2(0.f, 0.f);
   const float4 *U = reinterpret_cast<const float4 *>(S.U) + (fs - S.f_lo) * nU;
@@ -158,9 +157,11 @@ __device__ __forceinline__ void wide_run(const DiaSys &S, int s, unsigned char *
   const float *mu = S.mu_rec + (S.mu_stride ? fs * S.mu_stride : 0) + 1 + (own ? (int64_t)x * N + a : 0);
   float m = gld(mu);
   float2 p = make_float2(own ? m : 0.f, 0.f);
+  const int64_t srow = own ? (int64_t)(3 * s + x) * N + a : 0;
+  if (S.t0 && own) p = gld(S.state + srow);
   __syncthreads();
   double2 *out = S.partial + (int64_t)s * T;
-  for (int t = 0;; ++t) {
+  for (int t = S.t0;; ++t) {
     if (S.hist) {
       const int hr = t % S.hist_every == 0 ? t / S.hist_every : t == T - 1 ? t / S.hist_every + 1 : -1;
       if (hr >= 0 && own) gst(S.hist + ((int64_t)(3 * s + x) * S.nck + hr) * N + a, p);
@@ -176,9 +177,10 @@ __device__ __forceinline__ void wide_run(const DiaSys &S, int s, unsigned char *
       gst(out + t, z);
     }
     if (t == T - 1) break;
-    mu += S.mu_stride;
+    const bool more = t + 1 < S.t1;
+    mu += more ? S.mu_stride : 0;
     m = gld(mu);
-    U += nU;  // the refills: frame fs + t + 1 <= fs + T - 1
+    U += more ? nU : 0;  // the refills: the frame of step t + 1 < t1
     float2 y[3][RPL];
 #pragma unroll
     for (int v = 0; v < 3; ++v)
@@ -220,42 +222,48 @@ __device__ __forceinline__ void wide_run(const DiaSys &S, int s, unsigned char *
       for (int st = 1; st < kWideWaves; st <<= 1)
 #pragma unroll
         for (int w = 0; w < kWideWaves; w += 2 * st) q[w].x += q[w + st].x, q[w].y += q[w + st].y;
-      p = q[0];
+      p.x += q[0].x, p.y += q[0].y;
+    }
+    if (!more) {
+      if (own) gst(S.state + srow, p);
+      break;
     }
   }
 }
 
-// Workgroup: sample wmap.y of system wmap.x (N <= 128; N <= 64 pads).
-__global__ void __launch_bounds__(64 * kWideWaves) __attribute__((amdgpu_waves_per_eu(2)))
+// Workgroup: sample wmap.y of system wmap.x.  Up to three rows per lane two
+// workgroups share a CU (333 samples of a 77-site lattice on 256 CUs: propagators and
+// this 1.05 ms, 1.14 with one workgroup per CU).
+template <int RPL, int PPL>
+__global__ void __launch_bounds__(64 * kWideWaves) __attribute__((amdgpu_waves_per_eu(RPL < 4 ? 4 : 2)))
 dense_wide_kernel(const DiaSys *sys, const int2 *wmap, unsigned long long *times) {
-  __shared__ __align__(16) unsigned char smem[sizeof(WideLds<4, 4>)];
+  __shared__ __align__(16) unsigned char smem[sizeof(WideLds<RPL, PPL>)];
   const unsigned long long t_start = __builtin_amdgcn_s_memrealtime();
   const int2 wm = wmap[blockIdx.x];
   const DiaSys S = sys[__builtin_amdgcn_readfirstlane(wm.x)];
-  const int s = __builtin_amdgcn_readfirstlane(wm.y);
-  if (S.N <= 64) wide_run<2, 2>(S, s, smem);
-  else if (S.N <= 96) wide_run<3, 3>(S, s, smem);
-  else wide_run<4, 4>(S, s, smem);
+  wide_run<RPL, PPL>(S, __builtin_amdgcn_readfirstlane(wm.y), smem);
   if (threadIdx.x == 0 && times) {
     times[2 * blockIdx.x] = t_start;
     times[2 * blockIdx.x + 1] = __builtin_amdgcn_s_memrealtime();
   }
 }
 
-// sys / wmap: device copies, one workgroup per (system, sample), N <= 64.
-int launch_dense_vectors(const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t st, unsigned long long *times) {
-  if (nwg == 0) return NISE_OK;
-  hipLaunchKernelGGL(dense_vectors_kernel, dim3((unsigned)nwg), dim3(192), 0, st, sys, wmap, times);
-  NISE_HIP_CHECK(hipGetLastError());
-  return NISE_OK;
-}
+// Kernel by size: a wave per vector up to N = 32 (a row's half in a lane's
+// registers), above it the wide kernel, which reads U once for the three
+// vectors (exact propagators, 200 steps, wave and wide, ms: N = 64, 100
+// samples 0.87 and 0.51, 1,500 samples 5.6 and 4.1; N = 48, 1,500 samples 3.4
+// and 2.9; N = 36, 1,500 samples 2.4 and 2.6).
+constexpr int kDenseWaveN = 32;
+int dense_class(int N) { return N <= kDenseWaveN ? 0 : N <= 64 ? 1 : N <= 96 ? 2 : 3; }
 
-// sys / wmap: device copies, one workgroup per (system, sample), N <= 128;
-// partial holds one row per sample.
-int launch_dense_wide(const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t st, unsigned long long *times) {
+// sys / wmap: device copies.
+int launch_dense(int cls, const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t st, unsigned long long *times) {
   if (nwg == 0) return NISE_OK;
-  hipLaunchKernelGGL(dense_wide_kernel, dim3((unsigned)nwg), dim3(64 * kWideWaves), 0, st, sys, wmap, times);
-  NISE_HIP_CHECK(hipGetLastError());
+  const void *fn = cls == 0 ? (const void *)dense_vectors_kernel : cls == 1 ? (const void *)dense_wide_kernel<2, 2>
+                 : cls == 2 ? (const void *)dense_wide_kernel<3, 3> : cls == 3 ? (const void *)dense_wide_kernel<4, 4> : nullptr;
+  if (!fn) return set_error("dense propagators: bad class %d", cls), NISE_ERR_ARG;
+  void *kargs[] = {&sys, &wmap, &times};
+  NISE_HIP_CHECK(hipLaunchKernel(fn, dim3((unsigned)nwg), dim3(cls ? 64 * kWideWaves : 192), kargs, 0, st));
   return NISE_OK;
 }
 
@@ -265,9 +273,9 @@ int launch_dense_wide(const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t 
 // every vector step.  A conveyor wave walks tmax frames of nlayers dependent
 // LDS round trips, so runs with few waves are far from its throughput.  The
 // cycle counts are fits: measured (conveyor and this, ms) N = 16 chain, 200
-// samples 0.45 and 0.14; N = 77 lattice, 333 samples 2.66 and 1.09; N = 121
-// lattice, 600 samples 4.14 and 3.31; N = 64 lattice, 1,500 samples 2.74 and
-// 3.37 (conveyor); N = 100 lattice, 1,500 samples 4.12 (conveyor).
+// and 1,000 samples 0.45 and 0.13, 0.47 and 0.25; N = 77 lattice, 333 samples
+// 2.60 and 1.05; N = 64 lattice, 800 samples 2.43 and 1.24, 1,500 samples 2.72
+// (conveyor; 3.4); N = 121 lattice, 800 samples 4.50 and 4.41.
 // Kreal, nasap: rotations and layers of the layered schedule; m: Trotter
 // substeps; F: frames; S: samples.
 bool dense_pays(int N, int T, int64_t S, int64_t F, int Kreal, int nasap, int m) {
@@ -277,18 +285,12 @@ bool dense_pays(int N, int T, int64_t S, int64_t F, int Kreal, int nasap, int m)
   const double G = 64.0 / R, sweep = std::max({(double)nasap, (double)Kreal / R, 8.0}) * m;
   // conveyor: a wave's frame is a chain of LDS round trips and its share of
   // the sites; all waves together are bound by LDS instructions
-  const double site = 12.0 * N / R + 600.0, waves = 3.0 * S / G;
-  const double rows = T * std::max(sweep * 170.0 + site, waves / 256.0 * (sweep * 22.5 + site * 0.25));
-  const double build = F * std::ceil((N + (N & 1)) / G) / 256.0 * (sweep * 22.5 + 400.0) + 20000.0;
-  const double apply = N <= 64 ? T * std::max(700.0 + 20.0 * N, 3.0 * S / 1024.0 * (300.0 + 30.0 * N))
-                               : T * std::ceil(S / 256.0) * (1800.0 + 36.0 * N);
-  if (!(build + apply < 0.85 * rows)) return false;
-  // nise_absorption_batched_noalloc follows the same choice in windows of
-  // samples: a run that its array held with the conveyor's tables must hold
-  // one sample's window
-  const double K = std::max((double)nasap, (double)Kreal / R) * R * 1.1 + 8.0 * R;
-  const double part = 3.0 * S * T * 16 + K * 12 + S * 8 + 65536;
-  return F * (N + K) * 8 + part > kScratchBytes * 1.2 || T * ((N + K) * 8 + dense_u_bytes(N, 1)) + part < kScratchBytes * 0.9;
+  const double rows = T * (176.0 * sweep + 180.0 * N / R + 300.0) * (1.0 + 3.0 * S / G / 3400.0);
+  const double build = F * std::ceil((N + (N & 1)) / G) / 256.0 * (21.0 * sweep + 150.0) + 20000.0;
+  const double apply = dense_class(N) == 0
+                           ? T * std::max(500.0 + 24.0 * N, 3.0 * S / 1024.0 * (200.0 + 12.0 * N))
+                           : T * std::max(1.0, S / 256.0) * (1000.0 + 40.0 * N);
+  return build + apply < 0.85 * rows;
 }
 
 }  // namespace nise

@@ -188,8 +188,8 @@ __device__ void trig_poly(const double Bv[4][4], const double *B2, double *X, co
   }
 }
 
-// pairs = 0: U[m][a][b] row-major; pairs = 1: U[m][b / 2][a] as float4
-// (U_a,b, U_a,b+1), the second half zero past the last column (the layout
+// pairs = 0: U[m][a][b] row-major; pairs = 1: (U - I)[m][b / 2][a] as float4
+// (columns b, b + 1), the second half zero past the last column (the layout
 // of dense.hip: one 16-byte read gives a site two columns).
 // One system's frames for expm_jobs_kernel; b is set by launch_expm_jobs.
 struct ExpmJob {
@@ -318,7 +318,9 @@ __device__ __forceinline__ void expm_frame(const FrameSource &src, int N, int64_
       if (!g.in(i, j)) continue;
       const int a = g.ry + S * i, b = g.cx + S * j;
       float2 u = make_float2((float)ur[i][j], (float)ui[i][j]);
-      if (thres > 0.f && !(__fadd_rn(__fmul_rn(u.x, u.x), __fmul_rn(u.y, u.y)) > thres)) u = make_float2(0.f, 0.f);
+      const bool drop = thres > 0.f && !(__fadd_rn(__fmul_rn(u.x, u.x), __fmul_rn(u.y, u.y)) > thres);
+      if (drop) u = make_float2(0.f, 0.f);
+      if (pairs && a == b) u.x = drop ? -1.f : (float)(ur[i][j] - 1.0);
       Um[pairs ? ((b >> 1) * N + a) * 2 + (b & 1) : a * N + b] = u;
     }
   if (pairs && (N & 1))
@@ -674,7 +676,7 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
       d.N = N;
       d.tmax = s.T, d.begin = non->begin, d.sample = non->sample, d.nvec = s.nvec, d.f_lo = s.f_lo;
       d.U = s.U.as<float2>(), d.mu_rec = s.mu_dev, d.mu_stride = s.mu_stride;
-      s.nwg = s.nvec;  // partial rows: one per vector
+      s.nwg = dense_parts(N, s.nvec / 3);  // partial rows
       if ((rc = s.partial.alloc((size_t)s.nwg * s.T * sizeof(double2)))) return rc;
       d.partial = s.partial.as<double2>();
       dias.push_back(d);
@@ -758,7 +760,7 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
       if ((rc = launch_frame_tables(s.src, N, s.sch, s.ab.as<uint32_t>(), trotter_factor(non->deltat, 1, non->ts),
                                     s.f_lo, nfr, s.diag.as<float2>(), s.cs.as<float2>(), st)))
         return rc;
-      s.nwg = s.dense && N > 64 ? s.nvec / 3 : s.nvec;  // partial rows: one per vector or sample
+      s.nwg = s.dense ? dense_parts(N, s.nvec / 3) : s.nvec;  // partial rows
       if ((rc = s.partial.alloc((size_t)s.nwg * s.T * sizeof(double2)))) return rc;
       RowsArgs r;
       r.N = N, r.tmax = s.T, r.m = non->ts, r.nlayers = s.sch.nlayers(), r.K = s.sch.K, r.f_lo = s.f_lo;
@@ -790,20 +792,18 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
     const RowsArgs &a = rows[x.x], &b = rows[y.x];
     return (int64_t)a.nlayers * a.tmax * a.m > (int64_t)b.nlayers * b.tmax * b.m;
   });
-  // dmap: vectors of the DIA systems (second stream), then of the Trotter
-  // systems' propagators up to 64 sites and above (first stream)
-  size_t dend[3];
-  for (int kind = 0; kind < 3; ++kind) {
-    for (size_t i = 0; i < dias.size(); ++i) {
-      const SysState &s = *S[dia_of[i]];
-      if (kind != (!s.dense ? 0 : s.N <= 64 ? 1 : 2)) continue;
-      if (kind == 2)
+  // dmap: samples of the DIA systems (second stream), then of the Trotter
+  // systems' propagators (first stream), each by kernel class
+  size_t dend[2][4];
+  for (int tr = 0; tr < 2; ++tr)
+    for (int cls = 0; cls < 4; ++cls) {
+      for (size_t i = 0; i < dias.size(); ++i) {
+        const SysState &s = *S[dia_of[i]];
+        if (s.dense != (tr == 1) || dense_class(s.N) != cls) continue;
         for (int v = 0; v < s.nvec / 3; ++v) dmap.push_back(make_int2((int)i, v));
-      else
-        for (int v = 0; v < s.nvec; v += 3) dmap.push_back(make_int2((int)i, v));
+      }
+      dend[tr][cls] = dmap.size();
     }
-    dend[kind] = dmap.size();
-  }
   for (size_t i = 0; i < dias.size(); ++i) {
     if (!S[dia_of[i]]->dense && !dia_window_fits(dias[i].N, dias[i].tmax, dias[i].nvec))
       return set_error("multi: DIA window of %d steps is too long for N=%d", dias[i].tmax, dias[i].N), NISE_ERR_ARG;
@@ -832,10 +832,12 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
   const DiaSys *dsp = dsys.as<DiaSys>();
   const int2 *dmp = dwm.as<int2>();
   unsigned long long *td = tm + 2 * rmap.size();
-  if ((rc = launch_dense_vectors(dsp, dmp, (int)dend[0], sd, td)) ||
-      (rc = launch_dense_vectors(dsp, dmp + dend[0], (int)(dend[1] - dend[0]), st, td + 2 * dend[0])) ||
-      (rc = launch_dense_wide(dsp, dmp + dend[1], (int)(dend[2] - dend[1]), st, td + 2 * dend[1])))
-    return rc;
+  size_t d0 = 0;
+  for (int tr = 0; tr < 2; ++tr)
+    for (int cls = 0; cls < 4; ++cls) {
+      if ((rc = launch_dense(cls, dsp, dmp + d0, (int)(dend[tr][cls] - d0), tr ? st : sd, td + 2 * d0))) return rc;
+      d0 = dend[tr][cls];
+    }
   // the reductions and copies below wait for the DIA stream
   {
     hipEvent_t ev;

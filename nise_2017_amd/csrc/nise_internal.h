@@ -423,7 +423,7 @@ struct RowsArgs {
   int hist_every = 1, nck = 0;
 };
 int rows_prepare(const RowsArgs *sys, int nsys, int R, std::vector<int2> &wmap, size_t &smem, bool &pf);
-// U of every frame of the row tables (Trotter step propagators, DiaSys layout).
+// U - I of every frame of the row tables (Trotter step propagators, DiaSys layout).
 int launch_rows_u(const RowsArgs &a, int R, int64_t nfr, float2 *U, hipStream_t st);
 // times (optional): per workgroup (start, end) on the device wall clock.
 int launch_rows(const RowsArgs *sys, const int2 *wmap, int nwg, int R, bool pf, size_t smem, hipStream_t st,
@@ -434,12 +434,16 @@ int launch_rows(const RowsArgs *sys, const int2 *wmap, int nwg, int R, bool pf, 
 struct DiaSys {
   int N = 0, tmax = 0, begin = 0, sample = 1, nvec = 0;
   int64_t f_lo = 0;
-  const float2 *U = nullptr;     // [rows][(N + 1) / 2][N] column pairs (expm_per)
+  const float2 *U = nullptr;     // U - I: [rows][(N + 1) / 2][N] column pairs (expm_per)
   const float *mu_rec = nullptr;
   int64_t mu_stride = 0;
-  double2 *partial = nullptr;    // [vectors][tmax] (N > 64: [samples][tmax])
+  double2 *partial = nullptr;    // [vectors][tmax] (class > 0: [samples][tmax])
   float2 *hist = nullptr;        // checkpoints, as RowsArgs
   int hist_every = 1, nck = 0;
+  // steps t0 .. t1 - 1 only (U from the frame of step t0 on): the vectors come
+  // from and go to state [vectors][N], unless t0 is 0 and t1 >= tmax
+  int t0 = 0, t1 = 0x7fffffff;
+  float2 *state = nullptr;
 };
 // Trotter runs through propagators keep the reference's rounded rotation
 // coefficients but not its rounding of every product, which is biased where a
@@ -451,10 +455,12 @@ constexpr double kDenseMaxBytes = 1 << 30;  // of U
 constexpr size_t kScratchBytes = (size_t)32 << 20;  // noalloc.hip's array, per GPU
 bool dense_pays(int N, int T, int64_t S, int64_t F, int Kreal, int nasap, int m);
 inline size_t dense_u_bytes(int N, int64_t F) { return (size_t)F * 2 * ((N + 1) / 2) * N * 8; }
-// Workgroups: wmap entry (system, 3 * sample) for N <= 64 (launch_dense_vectors),
-// (system, sample) above (launch_dense_wide).
-int launch_dense_wide(const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t st, unsigned long long *times);
-int launch_dense_vectors(const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t st, unsigned long long *times);
+// Kernel class of a system (dense.hip): 0 one wave per vector, 1 .. 3 one
+// workgroup per sample with 2 .. 4 rows per lane.
+int dense_class(int N);
+inline int dense_parts(int N, int nsamples) { return dense_class(N) ? nsamples : 3 * nsamples; }
+// wmap: (system, sample) of each workgroup, systems of one class.
+int launch_dense(int cls, const DiaSys *sys, const int2 *wmap, int nwg, hipStream_t st, unsigned long long *times);
 // U = V exp(-i E f) V^T for nmat eigensystems (multi.hip); thres > 0 drops
 // the elements with FP32 |U_ab|^2 <= thres (the sparse scheme).
 int launch_dia_u(const double *w, const double *V, int N, int64_t nmat, float fac, float thres, float2 *U,

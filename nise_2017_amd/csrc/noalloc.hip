@@ -95,7 +95,7 @@ int run_dense(unsigned char *base, size_t used, const FrameSource &src, RowsArgs
               float fac, float *re_S, float *im_S) {
   int rc;
   const hipStream_t st = nullptr;
-  const int N = r.N, T = r.tmax, npart = N <= 64 ? 3 * ns : ns;
+  const int N = r.N, T = r.tmax, npart = dense_parts(N, ns);
   Schedule sch;
   pack_schedule_rows(asap, R, sch);
   std::vector<uint2> tab;
@@ -110,37 +110,42 @@ int run_dense(unsigned char *base, size_t used, const FrameSource &src, RowsArgs
   DiaSys *sysd = ar.take<DiaSys>(1);
   int2 *mapd = ar.take<int2>(ns);
   if (!steps || !abd || !partial || !out || !sysd || !mapd) return too_big(kScratchBytes + 1);
-  // samples per window: their frames' phases, rotations and U
-  auto frames = [&](int n) { return (int64_t)(n - 1) * r.sample + T; };
-  auto bytes = [&](int n) {
-    const size_t f = (size_t)frames(n);
-    return Arena::bytes_of(f * N, 8) + Arena::bytes_of(f * sch.K, 8) + Arena::bytes_of(dense_u_bytes(N, f), 1);
+  // samples per window, or, when one sample's window is too large, steps per
+  // segment of each sample
+  auto bytes = [&](int64_t f) {  // of f frames' phases, rotations and U
+    return Arena::bytes_of((size_t)f * N, 8) + Arena::bytes_of((size_t)f * sch.K, 8) +
+           Arena::bytes_of(dense_u_bytes(N, f), 1);
   };
-  int per = ns;
-  while (per > 1 && ar.used + bytes(per) > kScratchBytes) per = per > 16 ? per * 7 / 8 : per - 1;
-  if (ar.used + bytes(per) > kScratchBytes) return too_big(ar.used + bytes(per));
+  float2 *state = ar.take<float2>((size_t)3 * N);
+  if (!state || ar.used + bytes(1) > kScratchBytes) return too_big(ar.used + bytes(1));
+  int per = ns, seg = T;
+  auto frames = [&](int n) { return (int64_t)(n - 1) * r.sample + T; };
+  while (per > 1 && ar.used + bytes(frames(per)) > kScratchBytes) per = per > 16 ? per * 7 / 8 : per - 1;
+  while (per == 1 && seg > 1 && ar.used + bytes(seg) > kScratchBytes) seg = seg > 16 ? seg * 7 / 8 : seg - 1;
   NISE_HIP_CHECK(hipMemcpy(steps, tab.data(), tab.size() * sizeof(uint2), hipMemcpyHostToDevice));
   NISE_HIP_CHECK(hipMemcpy(abd, ab.data(), ab.size() * 4, hipMemcpyHostToDevice));
   std::vector<int2> map(ns);
-  for (int s = 0; s < ns; ++s) map[s] = make_int2(0, N <= 64 ? 3 * s : s);
+  for (int s = 0; s < ns; ++s) map[s] = make_int2(0, s);
   NISE_HIP_CHECK(hipMemcpy(mapd, map.data(), map.size() * sizeof(int2), hipMemcpyHostToDevice));
   r.nlayers = sch.nlayers(), r.K = sch.K, r.steps = steps;
-  for (int s0 = 0; s0 < ns; s0 += per) {
-    const int n = std::min(per, ns - s0);
-    const int64_t f0 = (int64_t)(r.begin + s0) * r.sample, nf = frames(n);
-    Arena w{base, ar.used};
-    float2 *diag = w.take<float2>((size_t)nf * N), *cs = w.take<float2>((size_t)nf * sch.K);
-    float2 *U = reinterpret_cast<float2 *>(w.take<unsigned char>(dense_u_bytes(N, nf)));
-    if (!diag || !cs || !U) return too_big(kScratchBytes + 1);
-    if ((rc = launch_frame_tables(src, N, sch, abd, fac, f0, nf, diag, cs, st, nullptr))) return rc;
-    r.diag = diag, r.cs = cs, r.f_lo = f0;
-    if ((rc = launch_rows_u(r, R, nf, U, st))) return rc;
-    DiaSys d;
-    d.N = N, d.tmax = T, d.begin = r.begin + s0, d.sample = r.sample, d.nvec = 3 * n, d.f_lo = f0, d.U = U;
-    d.mu_rec = r.mu_rec, d.mu_stride = r.mu_stride, d.partial = partial + (size_t)(N <= 64 ? 3 * s0 : s0) * T;
-    NISE_HIP_CHECK(hipMemcpy(sysd, &d, sizeof(d), hipMemcpyHostToDevice));  // waits for the previous window
-    if ((rc = (N <= 64 ? launch_dense_vectors : launch_dense_wide)(sysd, mapd, n, st, nullptr))) return rc;
-  }
+  for (int s0 = 0; s0 < ns; s0 += per)
+    for (int t0 = 0; t0 < T; t0 += seg) {
+      const int n = std::min(per, ns - s0);
+      const int64_t f0 = (int64_t)(r.begin + s0) * r.sample + t0, nf = seg < T ? std::min(seg, T - t0) : frames(n);
+      Arena w{base, ar.used};
+      float2 *diag = w.take<float2>((size_t)nf * N), *cs = w.take<float2>((size_t)nf * sch.K);
+      float2 *U = reinterpret_cast<float2 *>(w.take<unsigned char>(dense_u_bytes(N, nf)));
+      if (!diag || !cs || !U) return too_big(kScratchBytes + 1);
+      if ((rc = launch_frame_tables(src, N, sch, abd, fac, f0, nf, diag, cs, st, nullptr))) return rc;
+      r.diag = diag, r.cs = cs, r.f_lo = f0;
+      if ((rc = launch_rows_u(r, R, nf, U, st))) return rc;
+      DiaSys d;
+      d.N = N, d.tmax = T, d.begin = r.begin + s0, d.sample = r.sample, d.nvec = 3 * n, d.f_lo = f0, d.U = U;
+      d.mu_rec = r.mu_rec, d.mu_stride = r.mu_stride, d.partial = partial + (size_t)dense_parts(N, s0) * T;
+      if (seg < T) d.t0 = t0, d.t1 = t0 + (int)nf, d.state = state;
+      NISE_HIP_CHECK(hipMemcpy(sysd, &d, sizeof(d), hipMemcpyHostToDevice));  // waits for the previous window
+      if ((rc = launch_dense(dense_class(N), sysd, mapd, n, st, nullptr))) return rc;
+    }
   if ((rc = launch_reduce_partials(partial, npart, T, out, out + T, st))) return rc;
   NISE_HIP_CHECK(hipMemcpy(re_S, out, T * sizeof(float), hipMemcpyDeviceToHost));
   NISE_HIP_CHECK(hipMemcpy(im_S, out + T, T * sizeof(float), hipMemcpyDeviceToHost));

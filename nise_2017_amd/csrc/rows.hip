@@ -412,11 +412,15 @@ __global__ void __launch_bounds__(64) rows_mixed_kernel(const RowsArgs *__restri
 // The Trotter step propagator U of one frame, G = 64 / R columns per wave
 // (the unit vectors through the frame's sweeps, all at the same frame), in the
 // column-pair layout of dense.hip.  Frames are independent, so unlike the
-// vectors' chains these fill the chip.  The rotations round as the
-// reference's: with a cosine of 1 - k 2^-24 (weak couplings, short steps) its
-// rounded product is biased, a drift of 2e-5 over 512 steps that fused
-// products do not have, and results are compared with the reference's.  Bound
-// by LDS instructions as the conveyor.
+// vectors' chains these fill the chip.  Bound by LDS instructions as the
+// conveyor.  U - I is kept and stored, not U: a diagonal entry near 1 would
+// round by up to 3e-8 in every sweep layer, and with U shared by the samples
+// that overlap a frame this noise does not average out over them as a
+// vector's own does (chain of 32, 150 samples of 64 steps, error of the
+// imaginary part against 64 bits: 6.9e-6 for the conveyor, 7.4e-6 with a rounded
+// U, 1.8e-6 here).  The cosines are the
+// table's, rounded as the reference's: with exact ones the results leave the
+// reference's by more than 1e-5 on lattices of many weak couplings.
 template <int R>
 __global__ void __launch_bounds__(64) rows_u_kernel(RowsArgs A, float2 *U) {
   constexpr int G = 64 / R, B = G < 4 ? G : 4, kRingS = kRingL / B;
@@ -427,17 +431,35 @@ __global__ void __launch_bounds__(64) rows_u_kernel(RowsArgs A, float2 *U) {
   const uint32_t gofs = (uint32_t)g * 8u;
   const float2 *D = A.diag + row * N;
   for (int i = lane; i < (N + R) * G; i += 64) reinterpret_cast<float2 *>(smem)[i] = make_float2(0.f, 0.f);
-  if (q == 0 && c < N) *reinterpret_cast<float2 *>(smem + ((uint32_t)c * G * 8u + gofs)) = gld(D + c);
+  const uint32_t cofs = (uint32_t)c * G * 8u;  // the unit entry's row
+  auto one = [&](uint32_t ofs) { return ofs == cofs ? 1.f : 0.f; };
+  // x + (d - 1) (x + unit): the diagonal phase d
+  auto phase = [&](float2 x, float2 d, uint32_t ofs) {
+    const float2 u = make_float2(x.x + one(ofs), x.y);
+    d.x -= 1.f;
+    return make_float2(fmaf(d.x, u.x, fmaf(-d.y, u.y, x.x)), fmaf(d.x, u.y, fmaf(d.y, u.x, x.y)));
+  };
+  if (q == 0 && c < N) {
+    const float2 d = gld(D + c);
+    *reinterpret_cast<float2 *>(smem + (cofs + gofs)) = make_float2(d.x - 1.f, d.y);
+  }
   const uint32_t loff = (uint32_t)(B * q + (lane & (B - 1)));
   const float2 *csf = A.cs + row * A.K + loff;
   const uint2 *stp = A.steps + loff;
-  auto rot = [&](uint2 e, float2 cc) { rot_step(smem, gofs, e, cc); };
+  auto rot = [&](uint2 e, float2 cc) {  // cc: (cos - 1, sin)
+    float2 *ra = reinterpret_cast<float2 *>(smem + (e.x + gofs)), *rb = reinterpret_cast<float2 *>(smem + (e.y + gofs));
+    const float2 x = *ra, y = *rb;
+    const float ux = x.x + one(e.x), uy = y.x + one(e.y), c1 = cc.x, si = cc.y;
+    *ra = make_float2(fmaf(c1, ux, fmaf(-si, y.y, x.x)), fmaf(c1, x.y, fmaf(si, uy, x.y)));
+    *rb = make_float2(fmaf(c1, uy, fmaf(-si, x.y, y.x)), fmaf(c1, y.y, fmaf(si, ux, y.y)));
+  };
   for (int sub = 0; sub < A.m; ++sub) {
     if (sub)
       for (int i = q; i < N; i += R) {
         const float2 d = gld(D + i);
-        float2 *pp = reinterpret_cast<float2 *>(smem + ((uint32_t)i * G * 8u + gofs));
-        *pp = cmul_diag(cmul_diag(*pp, d), d);
+        const uint32_t ofs = (uint32_t)i * G * 8u;
+        float2 *pp = reinterpret_cast<float2 *>(smem + (ofs + gofs));
+        *pp = phase(phase(*pp, d, ofs), d, ofs);
       }
     uint2 re[kRingS];
     float2 rc[kRingS];
@@ -448,8 +470,9 @@ __global__ void __launch_bounds__(64) rows_u_kernel(RowsArgs A, float2 *U) {
 #pragma unroll
       for (int k = 0; k < kRingS; ++k) {
         const uint2 e = re[k];
-        const float2 cc = rc[k];
+        float2 cc = rc[k];
         re[k] = gld(stp + nx + B * k * R), rc[k] = gld(csf + nx + B * k * R);
+        cc.x -= 1.f;
         rot(make_uint2(grp_bcast<B, 0>(e.x), grp_bcast<B, 0>(e.y)), make_float2(grp_bcast<B, 0>(cc.x), grp_bcast<B, 0>(cc.y)));
         if constexpr (B > 1)
           rot(make_uint2(grp_bcast<B, 1>(e.x), grp_bcast<B, 1>(e.y)), make_float2(grp_bcast<B, 1>(cc.x), grp_bcast<B, 1>(cc.y)));
@@ -464,8 +487,9 @@ __global__ void __launch_bounds__(64) rows_u_kernel(RowsArgs A, float2 *U) {
   float2 *Um = U + row * 2 * Pr * N;
   if (c < 2 * Pr)  // an odd N's pad column holds zeros
     for (int i = q; i < N; i += R) {
-      const float2 p = *reinterpret_cast<const float2 *>(smem + ((uint32_t)i * G * 8u + gofs));
-      gst(Um + ((int64_t)(c >> 1) * N + i) * 2 + (c & 1), cmul_diag(p, gld(D + i)));
+      const uint32_t ofs = (uint32_t)i * G * 8u;
+      const float2 p = *reinterpret_cast<const float2 *>(smem + (ofs + gofs));
+      gst(Um + ((int64_t)(c >> 1) * N + i) * 2 + (c & 1), phase(p, gld(D + i), ofs));
     }
 }
 

@@ -97,14 +97,14 @@ def test_trotter_propagators_coupling_type_and_shifts():
     assert np.array_equal(re + 1j * im, d)
 
 
-@pytest.mark.parametrize("N", [40, 90])
-def test_noalloc_windows_match_plan(N):
+@pytest.mark.parametrize("N,T,ns,sr", [(40, 60, 200, 14), (90, 60, 90, 14), (126, 256, 3, 90)])
+def test_noalloc_windows_match_plan(N, T, ns, sr):
     """A run whose propagators exceed the fixed scratch array: windows of
-    samples, bit for bit the plan's result."""
+    samples, and segments of a sample's steps where one window is too large,
+    bit for bit the plan's result."""
     import ctypes as C
 
     import torch
-    T, ns, sr = 60, 90 if N == 90 else 200, 14
     non, H, mu = lattice_case(N, T, ns, sr, seed=880 + N)
     Hd, mud = torch.from_numpy(H).cuda(), torch.from_numpy(mu).cuda()
     torch.cuda.synchronize()
