@@ -26,27 +26,6 @@
 
 namespace nise {
 
-
-__device__ __forceinline__ float2 cmul_conj_d(float2 p, float2 d) {
-  // p * conj(d), d = (cos, -sin): the inverse of the reference's
-  // (cr*re - ci*im, ci*re + cr*im) product with d
-  return make_float2(__fadd_rn(__fmul_rn(p.x, d.x), __fmul_rn(p.y, d.y)),
-                     __fsub_rn(__fmul_rn(p.y, d.x), __fmul_rn(p.x, d.y)));
-}
-
-__device__ __forceinline__ void rotate_back(float2 &pa, float2 &pb, float co, float si) {
-  // R^dagger: the forward rotation of src/propagate.c:883-887 with -si
-  const float ar = __fadd_rn(__fmul_rn(co, pa.x), __fmul_rn(si, pb.y));
-  const float ai = __fsub_rn(__fmul_rn(co, pa.y), __fmul_rn(si, pb.x));
-  const float br = __fadd_rn(__fmul_rn(co, pb.x), __fmul_rn(si, pa.y));
-  const float bi = __fsub_rn(__fmul_rn(co, pb.y), __fmul_rn(si, pa.x));
-  pa = make_float2(ar, ai);
-  pb = make_float2(br, bi);
-}
-
-// Im(conj(x) y)
-__device__ __forceinline__ float im_cj(float2 x, float2 y) { return x.x * y.y - x.y * y.x; }
-
 // One wave per workgroup: VP vectors, 64/VP rotations of a layer at a time.
 // LDS operations of one wave execute in order, so layers need no barrier.
 template <int VP>
@@ -164,18 +143,30 @@ __global__ void __launch_bounds__(64) adjoint_kernel(AdjArgs A) {
   if (t == 0) A.part_c[g] = cg;
 }
 
-__global__ void adjoint_reduce_kernel(const double *pd, const double *pc, int nwg, int N,
-                                      double *out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < N) {
-    double s = 0.0;
-    for (int g = 0; g < nwg; ++g) s += pd[(int64_t)g * N + i];
+// out[i] = sum over the workgroups of gradient i (i < N: offsets, N: scale),
+// one wave each in a fixed order; read across i by the lanes of 16 (a thread
+// per i walking all partials took 0.1 ms for a thousand workgroups).
+constexpr int kAdjRedX = 16, kAdjRedY = 16;
+__global__ void __launch_bounds__(kAdjRedX * kAdjRedY) adjoint_reduce_kernel(const double *pd, const double *pc, int nwg,
+                                                                            int N, double *out) {
+  __shared__ double acc[kAdjRedY][kAdjRedX];
+  const int x = threadIdx.x % kAdjRedX, y = threadIdx.x / kAdjRedX, i = blockIdx.x * kAdjRedX + x;
+  double s = 0.0;
+  if (i <= N)
+    for (int g = y; g < nwg; g += kAdjRedY) s += i < N ? pd[(int64_t)g * N + i] : pc[g];
+  acc[y][x] = s;
+  __syncthreads();
+  if (y == 0 && i <= N) {
+    s = 0.0;
+    for (int k = 0; k < kAdjRedY; ++k) s += acc[k][x];
     out[i] = s;
-  } else if (i == N) {
-    double s = 0.0;
-    for (int g = 0; g < nwg; ++g) s += pc[g];
-    out[N] = s;
   }
+}
+
+int launch_adjoint_reduce(const double *pd, const double *pc, int nwg, int N, double *out, hipStream_t st) {
+  hipLaunchKernelGGL(adjoint_reduce_kernel, dim3(N / kAdjRedX + 1), dim3(kAdjRedX * kAdjRedY), 0, st, pd, pc, nwg, N, out);
+  NISE_HIP_CHECK(hipGetLastError());
+  return NISE_OK;
 }
 
 // Row variant (used with the row conveyor's schedule and tables): one wave
@@ -454,10 +445,7 @@ int launch_adjoint_rows(const AdjRowsArgs &a, int R, double *out, hipStream_t st
     void *kargs[] = {&args};
     NISE_HIP_CHECK(hipLaunchKernel(fn, dim3(nwg), dim3(64), kargs, smem, st));
   }
-  hipLaunchKernelGGL(adjoint_reduce_kernel, dim3((a.N + 1 + 127) / 128), dim3(128), 0, st,
-                     a.part_delta, a.part_c, nwg, a.N, out);
-  NISE_HIP_CHECK(hipGetLastError());
-  return NISE_OK;
+  return launch_adjoint_reduce(a.part_delta, a.part_c, nwg, a.N, out, st);
 }
 
 size_t adjoint_smem(int N, int vp, int T) {
@@ -481,10 +469,7 @@ int launch_adjoint(const AdjArgs &a, int vp, double *out, hipStream_t st) {
     void *kargs[] = {&args};
     NISE_HIP_CHECK(hipLaunchKernel(fn, dim3(a.nwg), dim3(64), kargs, smem, st));
   }
-  hipLaunchKernelGGL(adjoint_reduce_kernel, dim3((a.N + 1 + 127) / 128), dim3(128), 0, st,
-                     a.part_delta, a.part_c, a.nwg, a.N, out);
-  NISE_HIP_CHECK(hipGetLastError());
-  return NISE_OK;
+  return launch_adjoint_reduce(a.part_delta, a.part_c, a.nwg, a.N, out, st);
 }
 
 // Vectors per workgroup: one rotation lane per rotation of an average layer,

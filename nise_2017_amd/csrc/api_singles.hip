@@ -43,6 +43,8 @@ struct nise_abs_plan {
   bool dense = false;   // per-frame propagators instead of the row conveyor (dense.hip)
   RowsArgs row_desc;    // the uploaded descriptor
   DevBuf U, dsys, dmap;
+  int chain = 0;        // lanes per vector of the chain kernels (chain.hip), 0: not used
+  DevBuf rec;
   bool row_pf = false;  // the row conveyor prefetches each frame's first site batch
   int nsteps = 0;
   DevBuf ws_cs, resp_plain;
@@ -138,7 +140,9 @@ int build_rows(nise_abs_plan *P) {
   P->nwg = (3 * (P->end - P->begin) + G - 1) / G;
   P->npart = 3 * (P->end - P->begin);  // one row per vector
   if ((rc = P->partial.alloc((size_t)std::max(P->npart, 1) * P->tmax * sizeof(double2)))) return rc;
-  return upload_rows_desc(P);
+  if ((rc = upload_rows_desc(P))) return rc;
+  if (P->chain && !P->dense) P->nwg = chain_groups(P->npart, P->chain);
+  return NISE_OK;
 }
 
 // Slot assignment: consecutive samples, three polarisations each, spw
@@ -174,8 +178,26 @@ int build_slots(nise_abs_plan *P) {
   return NISE_OK;
 }
 
+// Descriptor of the chain kernels.
+ChainArgs chain_args(nise_abs_plan *P) {
+  ChainArgs a;
+  a.N = P->N, a.T = P->tmax, a.m = P->m, a.nvec = 3 * (P->end - P->begin), a.begin = P->begin, a.sample = P->sample;
+  a.f_lo = P->f_lo, a.fac = trotter_factor(P->non.deltat, 1, P->m);
+  a.rec = P->rec.as<float4>(), a.partial = P->partial.as<double2>();
+  if (P->every) {
+    a.hist = P->ck.as<float2>(), a.hist_every = a.every = P->every, a.nck = P->nck;
+    a.ck = P->ck.as<float2>(), a.g = P->gtab.as<float2>();
+  }
+  return a;
+}
+
 int run_tables(nise_abs_plan *P) {
   float fac = trotter_factor(P->non.deltat, 1, P->m);
+  if (P->chain && (!P->dense || P->every)) {
+    const int rc = launch_chain_tables(P->src, P->N, P->f_lo, P->f_hi - P->f_lo, fac, P->mu_dev, P->mu_stride,
+                                       P->rec.as<float4>(), P->st);
+    if (rc || !P->dense) return rc;
+  }
   return launch_frame_tables(P->src, P->N, P->sch, P->ab.as<uint32_t>(), fac, P->f_lo,
                              P->f_hi - P->f_lo, P->diag.as<float2>(), P->cs.as<float2>(), P->st,
                              P->every ? P->jf.as<float>() : nullptr);
@@ -187,6 +209,7 @@ int run_conveyor(nise_abs_plan *P) {
     if (rc) return rc;
     return launch_dense(dense_class(P->N), P->dsys.as<DiaSys>(), P->dmap.as<int2>(), P->nwg, P->st, nullptr);
   }
+  if (P->chain) return launch_chain(chain_args(P), P->chain, P->st);
   if (P->rows)
     return launch_rows(P->row_sys.as<RowsArgs>(), P->row_wmap.as<int2>(), P->nwg, P->rows, P->row_pf, P->row_smem,
                        P->st);
@@ -370,7 +393,9 @@ static int plan_create(nise_abs_plan **out, const t_non *non, const float *H_rec
     P->vp = 16, P->spw = 5;
     P->rows = rows_for(N, P->sch_asap.Kreal, P->sch_asap.nlayers());
     P->mask = mask;
-    P->dense = dense_pays(N, P->tmax, P->end - P->begin, nfr, P->sch_asap.Kreal, P->sch_asap.nlayers(), P->m);
+    if (chain_mask(N, mask)) P->chain = chain_rows(N, P->tmax, P->m, 3 * (int64_t)(P->end - P->begin), nfr);
+    P->dense = !P->chain && dense_pays(N, P->tmax, P->end - P->begin, nfr, P->sch_asap.Kreal, P->sch_asap.nlayers(), P->m);
+    if (P->chain && (rc = P->rec.alloc((size_t)nfr * N * 2 * sizeof(float4)))) return rc;
     P->packed = P->dense && one_run;  // a run made once does not pay for the list schedule
     if (P->packed) pack_schedule_rows(P->sch_asap, P->rows, P->sch_rows);
     else build_schedule_rows(N, mask, P->rows, P->sch_rows);
@@ -409,7 +434,7 @@ extern "C" int nise_abs_plan_set_shape(nise_abs_plan *P, int vp, int samples_per
       !(block == 64 || block == 256 || block == 512 || block == -2 || block == -4) ||
       (block > 0 && vp > block))
     return set_error("bad shape vp=%d spw=%d block=%d", vp, samples_per_wg, block), NISE_ERR_ARG;
-  P->vp = vp, P->spw = samples_per_wg, P->block = block, P->rows = 0, P->dense = false;
+  P->vp = vp, P->spw = samples_per_wg, P->block = block, P->rows = 0, P->dense = false, P->chain = 0;
   if (P->graph_ready) {
     (void)hipGraphExecDestroy(P->exec), (void)hipGraphDestroy(P->graph);
     P->exec = nullptr, P->graph = nullptr, P->graph_ready = false;
@@ -428,7 +453,7 @@ extern "C" int nise_abs_plan_set_rows(nise_abs_plan *P, int R) {
   if (rows_smem(P->N, R) > 160 * 1024)
     return set_error("N=%d does not fit the row conveyor with %d rows", P->N, R), NISE_ERR_ARG;
   if (R != P->rows || P->packed || P->sch_rows.ab.empty()) build_schedule_rows(P->N, P->mask, R, P->sch_rows);
-  P->rows = R, P->dense = P->packed = false;
+  P->rows = R, P->dense = P->packed = false, P->chain = 0;
   if (P->graph_ready) {
     (void)hipGraphExecDestroy(P->exec), (void)hipGraphDestroy(P->graph);
     P->exec = nullptr, P->graph = nullptr, P->graph_ready = false;
@@ -646,7 +671,18 @@ extern "C" int nise_abs_plan_adjoint(nise_abs_plan *P, const float *g_re, const 
   a.part_delta = P->part_d.as<double>(), a.part_c = P->part_c.as<double>();
   NISE_HIP_CHECK(hipEventRecord(P->ev[0], P->st));
   int rc;
-  if (P->rows) {  // time-skewed row variant on the row conveyor's tables
+  if (P->chain) {
+    // (sizes beyond the row variant's LDS stay refused, whichever kernel runs)
+    if (adjoint_rows_smem(N, P->rows) > 160 * 1024)
+      return set_error("adjoint: N=%d needs %zu B of LDS", N, adjoint_rows_smem(N, P->rows)), NISE_ERR_ARG;
+    ChainArgs r = chain_args(P);
+    const int nwg = chain_groups(r.nvec, P->chain);
+    if ((rc = P->part_d.alloc((size_t)std::max(nwg, 1) * N * 8)) ||
+        (rc = P->part_c.alloc((size_t)std::max(nwg, 1) * 8)))
+      return rc;
+    r.part_delta = P->part_d.as<double>(), r.part_c = P->part_c.as<double>();
+    rc = launch_chain_adjoint(r, P->chain, P->grad.as<double>(), P->st);
+  } else if (P->rows) {  // time-skewed row variant on the row conveyor's tables
     AdjRowsArgs r;
     r.N = N, r.T = T, r.m = P->m, r.nlayers = P->sch.nlayers(), r.every = P->every, r.nck = P->nck;
     r.nvec = 3 * (P->end - P->begin), r.begin = P->begin, r.sample = P->sample;

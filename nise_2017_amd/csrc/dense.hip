@@ -272,10 +272,11 @@ int launch_dense(int cls, const DiaSys *sys, const int2 *wmap, int nwg, hipStrea
 // each other) and one product per vector step, against rotation sweeps on
 // every vector step.  A conveyor wave walks tmax frames of nlayers dependent
 // LDS round trips, so runs with few waves are far from its throughput.  The
-// cycle counts are fits: measured (conveyor and this, ms) N = 16 chain, 200
-// and 1,000 samples 0.45 and 0.13, 0.47 and 0.25; N = 77 lattice, 333 samples
-// 2.60 and 1.05; N = 64 lattice, 800 samples 2.43 and 1.24, 1,500 samples 2.72
-// (conveyor; 3.4); N = 121 lattice, 800 samples 4.50 and 4.41.
+// cycle counts are fits: measured (conveyor and this, ms) N = 25 lattice,
+// 1,500 samples 1.56 and 0.59; N = 77 lattice, 333 samples 2.60 and 1.05;
+// N = 64 lattice, 800 samples 2.43 and 1.24, 1,500 samples 2.72 (conveyor;
+// 3.4); N = 121 lattice, 800 samples 4.50 and 4.41.  Nearest-neighbour chains
+// do not come here (chain.hip).
 // Kreal, nasap: rotations and layers of the layered schedule; m: Trotter
 // substeps; F: frames; S: samples.
 bool dense_pays(int N, int T, int64_t S, int64_t F, int Kreal, int nasap, int m) {

@@ -467,10 +467,11 @@ struct SysState {
   int N = 0, T = 0, dia = 0, nvec = 0, nwg = 0;  // nwg: rows of partial responses
   int Rk = 0;          // rows of a Trotter system in this call
   bool dense = false;  // Trotter system through per-frame propagators
+  int chain = 0;       // lanes per vector of a nearest-neighbour chain's kernel, 0: not one
   float thres = 0.f;  // sparse DIA threshold (0: full DIA)
   int64_t f_lo = 0, f_hi = 0;
   FrameSource src;
-  DevBuf H, mu, C, shs, sha, ab, diag, cs, steps, U, partial;
+  DevBuf H, mu, C, shs, sha, ab, diag, cs, steps, U, rec, partial;
   const float *mu_dev = nullptr;
   int64_t mu_stride = 0;
   Schedule sch_asap, sch;
@@ -485,6 +486,7 @@ struct SysState {
   void reset() {
     N = T = dia = nvec = nwg = 0;
     dense = false;
+    chain = 0;
     thres = 0.f;
     f_lo = f_hi = 0;
     src = FrameSource();
@@ -654,7 +656,8 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
   //    second stream, queued before the host builds the Trotter schedules so
   //    that the two overlap
   std::vector<RowsArgs> rows;
-  std::vector<int> rows_of;
+  std::vector<int> rows_of, chain_of;
+  std::vector<ChainArgs> chains;
   std::vector<DiaSys> dias;
   std::vector<int> dia_of;
   std::vector<ExpmJob> jobs;
@@ -736,6 +739,8 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
     const t_non *non = systems[k].non;
     if (s.dia) continue;
     s.Rk = R > 0 ? R : rows_for(s.N, s.sch_asap.Kreal, s.sch_asap.nlayers(), cap);
+    s.chain = own && chain_mask(s.N, s.mask) ? chain_rows(s.N, s.T, non->ts, s.nvec, s.f_hi - s.f_lo) : 0;
+    if (s.chain) continue;
     s.dense = own && dense_pays(s.N, s.T, s.nvec / 3, s.f_hi - s.f_lo, s.sch_asap.Kreal, s.sch_asap.nlayers(), non->ts);
     if (s.rows_N != s.N || s.rows_R != s.Rk || s.rows_packed != s.dense || s.rows_mask != s.mask) {
       s.rows_N = 0;  // until the tables below are on the device
@@ -756,6 +761,20 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
     const int N = s.N, Rk = s.Rk;
     const int64_t nfr = s.f_hi - s.f_lo;
     if (s.dia) continue;
+    if (s.chain) {
+      const float fac = trotter_factor(non->deltat, 1, non->ts);
+      s.nwg = s.nvec;
+      if ((rc = s.rec.alloc((size_t)nfr * N * 2 * sizeof(float4))) ||
+          (rc = s.partial.alloc((size_t)s.nwg * s.T * sizeof(double2))) ||
+          (rc = launch_chain_tables(s.src, N, s.f_lo, nfr, fac, s.mu_dev, s.mu_stride, s.rec.as<float4>(), st)))
+        return rc;
+      ChainArgs c;
+      c.N = N, c.T = s.T, c.m = non->ts, c.nvec = s.nvec, c.begin = non->begin, c.sample = non->sample;
+      c.f_lo = s.f_lo, c.fac = fac, c.rec = s.rec.as<float4>(), c.partial = s.partial.as<double2>();
+      chains.push_back(c);
+      chain_of.push_back(k);
+      continue;
+    }
       if ((rc = s.diag.alloc((size_t)nfr * N * 8)) || (rc = s.cs.alloc((size_t)nfr * s.sch.K * 8))) return rc;
       if ((rc = launch_frame_tables(s.src, N, s.sch, s.ab.as<uint32_t>(), trotter_factor(non->deltat, 1, non->ts),
                                     s.f_lo, nfr, s.diag.as<float2>(), s.cs.as<float2>(), st)))
@@ -809,7 +828,9 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
       return set_error("multi: DIA window of %d steps is too long for N=%d", dias[i].tmax, dias[i].N), NISE_ERR_ARG;
   }
   DevBuf &rsys = cache.rsys, &rwm = cache.rwm, &dsys = cache.dsys, &dwm = cache.dwm, &times = cache.times;
-  const size_t nt = rmap.size() + dmap.size();
+  size_t nt = rmap.size() + dmap.size();
+  std::vector<size_t> cend;  // ends of the chains' times
+  for (size_t i = 0; i < chains.size(); ++i) cend.push_back(nt += chain_groups(chains[i].nvec, S[chain_of[i]]->chain));
   if ((rc = up(rsys, rows.data(), rows.size() * sizeof(RowsArgs))) ||
       (rc = up(rwm, rmap.data(), rmap.size() * sizeof(int2))) ||
       (rc = up(dsys, dias.data(), dias.size() * sizeof(DiaSys))) ||
@@ -826,6 +847,11 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
     hipError_t e1 = hipEventRecord(ev, sd), e2 = e1 == hipSuccess ? hipStreamWaitEvent(st, ev, 0) : e1;
     (void)hipEventDestroy(ev);
     NISE_HIP_CHECK(e2);
+  }
+  for (size_t i = 0; i < chains.size(); ++i) {
+    const int Rc = S[chain_of[i]]->chain;
+    chains[i].times = tm + 2 * (cend[i] - chain_groups(chains[i].nvec, Rc));
+    if ((rc = launch_chain(chains[i], Rc, st))) return rc;
   }
   if (!rmap.empty() && (rc = launch_rows(rsys.as<RowsArgs>(), rwm.as<int2>(), (int)rmap.size(), R, rpf, rsmem, st, tm)))
     return rc;
@@ -885,6 +911,8 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
       const int k = dia_of[dmap[i].x];
       done[k] = std::max(done[k], ht[2 * (rmap.size() + i) + 1]);
     }
+    for (size_t i = 0, w = rmap.size() + dmap.size(); i < chains.size(); ++i)
+      for (; w < cend[i]; ++w) done[chain_of[i]] = std::max(done[chain_of[i]], ht[2 * w + 1]);
     for (int k = 0; k < nsys; ++k) done_ms[k] = khz > 0 ? (double)(done[k] - t0) / khz : -1.0;
   }
   return NISE_OK;

@@ -301,6 +301,27 @@ __device__ __forceinline__ void rotate_pair(float2 &pa, float2 &pb, float co, fl
   pb = make_float2(cr2, ci2);
 }
 
+// Their inverses, for the adjoints.
+__device__ __forceinline__ float2 cmul_conj_d(float2 p, float2 d) {
+  // p * conj(d), d = (cos, -sin): the inverse of the reference's
+  // (cr*re - ci*im, ci*re + cr*im) product with d
+  return make_float2(__fadd_rn(__fmul_rn(p.x, d.x), __fmul_rn(p.y, d.y)),
+                     __fsub_rn(__fmul_rn(p.y, d.x), __fmul_rn(p.x, d.y)));
+}
+
+__device__ __forceinline__ void rotate_back(float2 &pa, float2 &pb, float co, float si) {
+  // R^dagger: the forward rotation of src/propagate.c:883-887 with -si
+  const float ar = __fadd_rn(__fmul_rn(co, pa.x), __fmul_rn(si, pb.y));
+  const float ai = __fsub_rn(__fmul_rn(co, pa.y), __fmul_rn(si, pb.x));
+  const float br = __fadd_rn(__fmul_rn(co, pb.x), __fmul_rn(si, pa.y));
+  const float bi = __fsub_rn(__fmul_rn(co, pb.y), __fmul_rn(si, pa.x));
+  pa = make_float2(ar, ai);
+  pb = make_float2(br, bi);
+}
+
+// Im(conj(x) y)
+__device__ __forceinline__ float im_cj(float2 x, float2 y) { return x.x * y.y - x.y * y.x; }
+
 // Reference time factor f = deltat*icm2ifs*twoPi*sign/m (src/propagate.c:836).
 inline float trotter_factor(float deltat, int sign, int m) {
   volatile float f = deltat * kIcm2ifs;
@@ -545,6 +566,31 @@ struct AdjArgs {
 int launch_adjoint(const AdjArgs &a, int vp, double *out, hipStream_t st);
 
 // Row variant of the adjoint (the row conveyor's schedule and tables).
+// Nearest-neighbour chains (chain.hip): forward needs rec and partial,
+// backward rec, ck, g and the gradient partials (one row per workgroup).
+struct ChainArgs {
+  int N = 0, T = 0, m = 1, nvec = 0, begin = 0, sample = 1, every = 1, nck = 0;
+  int64_t f_lo = 0;
+  float fac = 0.f;
+  const float4 *rec = nullptr;  // [rows][N][2]
+  double2 *partial = nullptr;   // [vectors][T]
+  float2 *hist = nullptr;       // checkpoints, as RowsArgs
+  int hist_every = 1;
+  unsigned long long *times = nullptr;  // forward: device clock at start and end, per workgroup
+  const float2 *ck = nullptr, *g = nullptr;
+  double *part_delta = nullptr, *part_c = nullptr;
+};
+// Whether every kept pair joins neighbours (and there is one).
+bool chain_mask(int N, const std::vector<uint8_t> &mask);
+// Lanes per vector, or 0 where the tables or LDS do not take the run.
+int chain_rows(int N, int T, int m, int64_t nvec, int64_t nfr);
+inline int chain_groups(int nvec, int R) { return (nvec + 64 / R - 1) / (64 / R); }
+int launch_chain_tables(const FrameSource &src, int N, int64_t f_lo, int64_t nfr, float fac, const float *mu_rec,
+                        int64_t mu_stride, float4 *rec, hipStream_t st);
+int launch_chain(const ChainArgs &a, int R, hipStream_t st);
+int launch_chain_adjoint(const ChainArgs &a, int R, double *out, hipStream_t st);
+size_t adjoint_rows_smem(int N, int R);
+int launch_adjoint_reduce(const double *pd, const double *pc, int nwg, int N, double *out, hipStream_t st);
 struct AdjRowsArgs {
   int N = 0, T = 0, m = 1, nlayers = 0, every = 1, nck = 0, nvec = 0, begin = 0, sample = 1;
   int64_t K = 0, f_lo = 0;

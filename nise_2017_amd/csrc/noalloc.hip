@@ -152,6 +152,42 @@ int run_dense(unsigned char *base, size_t used, const FrameSource &src, RowsArgs
   return NISE_OK;
 }
 
+// A nearest-neighbour chain through its own kernel (chain.hip) in windows of
+// as many samples as the array holds, bit for bit the plan's partial rows.
+// ran stays false where one sample's records do not fit: the caller's row
+// conveyor gives the same results.
+int run_chain(unsigned char *base, size_t used, const FrameSource &src, const RowsArgs &r, int R, int ns, float fac,
+              float *re_S, float *im_S, bool &ran) {
+  int rc;
+  const hipStream_t st = nullptr;
+  const int N = r.N, T = r.tmax;
+  Arena ar{base, used};
+  double2 *partial = ar.take<double2>((size_t)3 * ns * T);
+  float *out = ar.take<float>(2 * (size_t)T);
+  if (!partial || !out) return NISE_OK;
+  auto frames = [&](int n) { return (int64_t)(n - 1) * r.sample + T; };
+  auto bytes = [&](int n) { return Arena::bytes_of((size_t)frames(n) * N, 2 * sizeof(float4)); };
+  int per = ns;
+  while (per && ar.used + bytes(per) > kScratchBytes) per = per > 16 ? per * 7 / 8 : per - 1;
+  if (!per) return NISE_OK;
+  float4 *rec = ar.take<float4>((size_t)frames(per) * N * 2);
+  if (!rec) return NISE_OK;
+  ran = true;
+  for (int s0 = 0; s0 < ns; s0 += per) {  // one stream: a window's tables wait for the previous window
+    const int n = std::min(per, ns - s0);
+    ChainArgs c;
+    c.N = N, c.T = T, c.m = r.m, c.nvec = 3 * n, c.begin = r.begin + s0, c.sample = r.sample, c.fac = fac;
+    c.f_lo = (int64_t)c.begin * r.sample, c.rec = rec, c.partial = partial + (size_t)3 * s0 * T;
+    if ((rc = launch_chain_tables(src, N, c.f_lo, frames(n), fac, r.mu_rec, r.mu_stride, rec, st)) ||
+        (rc = launch_chain(c, R, st)))
+      return rc;
+  }
+  if ((rc = launch_reduce_partials(partial, 3 * ns, T, out, out + T, st))) return rc;
+  NISE_HIP_CHECK(hipMemcpy(re_S, out, T * sizeof(float), hipMemcpyDeviceToHost));
+  NISE_HIP_CHECK(hipMemcpy(im_S, out + T, T * sizeof(float), hipMemcpyDeviceToHost));
+  return NISE_OK;
+}
+
 }  // namespace
 
 extern "C" int nise_absorption_batched_noalloc(const t_non *non, const float *H_rec, int64_t H_stride,
@@ -255,7 +291,11 @@ extern "C" int nise_absorption_batched_noalloc(const t_non *non, const float *H_
   bool pf = false;
   if ((rc = rows_prepare(&r, 1, R, wmap, smem, pf))) return rc;
   if ((int)wmap.size() != nwg) return set_error("row conveyor: workgroup map mismatch"), NISE_ERR_ARG;
-  if (dense_pays(N, T, end - begin, nfr, asap.Kreal, asap.nlayers(), m))
+  if (const int Rc = chain_mask(N, mask) ? chain_rows(N, T, m, nvec, nfr) : 0) {
+    bool ran = false;
+    if ((rc = run_chain(ds->ptr, ar0, src, r, Rc, end - begin, trotter_factor(non->deltat, 1, m), re_S, im_S, ran)) || ran)
+      return rc;
+  } else if (dense_pays(N, T, end - begin, nfr, asap.Kreal, asap.nlayers(), m))
     return run_dense(ds->ptr, ar0, src, r, asap, R, end - begin, trotter_factor(non->deltat, 1, m), re_S, im_S);
   if (!tab.empty()) NISE_HIP_CHECK(hipMemcpy(steps, tab.data(), tab.size() * sizeof(uint2), hipMemcpyHostToDevice));
   if (!ab.empty()) NISE_HIP_CHECK(hipMemcpy(abd, ab.data(), ab.size() * 4, hipMemcpyHostToDevice));
