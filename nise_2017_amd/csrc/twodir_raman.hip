@@ -160,16 +160,19 @@ __host__ __device__ inline size_t raman_contract_smem(int N) {
 // Diagram 1 at t3 (src/calc_2DIRraman.c:306-330): per (s, x1) the contraction
 // of fr[x1] with the six components, then for every item with this x1 and
 // every t1 the dot with rightrr = conj(L[x0][t1]) at t3 (at t3 = 0 without
-// the t3 propagation of fr and rightrr)
-__global__ void raman_d1_kernel(RamanArgs A, int t3) {
+// the t3 propagation of fr and rightrr).  frh: the fr vectors at every t3 (one
+// launch, t3 in blockIdx.y); else the fr state at t3 + blockIdx.y
+__global__ void raman_d1_kernel(RamanArgs A, int t3, const float2 *frh) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int N = A.N, N2 = N * (N + 1) / 2, T1 = A.T1, T3 = A.T3;
+  t3 += blockIdx.y;
   const int s = blockIdx.x / 3, x1 = blockIdx.x % 3;
+  const float2 *src = frh ? frh + (((int64_t)t3 * A.S + s) * 3 + x1) * N2 : A.dbl + fr_vec(A, s, x1) * N2;
   float *dipL = reinterpret_cast<float *>(smem), *ovL = dipL + 3 * N;
   float2 *psi = reinterpret_cast<float2 *>(smem + (((size_t)6 * N * 4 + 15) & ~(size_t)15));
   float2 *outL = psi + N2;
   const int64_t tl = r_tj(A, s) + t3;
-  for (int j = threadIdx.x; j < N2; j += blockDim.x) psi[j] = gld(A.dbl + fr_vec(A, s, x1) * N2 + j);
+  for (int j = threadIdx.x; j < N2; j += blockDim.x) psi[j] = gld(src + j);
   __syncthreads();
   raman_contract6(A, tl, psi, dipL, ovL, outL);
   const int nrow = 3 * T1 + 3, tr = A.p1 ? t3 : 0;
@@ -239,6 +242,11 @@ __global__ void raman_d2_kernel(RamanArgs A, int t3) {
 // every item with this x0 the k-th rounded dot term against conj(M[x1](t3))
 // at once, the sums over k in ascending order (the reference's operation
 // sequence, as raman_d2_kernel), then the doubles step of frame tj + t3.
+// With frh, the first S workgroups run the fr vectors instead (sqrt2 mu_x1(tj)
+// on |aa>, one in slot 0 of each wave) and write them at every t3, so that
+// diagram 1 is one launch over all t3: a launch per t3 and per doubles step, 25
+// and 16 us of latency each, took 2.0 of the 6.16 ms of N = 24, 100 samples, T1
+// = T3 = 48; 4.31 ms now, of which diagram 1 0.19.
 struct RamanPersistArgs {
   RamanArgs A;
   int K2 = 0, m = 1;
@@ -246,6 +254,7 @@ struct RamanPersistArgs {
   const float2 *D2 = nullptr;     // [frame - f_lo][N2]
   const float4 *cs2 = nullptr;    // [frame - f_lo][K2]
   int64_t f_lo = 0;
+  float2 *frh = nullptr;          // [T3][S][3][N2], or null
 };
 constexpr int kRamanItemBatch = 2;  // items whose dot terms share the LDS rows
 struct RamanLayout {
@@ -282,7 +291,9 @@ __global__ void __launch_bounds__(192) raman_persist_kernel(RamanPersistArgs P) 
   const RamanArgs &A = P.A;
   const int N = A.N, N2 = N * (N + 1) / 2, T1 = A.T1, T3 = A.T3, K2 = P.K2, t = threadIdx.x;
   const int wave = t >> 6, lane = t & 63, x0 = wave;
-  const int nblk = (T1 + VW - 1) / VW, s = blockIdx.x / nblk, t1a = (blockIdx.x % nblk) * VW;
+  const int nfr = P.frh ? A.S : 0, blk = (int)blockIdx.x - nfr;
+  const bool fr = blk < 0;
+  const int nblk = (T1 + VW - 1) / VW, s = fr ? blockIdx.x : blk / nblk, t1a = fr ? 0 : blk % nblk * VW;
   const int nv = min(VW, T1 - t1a);
   const RamanLayout Ly = raman_layout(N, VW, K2);
   uint2 *ixL = reinterpret_cast<uint2 *>(smem + Ly.ix);
@@ -309,6 +320,18 @@ __global__ void __launch_bounds__(192) raman_persist_kernel(RamanPersistArgs P) 
       dbl_diag<VW>(psi, d2, N2, lane);
     }
   };
+  if (fr) {
+    const float *mu = r_mu(A, tj, x0);
+    for (int a = lane; a < N; a += 64)
+      psi[((a * (2 * N - a + 1)) >> 1) * VW] = make_float2(__fmul_rn(kSqrt2, mu[a]), 0.f);
+    asm volatile("" ::: "memory");
+    for (int t3 = 0;; ++t3) {
+      float2 *d = P.frh + (((int64_t)t3 * A.S + s) * 3 + x0) * N2;
+      for (int j = lane; j < N2; j += 64) gst(d + j, psi[j * VW]);
+      if (t3 + 1 == T3) return;
+      step(tj + t3);
+    }
+  }
   // (1) formation and the t1 steps
   for (int64_t f = tj - (t1a + nv - 1); f <= tj; ++f) {
     const int qi = (int)(tj - f) - t1a;  // the slot formed at f
@@ -528,7 +551,7 @@ bool tech_eq(const t_non *n, const char *t) { return strcmp(n->technique, t) == 
 // Device buffers of the calling thread's Raman runs, kept between calls.
 struct RamanBufs {
   DevBuf Hb, mub, Cb, Alb, mk, ab, lay, diag, cs, ab2, D2, cs2, stp, wpl, ltb, Rd;
-  DevBuf L0, hist, dbl, t1n, h3, E, part, slots, wgb, slots2, wgb2, slots3, wgb3, gvb, gvc, grow, tvb, tvc, trow;
+  DevBuf L0, hist, dbl, frh, t1n, h3, E, part, slots, wgb, slots2, wgb2, slots3, wgb3, gvb, gvc, grow, tvb, tvc, trow;
 };
 
 // Groups of at most vw consecutive vectors [first, first + n): begins and
@@ -674,16 +697,19 @@ extern "C" int nise_2dirraman_batched(const t_non *non, const float *H_rec, int6
     return rc;
   NISE_HIP_CHECK(hipMemsetAsync(B.Rd.p, 0, (size_t)12 * plane * 8, st));
 
-  const int total = end - begin, nrow = 3 * T1 + 3;
-  const double per_sample = 8.0 * 3 * T1 * N + 8.0 * nrow * T3 * N + 8.0 * (3 * T1 + 3) * N2 + 8.0 * 9 * T1 * N +
-                            8.0 * 9 * T1 * T3 * N + 4.0 * 126 * plane;
-  const int chunk = (int)std::max(1.0, std::min<double>({(double)total, 1024.0, 8.0e9 / per_sample}));
-  const int vw = doubles_vw(N);
   // the kII vectors stay in LDS for all their frames (raman_persist_kernel)
   // when their states, rotation table and rows fit
   const int pnp = doubles_np(N);
   const size_t psm = raman_layout(N, 64 / pnp, (int)lex.size()).total;
   const bool pers = k2 && rot_table_fits(N, 64 / pnp, (int)lex.size()) && psm <= 160 * 1024;
+  // ... and so do diagram 1's fr vectors, in the same launch
+  const bool frh = pers && k1 && p1;
+  const int total = end - begin, nrow = 3 * T1 + 3;
+  const double per_sample = 8.0 * 3 * T1 * N + 8.0 * nrow * T3 * N + 8.0 * (3 * T1 + 3) * N2 + 8.0 * 9 * T1 * N +
+                            8.0 * 9 * T1 * T3 * N + 4.0 * 126 * plane +
+                            (frh ? 24.0 * T3 * N2 : 0.0);
+  const int chunk = (int)std::max(1.0, std::min<double>({(double)total, 1024.0, 8.0e9 / per_sample}));
+  const int vw = doubles_vw(N);
   const size_t csm = raman_contract_smem(N);
   NISE_HIP_CHECK(hipFuncSetAttribute((const void *)raman_d1_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)csm));
   NISE_HIP_CHECK(hipFuncSetAttribute((const void *)raman_d2_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)csm));
@@ -771,7 +797,9 @@ extern "C" int nise_2dirraman_batched(const t_non *non, const float *H_rec, int6
                                  : (const void *)raman_persist_kernel<64>;
       NISE_HIP_CHECK(hipFuncSetAttribute(fp, hipFuncAttributeMaxDynamicSharedMemorySize, (int)psm));
       void *kargs[] = {&pa};
-      const int nblk = (T1 + 64 / pnp - 1) / (64 / pnp);
+      const int nblk = (T1 + 64 / pnp - 1) / (64 / pnp) + (frh ? 1 : 0);
+      if (frh && (rc = B.frh.alloc((size_t)T3 * S * 3 * N2 * 8))) return rc;
+      pa.frh = frh ? B.frh.as<float2>() : nullptr;
       NISE_HIP_CHECK(hipLaunchKernel(fp, dim3((unsigned)(S * nblk)), dim3(192), kargs, psm, st));
     } else if (k2) {
       std::vector<int> vb, vc;
@@ -800,7 +828,7 @@ extern "C" int nise_2dirraman_batched(const t_non *non, const float *H_rec, int6
       hipLaunchKernelGGL(raman_inject_kernel, dim3(S * 3), dim3(256), 0, st, A, 0, 0);
       NISE_HIP_CHECK(hipGetLastError());
     }
-    if (k1) {
+    if (k1 && !frh) {
       hipLaunchKernelGGL(raman_inject_kernel, dim3(S * 3), dim3(256), 0, st, A, 0, 1);
       NISE_HIP_CHECK(hipGetLastError());
     }
@@ -813,14 +841,14 @@ extern "C" int nise_2dirraman_batched(const t_non *non, const float *H_rec, int6
     std::vector<int> gvb, gvc;
     for (int s = 0; s < S; ++s) {
       if (d2 && !pers) split_groups((int64_t)s * T1 * 3, 3 * T1, vw, gvb, gvc);
-      if (p1 && k1) split_groups((int64_t)S * T1 * 3 + s * 3, 3, vw, gvb, gvc);
+      if (p1 && k1 && !frh) split_groups((int64_t)S * T1 * 3 + s * 3, 3, vw, gvb, gvc);
     }
     const int G = (int)gvb.size();
     std::vector<int64_t> grow((size_t)std::max(T3 - 1, 0) * G);
     {
       int g = 0;
       for (int s = 0; s < S; ++s) {
-        const int ng = (d2 && !pers ? (3 * T1 + vw - 1) / vw : 0) + (p1 && k1 ? (3 + vw - 1) / vw : 0);
+        const int ng = (d2 && !pers ? (3 * T1 + vw - 1) / vw : 0) + (p1 && k1 && !frh ? (3 + vw - 1) / vw : 0);
         for (int j = 0; j < ng; ++j, ++g)
           for (int t3 = 0; t3 + 1 < T3; ++t3) grow[(size_t)t3 * G + g] = tj_of(s) + t3 - f_lo;
       }
@@ -829,9 +857,18 @@ extern "C" int nise_2dirraman_batched(const t_non *non, const float *H_rec, int6
         ((rc = upr(B.gvb, gvb.data(), gvb.size() * 4)) || (rc = upr(B.gvc, gvc.data(), gvc.size() * 4)) ||
          (rc = upr(B.grow, grow.data(), grow.size() * 8))))
       return rc;
-    for (int t3 = 0; t3 < T3; ++t3) {
-      if (k1) {
-        hipLaunchKernelGGL(raman_d1_kernel, dim3(S * 3), dim3(64), csm, st, A, t3);
+    // diagram 1 of all t3 at once from the fr vectors' history, or from an fr
+    // state that t3 does not change; with nothing left per t3, one pass
+    const bool d1_once = frh || !p1;
+    for (int t3 = 0; k1 && d1_once && t3 < T3; t3 += 65535) {
+      hipLaunchKernelGGL(raman_d1_kernel, dim3(S * 3, std::min(T3 - t3, 65535)), dim3(64), csm, st, A, t3,
+                         frh ? B.frh.as<float2>() : nullptr);
+      NISE_HIP_CHECK(hipGetLastError());
+    }
+    const bool per_t3 = (k1 && !d1_once) || (d2 && !pers) || G;
+    for (int t3 = 0; per_t3 && t3 < T3; ++t3) {
+      if (k1 && !d1_once) {
+        hipLaunchKernelGGL(raman_d1_kernel, dim3(S * 3), dim3(64), csm, st, A, t3, (const float2 *)nullptr);
         NISE_HIP_CHECK(hipGetLastError());
       }
       if (d2 && !pers) {
