@@ -25,6 +25,8 @@
 // Arithmetic: compiled with -ffp-contract=off so products and sums round
 // exactly as the reference's x86-64 SSE code (no FMA) does.
 
+#include <algorithm>
+
 #include "nise_internal.h"
 
 namespace nise {
@@ -35,8 +37,13 @@ namespace nise {
 // Workgroup of 256 threads: kMaskPairs consecutive pairs (a row segment of
 // a frame per load) x kMaskLanes frame lanes; lane fl reads frames fl, fl +
 // kMaskLanes, ..., kMaskInflight of them in flight, and stops at the first
-// kept coupling.  The lanes' flags are ORed in LDS.
-constexpr int kMaskPairs = 32, kMaskLanes = 8, kMaskInflight = 8;
+// kept coupling.  The lanes' flags are ORed in LDS.  Small systems have few
+// pairs for many frames (and pairs that are never kept are read in all of
+// them), so the frames are split over blockIdx.y until kMaskGroups workgroups
+// run, at least one batch of frames each; the flags then start at zero and a
+// group only ever stores ones (N = 32 ring, 2,118 frames: 116 us in one group
+// per pair block, 12 us so).
+constexpr int kMaskPairs = 32, kMaskLanes = 8, kMaskInflight = 8, kMaskGroups = 512;
 // (a, b) of the lexicographic pair index p (a < b < N): the row from the
 // quadratic's root, then corrected in integers (row a starts at a (2N - a -
 // 1) / 2).  A walk along the rows took up to N steps per thread.
@@ -62,7 +69,7 @@ __global__ void __launch_bounds__(256) union_mask_static_kernel(FrameSource s, i
 }
 
 __global__ void __launch_bounds__(256) union_mask_kernel(FrameSource s, int N, int64_t f_lo, int64_t nfr,
-                                                         uint8_t *mask) {
+                                                         int64_t per, uint8_t *mask) {
   __shared__ uint8_t kk[kMaskLanes][kMaskPairs];
   const int tp = threadIdx.x % kMaskPairs, fl = threadIdx.x / kMaskPairs;
   const int64_t npair = (int64_t)N * (N - 1) / 2;
@@ -71,8 +78,8 @@ __global__ void __launch_bounds__(256) union_mask_kernel(FrameSource s, int N, i
   if (p < npair) {
     int a, b;
     pair_of(p, N, a, b);
-    const int64_t nf = s.coupling_type ? 1 : nfr;
-    for (int64_t f0 = fl; f0 < nf && !keep; f0 += (int64_t)kMaskLanes * kMaskInflight) {
+    const int64_t nf = min(nfr, (int64_t)(blockIdx.y + 1) * per);  // this group's frames: y per .. nf - 1
+    for (int64_t f0 = (int64_t)blockIdx.y * per + fl; f0 < nf && !keep; f0 += (int64_t)kMaskLanes * kMaskInflight) {
       float v[kMaskInflight];
 #pragma unroll
       for (int u = 0; u < kMaskInflight; ++u) {
@@ -88,8 +95,13 @@ __global__ void __launch_bounds__(256) union_mask_kernel(FrameSource s, int N, i
   if (fl == 0 && p < npair) {
     uint8_t r = 0;
     for (int l = 0; l < kMaskLanes; ++l) r |= kk[l][tp];
-    mask[p] = r;
+    if (gridDim.y == 1 || r) mask[p] = r;
   }
+}
+
+__global__ void __launch_bounds__(256) zero_mask_kernel(uint8_t *mask, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) mask[i] = 0;
 }
 
 int launch_union_mask(const FrameSource &src, int N, int64_t f_lo, int64_t nfr, uint8_t *mask_dev,
@@ -102,8 +114,16 @@ int launch_union_mask(const FrameSource &src, int N, int64_t f_lo, int64_t nfr, 
     NISE_HIP_CHECK(hipGetLastError());
     return NISE_OK;
   }
-  dim3 grid((unsigned)((npair + kMaskPairs - 1) / kMaskPairs));
-  hipLaunchKernelGGL(union_mask_kernel, grid, dim3(256), 0, st, src, N, f_lo, nfr, mask_dev);
+  const int64_t gx = (npair + kMaskPairs - 1) / kMaskPairs, batch = kMaskLanes * kMaskInflight;
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>(kMaskGroups / gx, (nfr + batch - 1) / batch));
+  const int64_t per = ((nfr + want - 1) / want + batch - 1) / batch * batch;
+  const int64_t gy = std::max<int64_t>(1, (nfr + per - 1) / per);
+  if (gy > 1) {
+    hipLaunchKernelGGL(zero_mask_kernel, dim3((unsigned)((npair + 255) / 256)), dim3(256), 0, st, mask_dev, npair);
+    NISE_HIP_CHECK(hipGetLastError());
+  }
+  hipLaunchKernelGGL(union_mask_kernel, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, st, src, N, f_lo, nfr, per,
+                     mask_dev);
   NISE_HIP_CHECK(hipGetLastError());
   return NISE_OK;
 }
