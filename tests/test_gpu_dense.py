@@ -68,14 +68,45 @@ def test_trotter_propagators_against_conveyor(orc, N, T, ns, sr, ts, begin):
     """The Trotter scheme through per-frame propagators against the row
     conveyor and the oracle: both sides of every row class, odd N, Trotter
     substeps, samples that do not start at frame 0, windows with gaps, graph
-    replays.  1e-5 as for the conveyor (the propagators' own rounding is far
-    below over these windows)."""
+    replays.  1e-5 as for the conveyor: the distance between the two grows with
+    the sweeps (tmax times substeps), at most 7.1e-6 after 128 (test_longest_runs
+    has the largest)."""
     non, H, mu = lattice_case(N, T, ns, sr, seed=800 + N, ts=ts, begin=begin)
     print(f"[dense] Trotter N={N} T={T}", flush=True)
     d, r = both(non, H, mu)
     assert rel(d, r) < 1e-5
     o_re, o_im = orc.absorption(non, H, mu)
     assert rel(d, o_re + 1j * o_im) < 1e-5
+
+
+@pytest.mark.parametrize("N,T,ts", [(25, 256, 1), (25, 32, 8), (77, 256, 1), (77, 128, 2), (77, 64, 4)])
+def test_longest_runs(orc, N, T, ts):
+    """The most sweeps that go through propagators (256): within 1.5e-5 of the
+    reference's rounding, oracle and conveyor (twice the 7.1e-6 measured after
+    128 sweeps: each sweep's rounding is biased the same way), and nearer to
+    64 bits than it."""
+    non, H, mu = lattice_case(N, T, 8, 5, seed=840 + N + ts, ts=ts)
+    print(f"[dense] 256 sweeps: N={N} T={T} ts={ts}", flush=True)
+    d, r = both(non, H, mu)
+    assert not np.array_equal(d, r)
+    o_re, o_im = orc.absorption(non, H, mu)
+    assert rel(d, r) < 1.5e-5 and rel(d, o_re + 1j * o_im) < 1.5e-5
+    x_re, x_im = orc.absorption(non, H, mu, f64=True)
+    x = x_re + 1j * x_im
+    assert rel(d, x) < rel(r, x)
+
+
+@pytest.mark.parametrize("N,T,ts", [(25, 129, 2), (77, 128, 3), (77, 33, 8)])
+def test_runs_of_more_sweeps_keep_the_conveyor(N, T, ts):
+    """Substeps count: past 256 sweeps the default is the conveyor, bit for bit."""
+    non, H, mu = lattice_case(N, T, 8, 5, seed=850 + N, ts=ts)
+    print(f"[dense] {T * ts} sweeps: N={N} T={T} ts={ts}", flush=True)
+    p = abi.AbsPlan(non, H, H.shape[1], mu, mu.shape[1], H.shape[0])
+    default = p.execute()
+    p.set_rows(0)
+    rows = p.execute()
+    p.close()
+    assert np.array_equal(default[0], rows[0]) and np.array_equal(default[1], rows[1])
 
 
 def test_trotter_propagators_coupling_type_and_shifts():
