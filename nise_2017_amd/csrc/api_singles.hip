@@ -181,7 +181,7 @@ int build_slots(nise_abs_plan *P) {
 // Descriptor of the chain kernels.
 ChainArgs chain_args(nise_abs_plan *P) {
   ChainArgs a;
-  a.N = P->N, a.T = P->tmax, a.m = P->m, a.nvec = 3 * (P->end - P->begin), a.begin = P->begin, a.sample = P->sample;
+  a.R = P->chain, a.N = P->N, a.T = P->tmax, a.m = P->m, a.nvec = 3 * (P->end - P->begin), a.begin = P->begin, a.sample = P->sample;
   a.f_lo = P->f_lo, a.fac = trotter_factor(P->non.deltat, 1, P->m);
   a.rec = P->rec.as<float4>(), a.partial = P->partial.as<double2>();
   if (P->every) {
@@ -209,7 +209,7 @@ int run_conveyor(nise_abs_plan *P) {
     if (rc) return rc;
     return launch_dense(dense_class(P->N), P->dsys.as<DiaSys>(), P->dmap.as<int2>(), P->nwg, P->st, nullptr);
   }
-  if (P->chain) return launch_chain(chain_args(P), P->chain, P->st);
+  if (P->chain) return launch_chain(chain_args(P), P->st);
   if (P->rows)
     return launch_rows(P->row_sys.as<RowsArgs>(), P->row_wmap.as<int2>(), P->nwg, P->rows, P->row_pf, P->row_smem,
                        P->st);
@@ -681,7 +681,7 @@ extern "C" int nise_abs_plan_adjoint(nise_abs_plan *P, const float *g_re, const 
         (rc = P->part_c.alloc((size_t)std::max(nwg, 1) * 8)))
       return rc;
     r.part_delta = P->part_d.as<double>(), r.part_c = P->part_c.as<double>();
-    rc = launch_chain_adjoint(r, P->chain, P->grad.as<double>(), P->st);
+    rc = launch_chain_adjoint(r, P->grad.as<double>(), P->st);
   } else if (P->rows) {  // time-skewed row variant on the row conveyor's tables
     AdjRowsArgs r;
     r.N = N, r.T = T, r.m = P->m, r.nlayers = P->sch.nlayers(), r.every = P->every, r.nck = P->nck;

@@ -104,14 +104,13 @@ struct Sweep {
 
 constexpr int kAhead = 4;  // steps from a record's load to its use (L2 latency; 8 registers a step backward)
 
+// Forward of the vectors [group V, group V + V) of one system.
 template <int R>
-__global__ void __launch_bounds__(64) chain_kernel(ChainArgs A) {
+__device__ __forceinline__ void chain_run(const ChainArgs &A, int group, unsigned char *smem) {
   constexpr int V = 64 / R;
-  extern __shared__ __align__(16) unsigned char smem[];
-  const unsigned long long t_start = __builtin_amdgcn_s_memrealtime();
   const int N = A.N, T = A.T, m = A.m, P = chain_period(N, R), M = (T - 1) * m + 1;
   const int lane = threadIdx.x, vs = min(lane / R, V - 1), q = lane - vs * R;  // lanes past V R: q >= R, idle
-  const int v = blockIdx.x * V + vs, vv = min(v, A.nvec - 1), x = vv % 3;
+  const int v = group * V + vs, vv = min(v, A.nvec - 1), x = vv % 3;
   const bool has = q < R && v < A.nvec;
   const uint32_t row0 = (uint32_t)((int64_t)(A.begin + vv / 3) * A.sample - A.f_lo);
   float2 *ret = reinterpret_cast<float2 *>(smem) + vs * N;  // lane R - 1's sites for lane 0
@@ -182,9 +181,32 @@ __global__ void __launch_bounds__(64) chain_kernel(ChainArgs A) {
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  if (A.times && lane == 0) {
-    gst(A.times + 2 * blockIdx.x, t_start);
-    gst(A.times + 2 * blockIdx.x + 1, (unsigned long long)__builtin_amdgcn_s_memrealtime());
+}
+
+template <int R>
+__global__ void __launch_bounds__(64) chain_kernel(ChainArgs A) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  chain_run<R>(A, blockIdx.x, smem);
+}
+
+// The chains of a batch, each with its own R: workgroup = group wmap.y of
+// system wmap.x, with its start and end on the device clock.  One launch, because
+// one system's few waves leave the chip idle (48 chains of 64 sites, 100 samples of
+// 256 steps, whole call: one launch after the other 12.8 ms, the row conveyor 6.7,
+// this 2.5).
+__global__ void __launch_bounds__(64) chain_batch_kernel(const ChainArgs *sys, const int2 *wmap,
+                                                         unsigned long long *times) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const unsigned long long t_start = __builtin_amdgcn_s_memrealtime();
+  const int2 wm = wmap[blockIdx.x];
+  const ChainArgs A = sys[__builtin_amdgcn_readfirstlane(wm.x)];
+  const int group = __builtin_amdgcn_readfirstlane(wm.y);
+  if (A.R == 21) chain_run<21>(A, group, smem);
+  else if (A.R == 10) chain_run<10>(A, group, smem);
+  else chain_run<5>(A, group, smem);
+  if (threadIdx.x == 0) {
+    times[2 * blockIdx.x] = t_start;
+    times[2 * blockIdx.x + 1] = __builtin_amdgcn_s_memrealtime();
   }
 }
 
@@ -312,12 +334,13 @@ __global__ void __launch_bounds__(64) chain_adjoint_kernel(ChainArgs A) {
   if (lane == 0) gst(A.part_c + blockIdx.x, cg);
 }
 
-// LDS of a launch (the backward kernel's, which is the larger).
-size_t chain_smem(int N, int T, int R) { return (size_t)(64 / R) * N * 24 + (size_t)T * 8; }
+// LDS of a workgroup, forward and backward.
+static size_t chain_smem_fwd(int N, int R) { return (size_t)(64 / R) * N * 8; }
+static size_t chain_smem(int N, int T, int R) { return (size_t)(64 / R) * N * 24 + (size_t)T * 8; }
 
 // Fewer lanes per vector where a short chain would leave lanes idle (the
 // period is at least 2 R + 2 steps): the R with the fewest steps, times the
-// waves that share a SIMD.
+// waves that share a SIMD.  nvec: all vectors of the launch.
 int chain_rows(int N, int T, int m, int64_t nvec, int64_t nfr) {
   if (nfr * N >= (int64_t)1 << 30) return 0;  // 32-bit record indexes
   const int64_t M = (int64_t)(T - 1) * m + 1;
@@ -333,11 +356,10 @@ int chain_rows(int N, int T, int m, int64_t nvec, int64_t nfr) {
   return best;
 }
 
-static int launch_chain_fn(const void *fn, const ChainArgs &a, int R, hipStream_t st) {
-  const int nwg = chain_groups(a.nvec, R);
+static int launch_chain_fn(const void *fn, const ChainArgs &a, size_t smem, hipStream_t st) {
+  const int nwg = chain_groups(a.nvec, a.R);
   if (nwg <= 0) return NISE_OK;
-  const size_t smem = chain_smem(a.N, a.T, R);
-  if (!fn || smem > 160 * 1024) return set_error("chain: N=%d with %d lanes per vector", a.N, R), NISE_ERR_ARG;
+  if (!fn || smem > 160 * 1024) return set_error("chain: N=%d with %d lanes per vector", a.N, a.R), NISE_ERR_ARG;
   NISE_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
   ChainArgs args = a;
   void *kargs[] = {&args};
@@ -345,17 +367,49 @@ static int launch_chain_fn(const void *fn, const ChainArgs &a, int R, hipStream_
   return NISE_OK;
 }
 
-int launch_chain(const ChainArgs &a, int R, hipStream_t st) {
-  return launch_chain_fn(R == 21 ? (const void *)chain_kernel<21> : R == 10 ? (const void *)chain_kernel<10>
-                         : R == 5 ? (const void *)chain_kernel<5> : nullptr, a, R, st);
+int launch_chain(const ChainArgs &a, hipStream_t st) {
+  return launch_chain_fn(a.R == 21 ? (const void *)chain_kernel<21> : a.R == 10 ? (const void *)chain_kernel<10>
+                         : a.R == 5 ? (const void *)chain_kernel<5> : nullptr, a, chain_smem_fwd(a.N, a.R), st);
 }
 
-int launch_chain_adjoint(const ChainArgs &a, int R, double *out, hipStream_t st) {
-  const int rc = launch_chain_fn(R == 21 ? (const void *)chain_adjoint_kernel<21>
-                                 : R == 10 ? (const void *)chain_adjoint_kernel<10>
-                                 : R == 5 ? (const void *)chain_adjoint_kernel<5> : nullptr, a, R, st);
+int launch_chain_adjoint(const ChainArgs &a, double *out, hipStream_t st) {
+  const int rc = launch_chain_fn(a.R == 21 ? (const void *)chain_adjoint_kernel<21>
+                                 : a.R == 10 ? (const void *)chain_adjoint_kernel<10>
+                                 : a.R == 5 ? (const void *)chain_adjoint_kernel<5> : nullptr, a,
+                                 chain_smem(a.N, a.T, a.R), st);
   if (rc) return rc;
-  return launch_adjoint_reduce(a.part_delta, a.part_c, chain_groups(a.nvec, R), a.N, out, st);
+  return launch_adjoint_reduce(a.part_delta, a.part_c, chain_groups(a.nvec, a.R), a.N, out, st);
+}
+
+// Workgroups of a batch's chains, the longest first.
+void chain_batch_map(const std::vector<ChainArgs> &sys, std::vector<int2> &wmap) {
+  std::vector<int> order(sys.size());
+  for (size_t i = 0; i < sys.size(); ++i) order[i] = (int)i;
+  auto steps = [&](int i) {
+    const ChainArgs &a = sys[i];
+    return ((int64_t)(a.T - 1) * a.m / a.R + 1) * chain_period(a.N, a.R);
+  };
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return steps(x) > steps(y); });
+  wmap.clear();
+  for (int i : order)
+    for (int g = 0; g < chain_groups(sys[i].nvec, sys[i].R); ++g) wmap.push_back(make_int2(i, g));
+}
+
+// sys_h / nwg: host descriptors and chain_batch_map's size; sys / wmap: device copies.
+int launch_chain_batch(const std::vector<ChainArgs> &sys_h, const ChainArgs *sys, const int2 *wmap, int nwg,
+                       hipStream_t st, unsigned long long *times) {
+  if (nwg <= 0) return NISE_OK;
+  size_t smem = 0;
+  for (const ChainArgs &a : sys_h) {
+    smem = std::max(smem, chain_smem_fwd(a.N, a.R));
+    if (smem > 160 * 1024 || !(a.R == 21 || a.R == 10 || a.R == 5))
+      return set_error("chain: N=%d with %d lanes per vector", a.N, a.R), NISE_ERR_ARG;
+  }
+  const void *fn = (const void *)chain_batch_kernel;
+  NISE_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+  void *kargs[] = {&sys, &wmap, &times};
+  NISE_HIP_CHECK(hipLaunchKernel(fn, dim3((unsigned)nwg), dim3(64), kargs, smem, st));
+  return NISE_OK;
 }
 
 bool chain_mask(int N, const std::vector<uint8_t> &mask) {

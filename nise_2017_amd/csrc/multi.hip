@@ -2,11 +2,13 @@
 //
 // Systems with propagation 1 (Trotter coupling scheme) run on the row
 // conveyor in one launch: every workgroup reads its own system descriptor,
-// so waves of different N share the launch.  Systems with propagation 0
-// (exact exponential, src/propagate.c:60-125) and N <= 64 run in a second
-// launch: per frame U = exp(-i H f) is formed once (FP64 Taylor series with
-// scaling and squaring, rounded to FP32) and dense_vectors_kernel applies it,
-// one wave per vector.
+// so waves of different N share the launch.  Nearest-neighbour chains share one
+// launch of their own (chain.hip) on a second stream beside it, and systems
+// that pay for it go through per-frame propagators (dense.hip).  Systems with
+// propagation 0 (exact exponential, src/propagate.c:60-125) and N <= 64 run on
+// the second stream: per frame U = exp(-i H f) is formed once (FP64 Taylor
+// series with scaling and squaring, rounded to FP32), and the kernels of
+// dense.hip apply it, one launch per size class.
 //
 // Each workgroup records its start and end on the device wall clock; a
 // system's completion latency is the end of its last workgroup measured from
@@ -502,7 +504,7 @@ struct SysState {
 // call).  Every call ends with both streams synchronised.
 struct MultiCache {
   std::vector<std::unique_ptr<SysState>> sys;
-  DevBuf mk, rsys, rwm, dsys, dwm, times, out, ejobs;
+  DevBuf mk, rsys, rwm, dsys, dwm, csys, cwm, times, out, ejobs;
   std::vector<ExpmJob> ejobs_h;  // the job table of the last upload
   // the row count nise_absorption_multi_tune chose for a batch of this shape
   std::vector<int64_t> tune_sig;
@@ -734,12 +736,15 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
   //    independent; one after the other they took 40 ms for 16 systems up to
   //    N = 384 against a GPU time of 10).
   std::vector<SchedJob> jobs4;
+  int64_t chain_vec = 0;  // vectors of the chains' launch
+  for (int k = 0; k < nsys && own; ++k)
+    if (!S[k]->dia && chain_mask(S[k]->N, S[k]->mask)) chain_vec += S[k]->nvec;
   for (int k = 0; k < nsys; ++k) {
     SysState &s = *S[k];
     const t_non *non = systems[k].non;
     if (s.dia) continue;
     s.Rk = R > 0 ? R : rows_for(s.N, s.sch_asap.Kreal, s.sch_asap.nlayers(), cap);
-    s.chain = own && chain_mask(s.N, s.mask) ? chain_rows(s.N, s.T, non->ts, s.nvec, s.f_hi - s.f_lo) : 0;
+    s.chain = own && chain_mask(s.N, s.mask) ? chain_rows(s.N, s.T, non->ts, chain_vec, s.f_hi - s.f_lo) : 0;
     if (s.chain) continue;
     s.dense = own && dense_pays(s.N, s.T, s.nvec / 3, s.f_hi - s.f_lo, s.sch_asap.Kreal, s.sch_asap.nlayers(), non->ts);
     if (s.rows_N != s.N || s.rows_R != s.Rk || s.rows_packed != s.dense || s.rows_mask != s.mask) {
@@ -769,7 +774,7 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
           (rc = launch_chain_tables(s.src, N, s.f_lo, nfr, fac, s.mu_dev, s.mu_stride, s.rec.as<float4>(), st)))
         return rc;
       ChainArgs c;
-      c.N = N, c.T = s.T, c.m = non->ts, c.nvec = s.nvec, c.begin = non->begin, c.sample = non->sample;
+      c.R = s.chain, c.N = N, c.T = s.T, c.m = non->ts, c.nvec = s.nvec, c.begin = non->begin, c.sample = non->sample;
       c.f_lo = s.f_lo, c.fac = fac, c.rec = s.rec.as<float4>(), c.partial = s.partial.as<double2>();
       chains.push_back(c);
       chain_of.push_back(k);
@@ -827,14 +832,17 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
     if (!S[dia_of[i]]->dense && !dia_window_fits(dias[i].N, dias[i].tmax, dias[i].nvec))
       return set_error("multi: DIA window of %d steps is too long for N=%d", dias[i].tmax, dias[i].N), NISE_ERR_ARG;
   }
+  std::vector<int2> cmap;
+  chain_batch_map(chains, cmap);
   DevBuf &rsys = cache.rsys, &rwm = cache.rwm, &dsys = cache.dsys, &dwm = cache.dwm, &times = cache.times;
-  size_t nt = rmap.size() + dmap.size();
-  std::vector<size_t> cend;  // ends of the chains' times
-  for (size_t i = 0; i < chains.size(); ++i) cend.push_back(nt += chain_groups(chains[i].nvec, S[chain_of[i]]->chain));
+  DevBuf &csys = cache.csys, &cwm = cache.cwm;
+  const size_t nt = rmap.size() + dmap.size() + cmap.size();
   if ((rc = up(rsys, rows.data(), rows.size() * sizeof(RowsArgs))) ||
       (rc = up(rwm, rmap.data(), rmap.size() * sizeof(int2))) ||
       (rc = up(dsys, dias.data(), dias.size() * sizeof(DiaSys))) ||
-      (rc = up(dwm, dmap.data(), dmap.size() * sizeof(int2))) || (rc = times.alloc(nt * 16 + 16)))
+      (rc = up(dwm, dmap.data(), dmap.size() * sizeof(int2))) ||
+      (rc = up(csys, chains.data(), chains.size() * sizeof(ChainArgs))) ||
+      (rc = up(cwm, cmap.data(), cmap.size() * sizeof(int2))) || (rc = times.alloc(nt * 16 + 16)))
     return rc;
   unsigned long long *tm = times.as<unsigned long long>();
   // The row conveyor starts after the matrix exponentials: its long-lived
@@ -848,10 +856,16 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
     (void)hipEventDestroy(ev);
     NISE_HIP_CHECK(e2);
   }
-  for (size_t i = 0; i < chains.size(); ++i) {
-    const int Rc = S[chain_of[i]]->chain;
-    chains[i].times = tm + 2 * (cend[i] - chain_groups(chains[i].nvec, Rc));
-    if ((rc = launch_chain(chains[i], Rc, st))) return rc;
+  // the chains beside the row conveyor, after their tables
+  if (!cmap.empty()) {
+    hipEvent_t ev;
+    NISE_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    hipError_t e1 = hipEventRecord(ev, st), e2 = e1 == hipSuccess ? hipStreamWaitEvent(sd, ev, 0) : e1;
+    (void)hipEventDestroy(ev);
+    NISE_HIP_CHECK(e2);
+    if ((rc = launch_chain_batch(chains, csys.as<ChainArgs>(), cwm.as<int2>(), (int)cmap.size(), sd,
+                                 tm + 2 * (rmap.size() + dmap.size()))))
+      return rc;
   }
   if (!rmap.empty() && (rc = launch_rows(rsys.as<RowsArgs>(), rwm.as<int2>(), (int)rmap.size(), R, rpf, rsmem, st, tm)))
     return rc;
@@ -864,7 +878,7 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
       if ((rc = launch_dense(cls, dsp, dmp + d0, (int)(dend[tr][cls] - d0), tr ? st : sd, td + 2 * d0))) return rc;
       d0 = dend[tr][cls];
     }
-  // the reductions and copies below wait for the DIA stream
+  // the reductions and copies below wait for the second stream
   {
     hipEvent_t ev;
     NISE_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -911,8 +925,10 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
       const int k = dia_of[dmap[i].x];
       done[k] = std::max(done[k], ht[2 * (rmap.size() + i) + 1]);
     }
-    for (size_t i = 0, w = rmap.size() + dmap.size(); i < chains.size(); ++i)
-      for (; w < cend[i]; ++w) done[chain_of[i]] = std::max(done[chain_of[i]], ht[2 * w + 1]);
+    for (size_t i = 0; i < cmap.size(); ++i) {
+      const int k = chain_of[cmap[i].x];
+      done[k] = std::max(done[k], ht[2 * (rmap.size() + dmap.size() + i) + 1]);
+    }
     for (int k = 0; k < nsys; ++k) done_ms[k] = khz > 0 ? (double)(done[k] - t0) / khz : -1.0;
   }
   return NISE_OK;

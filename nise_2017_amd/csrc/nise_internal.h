@@ -569,10 +569,10 @@ struct AdjArgs {
 };
 int launch_adjoint(const AdjArgs &a, int vp, double *out, hipStream_t st);
 
-// Row variant of the adjoint (the row conveyor's schedule and tables).
 // Nearest-neighbour chains (chain.hip): forward needs rec and partial,
 // backward rec, ck, g and the gradient partials (one row per workgroup).
 struct ChainArgs {
+  int R = 0;  // lanes per vector (chain_rows)
   int N = 0, T = 0, m = 1, nvec = 0, begin = 0, sample = 1, every = 1, nck = 0;
   int64_t f_lo = 0;
   float fac = 0.f;
@@ -580,7 +580,6 @@ struct ChainArgs {
   double2 *partial = nullptr;   // [vectors][T]
   float2 *hist = nullptr;       // checkpoints, as RowsArgs
   int hist_every = 1;
-  unsigned long long *times = nullptr;  // forward: device clock at start and end, per workgroup
   const float2 *ck = nullptr, *g = nullptr;
   double *part_delta = nullptr, *part_c = nullptr;
 };
@@ -591,10 +590,14 @@ int chain_rows(int N, int T, int m, int64_t nvec, int64_t nfr);
 inline int chain_groups(int nvec, int R) { return (nvec + 64 / R - 1) / (64 / R); }
 int launch_chain_tables(const FrameSource &src, int N, int64_t f_lo, int64_t nfr, float fac, const float *mu_rec,
                         int64_t mu_stride, float4 *rec, hipStream_t st);
-int launch_chain(const ChainArgs &a, int R, hipStream_t st);
-int launch_chain_adjoint(const ChainArgs &a, int R, double *out, hipStream_t st);
-size_t adjoint_rows_smem(int N, int R);
+int launch_chain(const ChainArgs &a, hipStream_t st);
+int launch_chain_adjoint(const ChainArgs &a, double *out, hipStream_t st);
+void chain_batch_map(const std::vector<ChainArgs> &sys, std::vector<int2> &wmap);
+int launch_chain_batch(const std::vector<ChainArgs> &sys_h, const ChainArgs *sys, const int2 *wmap, int nwg,
+                       hipStream_t st, unsigned long long *times);
 int launch_adjoint_reduce(const double *pd, const double *pc, int nwg, int N, double *out, hipStream_t st);
+size_t adjoint_rows_smem(int N, int R);
+// Row variant of the adjoint (the row conveyor's schedule and tables).
 struct AdjRowsArgs {
   int N = 0, T = 0, m = 1, nlayers = 0, every = 1, nck = 0, nvec = 0, begin = 0, sample = 1;
   int64_t K = 0, f_lo = 0;

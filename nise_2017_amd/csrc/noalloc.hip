@@ -176,10 +176,10 @@ int run_chain(unsigned char *base, size_t used, const FrameSource &src, const Ro
   for (int s0 = 0; s0 < ns; s0 += per) {  // one stream: a window's tables wait for the previous window
     const int n = std::min(per, ns - s0);
     ChainArgs c;
-    c.N = N, c.T = T, c.m = r.m, c.nvec = 3 * n, c.begin = r.begin + s0, c.sample = r.sample, c.fac = fac;
+    c.R = R, c.N = N, c.T = T, c.m = r.m, c.nvec = 3 * n, c.begin = r.begin + s0, c.sample = r.sample, c.fac = fac;
     c.f_lo = (int64_t)c.begin * r.sample, c.rec = rec, c.partial = partial + (size_t)3 * s0 * T;
     if ((rc = launch_chain_tables(src, N, c.f_lo, frames(n), fac, r.mu_rec, r.mu_stride, rec, st)) ||
-        (rc = launch_chain(c, R, st)))
+        (rc = launch_chain(c, st)))
       return rc;
   }
   if ((rc = launch_reduce_partials(partial, 3 * ns, T, out, out + T, st))) return rc;

@@ -88,3 +88,35 @@ def test_chain_batch_and_noalloc_match_plan(N, T, ns, sr):
     for k in (0, 2):
         assert np.array_equal(re, out[k][0]) and np.array_equal(im, out[k][1])
     assert np.all(done > 0)
+
+
+def test_batch_runs_its_chains_together():
+    """Equal chains of a batch share one launch: they end at about the same
+    time.  One after the other, the last of 24 would end 24 times as late as the
+    first."""
+    case = chain_case(64, 200, 60, 10)
+    system = (*case, None)
+    print("[chain] 24 equal chains", flush=True)
+    abi.absorption_multi([system] * 24)
+    out, done = abi.absorption_multi([system] * 24)
+    assert max(done) < 4 * min(done), done
+    for re, im in out:
+        assert np.array_equal(re, out[0][0]) and np.array_equal(im, out[0][1])
+
+
+def test_batch_of_uneven_chains_matches_plans():
+    """Chains of every lanes-per-vector count, with substeps, beside a lattice
+    and an exact-exponential system: bit for bit their plans' results."""
+    from test_gpu_multi import system
+    cases = [chain_case(N, T, ns, sr, ts, begin)
+             for N, T, ns, sr, ts, begin in [(3, 17, 4, 2, 1, 0), (9, 40, 30, 3, 2, 1), (21, 33, 5, 7, 1, 0),
+                                             (70, 50, 12, 4, 3, 2), (130, 24, 3, 30, 1, 0), (2, 1, 1, 1, 1, 0)]]
+    batch = [(*c, None) for c in cases] + [system(23, 1, 3), system(20, 0, 4)]
+    print("[chain] uneven batch", flush=True)
+    out, done = abi.absorption_multi(batch)
+    for (non, H, mu), (re, im) in zip(cases, out):
+        p = abi.AbsPlan(non, H, H.shape[1], mu, mu.shape[1], H.shape[0])
+        r, i = p.execute()
+        p.close()
+        assert np.array_equal(re, r) and np.array_equal(im, i), non.singles
+    assert np.all(done > 0)
