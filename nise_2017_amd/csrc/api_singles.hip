@@ -394,7 +394,8 @@ static int plan_create(nise_abs_plan **out, const t_non *non, const float *H_rec
     P->rows = rows_for(N, P->sch_asap.Kreal, P->sch_asap.nlayers());
     P->mask = mask;
     if (chain_mask(N, mask)) P->chain = chain_rows(N, P->tmax, P->m, 3 * (int64_t)(P->end - P->begin), nfr);
-    P->dense = !P->chain && dense_pays(N, P->tmax, P->end - P->begin, nfr, P->sch_asap.Kreal, P->sch_asap.nlayers(), P->m);
+    P->dense = !P->chain &&
+               dense_pays({N, P->tmax, P->m, P->end - P->begin, nfr, P->sch_asap.Kreal, P->sch_asap.nlayers()});
     if (P->chain && (rc = P->rec.alloc((size_t)nfr * N * 2 * sizeof(float4)))) return rc;
     P->packed = P->dense && one_run;  // a run made once does not pay for the list schedule
     if (P->packed) pack_schedule_rows(P->sch_asap, P->rows, P->sch_rows);

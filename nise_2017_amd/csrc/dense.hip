@@ -267,31 +267,86 @@ int launch_dense(int cls, const DiaSys *sys, const int2 *wmap, int nwg, hipStrea
   return NISE_OK;
 }
 
-// Whether a Trotter run goes through per-frame propagators instead of the row
-// conveyor: rotation sweeps on the N columns of every frame (independent of
-// each other) and one product per vector step, against rotation sweeps on
-// every vector step.  A conveyor wave walks tmax frames of nlayers dependent
-// LDS round trips, so runs with few waves are far from its throughput.  The
-// cycle counts are fits: measured (conveyor and this, ms) N = 25 lattice,
-// 1,500 samples 1.56 and 0.59; N = 77 lattice, 333 samples 2.60 and 1.05;
-// N = 64 lattice, 800 samples 2.43 and 1.24, 1,500 samples 2.72 (conveyor;
-// 3.4); N = 121 lattice, 800 samples 4.50 and 4.41.  Nearest-neighbour chains
-// do not come here (chain.hip).
-// Kreal, nasap: rotations and layers of the layered schedule; m: Trotter
-// substeps; F: frames; S: samples.
-bool dense_pays(int N, int T, int64_t S, int64_t F, int Kreal, int nasap, int m) {
-  if ((int64_t)T * m > kDenseMaxSweeps) return false;
-  if (N > kDenseMaxN || F >= (1 << 30) || (double)dense_u_bytes(N, F) > kDenseMaxBytes) return false;
-  const int R = rows_for(N, Kreal, nasap);
-  const double G = 64.0 / R, sweep = std::max({(double)nasap, (double)Kreal / R, 8.0}) * m;
-  // conveyor: a wave's frame is a chain of LDS round trips and its share of
-  // the sites; all waves together are bound by LDS instructions
-  const double rows = T * (176.0 * sweep + 180.0 * N / R + 300.0) * (1.0 + 3.0 * S / G / 3400.0);
-  const double build = F * std::ceil((N + (N & 1)) / G) / 256.0 * (21.0 * sweep + 150.0) + 20000.0;
-  const double apply = dense_class(N) == 0
-                           ? T * std::max(500.0 + 24.0 * N, 3.0 * S / 1024.0 * (200.0 + 12.0 * N))
-                           : T * std::max(1.0, S / 256.0) * (1000.0 + 40.0 * N);
-  return build + apply < 0.85 * rows;
+// Costs in cycles of a Trotter run on the row conveyor and through per-frame
+// propagators.  A conveyor wave walks tmax frames of nlayers dependent LDS
+// round trips, each with its share of the sites, and all waves together are
+// bound by LDS instructions; propagators are rotation sweeps on the N columns of
+// every frame (independent of each other, so they fill the chip) and one product
+// per vector step, a chain of tmax of them or bound by all vectors' products.
+// The constants are fits.
+struct RunCost {
+  double rows, load;       // a conveyor wave's chain; the waves, in chips full
+  double build;            // U of every frame
+  double chain, work;      // the products: one vector's chain, all vectors' work
+};
+static RunCost run_cost(const TrotterRun &r) {
+  const int R = rows_for(r.N, r.Kreal, r.nasap);
+  const double N = r.N, T = r.T, S = (double)r.S, G = 64.0 / R;
+  const double sweep = std::max({(double)r.nasap, (double)r.Kreal / R, 8.0}) * r.m;
+  RunCost c;
+  c.rows = T * (176.0 * sweep + 180.0 * N / R + 300.0), c.load = 3.0 * S / G / 3400.0;
+  c.build = (double)r.F * std::ceil((N + (r.N & 1)) / G) / 256.0 * (21.0 * sweep + 150.0);
+  if (dense_class(r.N) == 0) c.chain = T * (500.0 + 24.0 * N), c.work = T * 3.0 * S / 1024.0 * (200.0 + 12.0 * N);
+  else c.chain = T * (1000.0 + 40.0 * N), c.work = S / 256.0 * c.chain;
+  return c;
+}
+constexpr double kLaunches = 20000.0;  // of the propagators
+
+static bool dense_fits(const TrotterRun &r) {
+  return (int64_t)r.T * r.m <= kDenseMaxSweeps && r.N <= kDenseMaxN && r.F < (1 << 30) &&
+         (double)dense_u_bytes(r.N, r.F) <= kDenseMaxBytes;
+}
+
+// A run by itself: propagators where they take less than 0.85 of the conveyor's
+// time (kernels, ms, conveyor and propagators: N = 25 lattice, 1,500 samples 1.56
+// and 0.59; N = 77, 333 samples 2.60 and 1.05; N = 64, 800 samples 2.43 and 1.24,
+// 1,500 samples 2.72 and 3.4; N = 121, 800 samples 4.50 and 4.41).
+bool dense_pays(const TrotterRun &r) {
+  if (!dense_fits(r)) return false;
+  const RunCost c = run_cost(r);
+  return kLaunches + c.build + std::max(c.chain, c.work) < 0.85 * c.rows * (1.0 + c.load);
+}
+
+// Which Trotter runs of a batch go through propagators: those that pay by
+// themselves, U of all of them within kDenseBatchBytes.  But runs that share the
+// conveyor's launch fill the chip together, which gains little per run beside
+// many others: only the longest of them, or none, where that takes less than
+// three quarters of the time (propagators are the nearer to 64 bits, and beside a
+// conveyor that leaves the chip idle they run on a second stream: half of the
+// shorter side is counted; above 96 sites one workgroup fills a CU, and the
+// products take 1.3 of run_cost's).  Whole calls, ms, all on the conveyor and all
+// through propagators, lattices with 100 samples: N = 100, 256 steps, 1 of them
+// 4.5 and 1.0, 4 4.7 and 2.7, 16 6.2 and 9.2, 48 9.4 and 26; N = 64, 200 steps, 8
+// of them 3.0 and 1.7, 48 5.0 and 9.8; N = 25, 256 steps, 48 of them 4.6 and 3.9.
+void dense_choice(const std::vector<TrotterRun> &runs, std::vector<char> &dense) {
+  const size_t n = runs.size();
+  dense.assign(n, 0);
+  std::vector<RunCost> c(n);
+  std::vector<size_t> order(n), pay;
+  double load = 0.0, bytes = 0.0, stay = 0.0;  // stay: the longest chain that keeps the conveyor
+  for (size_t i = 0; i < n; ++i) c[i] = run_cost(runs[i]), order[i] = i, load += c[i].load;
+  std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return c[x].rows > c[y].rows; });
+  for (size_t i : order) {
+    const double u = (double)dense_u_bytes(runs[i].N, runs[i].F);
+    if (dense_pays(runs[i]) && bytes + u <= kDenseBatchBytes) pay.push_back(i), bytes += u;
+    else stay = std::max(stay, c[i].rows);
+  }
+  double build = 0.0, chain[4] = {}, work[4] = {}, best = 0.0, total = 0.0;
+  size_t keep = 0;
+  for (size_t j = 0; j <= pay.size(); ++j) {  // the first j through propagators
+    const double rows = std::max(stay, j < pay.size() ? c[pay[j]].rows : 0.0) * (1.0 + load);
+    double props = build;
+    for (int q = 0; q < 4; ++q) props += std::max(chain[q], work[q]);
+    total = std::max(rows, props) + 0.5 * std::min(rows, props);
+    if (j == 0 || total < best) best = total, keep = j;
+    if (j == pay.size()) break;
+    const RunCost &x = c[pay[j]];
+    const int k = dense_class(runs[pay[j]].N);
+    load -= x.load, build += x.build + (j ? 0.0 : kLaunches);
+    chain[k] = std::max(chain[k], x.chain), work[k] += x.work * (k == 3 ? 1.3 : 1.0);
+  }
+  if (best >= 0.75 * total) keep = pay.size();
+  for (size_t j = 0; j < keep; ++j) dense[pay[j]] = 1;
 }
 
 }  // namespace nise

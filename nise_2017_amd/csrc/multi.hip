@@ -735,18 +735,27 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
   //    are built first, on up to kSchedThreads host threads (they are
   //    independent; one after the other they took 40 ms for 16 systems up to
   //    N = 384 against a GPU time of 10).
-  std::vector<SchedJob> jobs4;
   int64_t chain_vec = 0;  // vectors of the chains' launch
   for (int k = 0; k < nsys && own; ++k)
     if (!S[k]->dia && chain_mask(S[k]->N, S[k]->mask)) chain_vec += S[k]->nvec;
+  std::vector<TrotterRun> runs;
+  std::vector<SysState *> run_of;
   for (int k = 0; k < nsys; ++k) {
     SysState &s = *S[k];
-    const t_non *non = systems[k].non;
+    const int64_t nfr = s.f_hi - s.f_lo;
     if (s.dia) continue;
     s.Rk = R > 0 ? R : rows_for(s.N, s.sch_asap.Kreal, s.sch_asap.nlayers(), cap);
-    s.chain = own && chain_mask(s.N, s.mask) ? chain_rows(s.N, s.T, non->ts, chain_vec, s.f_hi - s.f_lo) : 0;
+    s.chain = own && chain_mask(s.N, s.mask) ? chain_rows(s.N, s.T, systems[k].non->ts, chain_vec, nfr) : 0;
     if (s.chain) continue;
-    s.dense = own && dense_pays(s.N, s.T, s.nvec / 3, s.f_hi - s.f_lo, s.sch_asap.Kreal, s.sch_asap.nlayers(), non->ts);
+    runs.push_back({s.N, s.T, systems[k].non->ts, s.nvec / 3, nfr, s.sch_asap.Kreal, s.sch_asap.nlayers()});
+    run_of.push_back(&s);
+  }
+  std::vector<char> dense;
+  if (own) dense_choice(runs, dense);
+  for (size_t i = 0; i < dense.size(); ++i) run_of[i]->dense = dense[i];
+  std::vector<SchedJob> jobs4;
+  for (SysState *sp : run_of) {
+    SysState &s = *sp;
     if (s.rows_N != s.N || s.rows_R != s.Rk || s.rows_packed != s.dense || s.rows_mask != s.mask) {
       s.rows_N = 0;  // until the tables below are on the device
       jobs4.emplace_back();
@@ -804,8 +813,8 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
       rows.push_back(r);
       rows_of.push_back(k);
   }
-  // 5. the two launches (row conveyor for all Trotter systems, dense vectors
-  //    for all DIA systems), timed on the device clock
+  // 5. the launches (row conveyor, chains, dense vectors), timed on the device
+  //    clock
   std::vector<int2> rmap, dmap;
   size_t rsmem = 0;
   bool rpf = false;
@@ -816,8 +825,8 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
     const RowsArgs &a = rows[x.x], &b = rows[y.x];
     return (int64_t)a.nlayers * a.tmax * a.m > (int64_t)b.nlayers * b.tmax * b.m;
   });
-  // dmap: samples of the DIA systems (second stream), then of the Trotter
-  // systems' propagators (first stream), each by kernel class
+  // dmap: samples of the DIA systems, then of the Trotter systems'
+  // propagators, each by kernel class
   size_t dend[2][4];
   for (int tr = 0; tr < 2; ++tr)
     for (int cls = 0; cls < 4; ++cls) {
@@ -856,17 +865,20 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
     (void)hipEventDestroy(ev);
     NISE_HIP_CHECK(e2);
   }
-  // the chains beside the row conveyor, after their tables
-  if (!cmap.empty()) {
+  // beside the row conveyor on the second stream, after their tables: the
+  // chains, and the Trotter systems' propagators (without a conveyor these
+  // stay on the first stream, beside the DIA systems)
+  const bool shared = !rmap.empty() && dend[1][3] > dend[0][3];
+  if (!cmap.empty() || shared) {
     hipEvent_t ev;
     NISE_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     hipError_t e1 = hipEventRecord(ev, st), e2 = e1 == hipSuccess ? hipStreamWaitEvent(sd, ev, 0) : e1;
     (void)hipEventDestroy(ev);
     NISE_HIP_CHECK(e2);
-    if ((rc = launch_chain_batch(chains, csys.as<ChainArgs>(), cwm.as<int2>(), (int)cmap.size(), sd,
-                                 tm + 2 * (rmap.size() + dmap.size()))))
-      return rc;
   }
+  if ((rc = launch_chain_batch(chains, csys.as<ChainArgs>(), cwm.as<int2>(), (int)cmap.size(), sd,
+                               tm + 2 * (rmap.size() + dmap.size()))))
+    return rc;
   if (!rmap.empty() && (rc = launch_rows(rsys.as<RowsArgs>(), rwm.as<int2>(), (int)rmap.size(), R, rpf, rsmem, st, tm)))
     return rc;
   const DiaSys *dsp = dsys.as<DiaSys>();
@@ -875,7 +887,7 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
   size_t d0 = 0;
   for (int tr = 0; tr < 2; ++tr)
     for (int cls = 0; cls < 4; ++cls) {
-      if ((rc = launch_dense(cls, dsp, dmp + d0, (int)(dend[tr][cls] - d0), tr ? st : sd, td + 2 * d0))) return rc;
+      if ((rc = launch_dense(cls, dsp, dmp + d0, (int)(dend[tr][cls] - d0), tr && !shared ? st : sd, td + 2 * d0))) return rc;
       d0 = dend[tr][cls];
     }
   // the reductions and copies below wait for the second stream

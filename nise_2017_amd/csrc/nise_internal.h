@@ -476,9 +476,18 @@ struct DiaSys {
 // to 2.7e-5 off 64 bits at 256 and the propagators half of that.  The limit keeps
 // the distance within 1.5e-5; longer runs keep the conveyor.
 constexpr int kDenseMaxN = 128, kDenseMaxSweeps = 256;
-constexpr double kDenseMaxBytes = 1 << 30;  // of U
+constexpr double kDenseMaxBytes = 1 << 30, kDenseBatchBytes = 4.0 * (1 << 30);  // of U: one run, a batch
 constexpr size_t kScratchBytes = (size_t)32 << 20;  // noalloc.hip's array, per GPU
-bool dense_pays(int N, int T, int64_t S, int64_t F, int Kreal, int nasap, int m);
+// A Trotter run for the choice between the conveyor and propagators: S samples
+// over F frames; Kreal, nasap: rotations and layers of the layered schedule; m:
+// substeps.  Nearest-neighbour chains do not come here (chain.hip).
+struct TrotterRun {
+  int N = 0, T = 0, m = 1;
+  int64_t S = 0, F = 0;
+  int Kreal = 0, nasap = 0;
+};
+bool dense_pays(const TrotterRun &run);
+void dense_choice(const std::vector<TrotterRun> &runs, std::vector<char> &dense);
 inline size_t dense_u_bytes(int N, int64_t F) { return (size_t)F * 2 * ((N + 1) / 2) * N * 8; }
 // Kernel class of a system (dense.hip): 0 one wave per vector, 1 .. 3 one
 // workgroup per sample with 2 .. 4 rows per lane.

@@ -295,7 +295,7 @@ extern "C" int nise_absorption_batched_noalloc(const t_non *non, const float *H_
     bool ran = false;
     if ((rc = run_chain(ds->ptr, ar0, src, r, Rc, end - begin, trotter_factor(non->deltat, 1, m), re_S, im_S, ran)) || ran)
       return rc;
-  } else if (dense_pays(N, T, end - begin, nfr, asap.Kreal, asap.nlayers(), m))
+  } else if (dense_pays({N, T, m, end - begin, nfr, asap.Kreal, asap.nlayers()}))
     return run_dense(ds->ptr, ar0, src, r, asap, R, end - begin, trotter_factor(non->deltat, 1, m), re_S, im_S);
   if (!tab.empty()) NISE_HIP_CHECK(hipMemcpy(steps, tab.data(), tab.size() * sizeof(uint2), hipMemcpyHostToDevice));
   if (!ab.empty()) NISE_HIP_CHECK(hipMemcpy(abd, ab.data(), ab.size() * 4, hipMemcpyHostToDevice));

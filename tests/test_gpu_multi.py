@@ -117,3 +117,43 @@ def test_calls_of_changing_shape_reuse_buffers(orc):
     again, _ = abi.absorption_multi(a)
     for (r0, i0), (r1, i1) in zip(out_a, again):
         assert np.array_equal(r0, r1) and np.array_equal(i0, i1)
+
+
+def test_batch_choice_counts_the_whole_batch():
+    """A lattice that alone goes through per-frame propagators keeps the row
+    conveyor in a batch whose systems fill the chip together (the two differ by
+    the reference's rounding, 1e-7 to 1e-5 here; within the conveyor the results
+    agree to the rounding of the sums)."""
+    from test_gpu_dense import lattice_case
+    non, H, mu = lattice_case(100, 60, 60, 4, seed=61)
+    p = abi.AbsPlan(non, H, H.shape[1], mu, mu.shape[1], H.shape[0])
+    dense = p.execute()
+    p.set_rows(0)
+    rows = p.execute()
+    p.close()
+    d, r = dense[0] + 1j * dense[1], rows[0] + 1j * rows[1]
+    assert rel(d, r) > 3e-7
+    for n in (1, 64):
+        say(f"{n} lattices of 100 sites")
+        out, _ = abi.absorption_multi([(non, H, mu, None)] * n)
+        for re, im in out:
+            assert rel(re + 1j * im, d if n == 1 else r) < 1e-7
+
+
+def test_batch_with_every_kernel(orc):
+    """Conveyor, propagators, a chain and an exact-exponential system in one
+    call, on two streams: the lattice as its plan, all within the oracle's bar."""
+    from test_gpu_chain import chain_case
+    from test_gpu_dense import lattice_case
+    lattice = (*lattice_case(64, 40, 20, 4, seed=62), None)
+    batch = [lattice, system(150, 1, 63, ns=8), (*chain_case(30, 40, 6, 5), None), system(40, 0, 64)]
+    say("conveyor, propagators, chain, exact exponential")
+    out, done = abi.absorption_multi(batch)
+    assert np.all(done > 0)
+    for (non, H, mu, Cr), (re, im) in zip(batch, out):
+        o_re, o_im = orc.absorption(non, H, mu, C_rec=Cr)
+        assert rel(re + 1j * im, o_re + 1j * o_im) < 1e-5
+    p = abi.AbsPlan(lattice[0], lattice[1], lattice[1].shape[1], lattice[2], lattice[2].shape[1], lattice[1].shape[0])
+    re, im = p.execute()
+    p.close()
+    assert np.array_equal(re, out[0][0]) and np.array_equal(im, out[0][1])
