@@ -338,22 +338,33 @@ __global__ void __launch_bounds__(64) chain_adjoint_kernel(ChainArgs A) {
 static size_t chain_smem_fwd(int N, int R) { return (size_t)(64 / R) * N * 8; }
 static size_t chain_smem(int N, int T, int R) { return (size_t)(64 / R) * N * 24 + (size_t)T * 8; }
 
+// Steps of a launch, times the waves that share a SIMD.
+static double chain_steps(int N, int T, int m, int64_t nvec, int R) {
+  const int64_t M = (int64_t)(T - 1) * m + 1;
+  return ((double)((M - 1) / R) * chain_period(N, R) + 2 * R + N) *
+         std::max(1.0, (double)((nvec + 64 / R - 1) / (64 / R)) / 1024.0);
+}
+
 // Fewer lanes per vector where a short chain would leave lanes idle (the
-// period is at least 2 R + 2 steps): the R with the fewest steps, times the
-// waves that share a SIMD.  nvec: all vectors of the launch.
+// period is at least 2 R + 2 steps): the R with the fewest steps.  nvec: all
+// vectors of the launch.
 int chain_rows(int N, int T, int m, int64_t nvec, int64_t nfr) {
   if (nfr * N >= (int64_t)1 << 30) return 0;  // 32-bit record indexes
-  const int64_t M = (int64_t)(T - 1) * m + 1;
-  if (M * (N + 1) >= (int64_t)1 << 30) return 0;
+  if (((int64_t)(T - 1) * m + 1) * (N + 1) >= (int64_t)1 << 30) return 0;
   int best = 0;
   double cost = 0.0;
   for (int R : {21, 10, 5}) {
     if (chain_smem(N, T, R) > 160 * 1024) continue;
-    const double c = ((double)((M - 1) / R) * chain_period(N, R) + 2 * R + N) *
-                     std::max(1.0, (double)((nvec + 64 / R - 1) / (64 / R)) / 1024.0);
+    const double c = chain_steps(N, T, m, nvec, R);
     if (!best || c < cost) best = R, cost = c;
   }
   return best;
+}
+
+// (a step takes about 700 cycles: N = 128, 1,000 samples of 256 steps, 1,600 steps
+// in 0.55 ms; N = 16, 200 samples of 128, 286 in 0.09)
+bool chain_pays(const TrotterRun &r, int R, int windows, int per) {
+  return windows * (20000.0 + 700.0 * chain_steps(r.N, r.T, r.m, 3 * (int64_t)per, R)) < rows_cost(r);
 }
 
 static int launch_chain_fn(const void *fn, const ChainArgs &a, size_t smem, hipStream_t st) {

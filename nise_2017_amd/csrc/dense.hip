@@ -291,6 +291,15 @@ static RunCost run_cost(const TrotterRun &r) {
   return c;
 }
 constexpr double kLaunches = 20000.0;  // of the propagators
+double rows_cost(const TrotterRun &r) {
+  const RunCost c = run_cost(r);
+  return c.rows * (1.0 + c.load);
+}
+
+double dense_cost(const TrotterRun &r) {
+  const RunCost c = run_cost(r);
+  return kLaunches + c.build + std::max(c.chain, c.work);
+}
 
 static bool dense_fits(const TrotterRun &r) {
   return (int64_t)r.T * r.m <= kDenseMaxSweeps && r.N <= kDenseMaxN && r.F < (1 << 30) &&
@@ -301,11 +310,8 @@ static bool dense_fits(const TrotterRun &r) {
 // time (kernels, ms, conveyor and propagators: N = 25 lattice, 1,500 samples 1.56
 // and 0.59; N = 77, 333 samples 2.60 and 1.05; N = 64, 800 samples 2.43 and 1.24,
 // 1,500 samples 2.72 and 3.4; N = 121, 800 samples 4.50 and 4.41).
-bool dense_pays(const TrotterRun &r) {
-  if (!dense_fits(r)) return false;
-  const RunCost c = run_cost(r);
-  return kLaunches + c.build + std::max(c.chain, c.work) < 0.85 * c.rows * (1.0 + c.load);
-}
+bool dense_pays(const TrotterRun &r, double cost) { return dense_fits(r) && cost < 0.85 * rows_cost(r); }
+bool dense_pays(const TrotterRun &r) { return dense_pays(r, dense_cost(r)); }
 
 // Which Trotter runs of a batch go through propagators: those that pay by
 // themselves, U of all of them within kDenseBatchBytes.  But runs that share the

@@ -486,7 +486,9 @@ struct TrotterRun {
   int64_t S = 0, F = 0;
   int Kreal = 0, nasap = 0;
 };
+double rows_cost(const TrotterRun &run), dense_cost(const TrotterRun &run);  // cycles
 bool dense_pays(const TrotterRun &run);
+bool dense_pays(const TrotterRun &run, double cost);  // cost: of the propagators, as the caller runs them
 void dense_choice(const std::vector<TrotterRun> &runs, std::vector<char> &dense);
 inline size_t dense_u_bytes(int N, int64_t F) { return (size_t)F * 2 * ((N + 1) / 2) * N * 8; }
 // Kernel class of a system (dense.hip): 0 one wave per vector, 1 .. 3 one
@@ -596,6 +598,8 @@ struct ChainArgs {
 bool chain_mask(int N, const std::vector<uint8_t> &mask);
 // Lanes per vector, or 0 where the tables or LDS do not take the run.
 int chain_rows(int N, int T, int m, int64_t nvec, int64_t nfr);
+// Whether windows of `per` samples, one after the other, are faster than the row conveyor.
+bool chain_pays(const TrotterRun &run, int R, int windows, int per);
 inline int chain_groups(int nvec, int R) { return (nvec + 64 / R - 1) / (64 / R); }
 int launch_chain_tables(const FrameSource &src, int N, int64_t f_lo, int64_t nfr, float fac, const float *mu_rec,
                         int64_t mu_stride, float4 *rec, hipStream_t st);

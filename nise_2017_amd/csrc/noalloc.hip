@@ -86,13 +86,18 @@ int too_big(size_t need) {
   return NISE_ERR_RANGE;
 }
 
-// The run through per-frame propagators (dense.hip, the choice and kernels of
+// The run through per-frame propagators (dense.hip, the kernels of
 // nise_abs_plan_create) in windows of as many samples as the array holds; a
 // sample's response depends on its own frames only, so the windows give the
-// plan's partial rows bit for bit.  r: the conveyor's descriptor (sizes and
-// inputs); the array is free from `used` on.
-int run_dense(unsigned char *base, size_t used, const FrameSource &src, RowsArgs r, const Schedule &asap, int R, int ns,
-              float fac, float *re_S, float *im_S) {
+// plan's partial rows bit for bit.  Windows run one after the other, each as
+// long as a sample's chain of steps, and form the U of the frames that they
+// share again, so the choice counts them (100-site lattice, 150 samples every
+// 10, 256 steps: 17 windows 15.2 ms, the conveyor 4.5; 90 sites, 90 samples every
+// 14, 60 steps: 4 windows 1.3 ms, the conveyor 1.8).  ran stays false where the
+// conveyor is the better one.  r: the conveyor's descriptor (sizes and inputs);
+// the array is free from `used` on.
+int run_dense(unsigned char *base, size_t used, const FrameSource &src, RowsArgs r, const TrotterRun &run,
+              const Schedule &asap, int R, int ns, float fac, float *re_S, float *im_S, bool &ran) {
   int rc;
   const hipStream_t st = nullptr;
   const int N = r.N, T = r.tmax, npart = dense_parts(N, ns);
@@ -109,19 +114,34 @@ int run_dense(unsigned char *base, size_t used, const FrameSource &src, RowsArgs
   float *out = ar.take<float>(2 * (size_t)T);
   DiaSys *sysd = ar.take<DiaSys>(1);
   int2 *mapd = ar.take<int2>(ns);
-  if (!steps || !abd || !partial || !out || !sysd || !mapd) return too_big(kScratchBytes + 1);
+  float2 *state = ar.take<float2>((size_t)3 * N);
+  if (!steps || !abd || !partial || !out || !sysd || !mapd || !state) return NISE_OK;
   // samples per window, or, when one sample's window is too large, steps per
   // segment of each sample
   auto bytes = [&](int64_t f) {  // of f frames' phases, rotations and U
     return Arena::bytes_of((size_t)f * N, 8) + Arena::bytes_of((size_t)f * sch.K, 8) +
            Arena::bytes_of(dense_u_bytes(N, f), 1);
   };
-  float2 *state = ar.take<float2>((size_t)3 * N);
-  if (!state || ar.used + bytes(1) > kScratchBytes) return too_big(ar.used + bytes(1));
+  if (ar.used + bytes(1) > kScratchBytes) return NISE_OK;
   int per = ns, seg = T;
   auto frames = [&](int n) { return (int64_t)(n - 1) * r.sample + T; };
   while (per > 1 && ar.used + bytes(frames(per)) > kScratchBytes) per = per > 16 ? per * 7 / 8 : per - 1;
   while (per == 1 && seg > 1 && ar.used + bytes(seg) > kScratchBytes) seg = seg > 16 ? seg * 7 / 8 : seg - 1;
+  auto window = [&](int s0, int t0, int &n, int64_t &nf) {  // its samples and frames
+    n = std::min(per, ns - s0), nf = seg < T ? std::min(seg, T - t0) : frames(n);
+  };
+  int n;
+  int64_t nf;
+  double cost = 0.0;
+  for (int s0 = 0; s0 < ns; s0 += per)
+    for (int t0 = 0; t0 < T; t0 += seg) {
+      window(s0, t0, n, nf);
+      TrotterRun w = run;
+      w.S = n, w.F = nf, w.T = seg < T ? (int)nf : T;
+      cost += dense_cost(w);
+    }
+  if (!dense_pays(run, cost)) return NISE_OK;
+  ran = true;
   NISE_HIP_CHECK(hipMemcpy(steps, tab.data(), tab.size() * sizeof(uint2), hipMemcpyHostToDevice));
   NISE_HIP_CHECK(hipMemcpy(abd, ab.data(), ab.size() * 4, hipMemcpyHostToDevice));
   std::vector<int2> map(ns);
@@ -130,8 +150,8 @@ int run_dense(unsigned char *base, size_t used, const FrameSource &src, RowsArgs
   r.nlayers = sch.nlayers(), r.K = sch.K, r.steps = steps;
   for (int s0 = 0; s0 < ns; s0 += per)
     for (int t0 = 0; t0 < T; t0 += seg) {
-      const int n = std::min(per, ns - s0);
-      const int64_t f0 = (int64_t)(r.begin + s0) * r.sample + t0, nf = seg < T ? std::min(seg, T - t0) : frames(n);
+      window(s0, t0, n, nf);
+      const int64_t f0 = (int64_t)(r.begin + s0) * r.sample + t0;
       Arena w{base, ar.used};
       float2 *diag = w.take<float2>((size_t)nf * N), *cs = w.take<float2>((size_t)nf * sch.K);
       float2 *U = reinterpret_cast<float2 *>(w.take<unsigned char>(dense_u_bytes(N, nf)));
@@ -154,10 +174,12 @@ int run_dense(unsigned char *base, size_t used, const FrameSource &src, RowsArgs
 
 // A nearest-neighbour chain through its own kernel (chain.hip) in windows of
 // as many samples as the array holds, bit for bit the plan's partial rows.
-// ran stays false where one sample's records do not fit: the caller's row
-// conveyor gives the same results.
-int run_chain(unsigned char *base, size_t used, const FrameSource &src, const RowsArgs &r, int R, int ns, float fac,
-              float *re_S, float *im_S, bool &ran) {
+// ran stays false where one sample's records do not fit, or where so many
+// windows, one after the other, take longer than the caller's row conveyor,
+// which gives the same results (150 sites, 20 samples every 100, 5,750 steps: 20
+// windows 210 ms, the conveyor 128; 5,500 steps: 5 windows 51 ms, 124).
+int run_chain(unsigned char *base, size_t used, const FrameSource &src, const RowsArgs &r, const TrotterRun &run, int R,
+              int ns, float fac, float *re_S, float *im_S, bool &ran) {
   int rc;
   const hipStream_t st = nullptr;
   const int N = r.N, T = r.tmax;
@@ -169,7 +191,7 @@ int run_chain(unsigned char *base, size_t used, const FrameSource &src, const Ro
   auto bytes = [&](int n) { return Arena::bytes_of((size_t)frames(n) * N, 2 * sizeof(float4)); };
   int per = ns;
   while (per && ar.used + bytes(per) > kScratchBytes) per = per > 16 ? per * 7 / 8 : per - 1;
-  if (!per) return NISE_OK;
+  if (!per || (per < ns && !chain_pays(run, R, (ns + per - 1) / per, per))) return NISE_OK;
   float4 *rec = ar.take<float4>((size_t)frames(per) * N * 2);
   if (!rec) return NISE_OK;
   ran = true;
@@ -291,17 +313,18 @@ extern "C" int nise_absorption_batched_noalloc(const t_non *non, const float *H_
   bool pf = false;
   if ((rc = rows_prepare(&r, 1, R, wmap, smem, pf))) return rc;
   if ((int)wmap.size() != nwg) return set_error("row conveyor: workgroup map mismatch"), NISE_ERR_ARG;
-  if (const int Rc = chain_mask(N, mask) ? chain_rows(N, T, m, nvec, nfr) : 0) {
-    bool ran = false;
-    if ((rc = run_chain(ds->ptr, ar0, src, r, Rc, end - begin, trotter_factor(non->deltat, 1, m), re_S, im_S, ran)) || ran)
-      return rc;
-  } else if (dense_pays({N, T, m, end - begin, nfr, asap.Kreal, asap.nlayers()}))
-    return run_dense(ds->ptr, ar0, src, r, asap, R, end - begin, trotter_factor(non->deltat, 1, m), re_S, im_S);
+  const TrotterRun run{N, T, m, end - begin, nfr, asap.Kreal, asap.nlayers()};
+  const float fac = trotter_factor(non->deltat, 1, m);
+  bool ran = false;
+  if (const int Rc = chain_mask(N, mask) ? chain_rows(N, T, m, nvec, nfr) : 0)
+    rc = run_chain(ds->ptr, ar0, src, r, run, Rc, end - begin, fac, re_S, im_S, ran);
+  else if (dense_pays(run))
+    rc = run_dense(ds->ptr, ar0, src, r, run, asap, R, end - begin, fac, re_S, im_S, ran);
+  if (rc || ran) return rc;
   if (!tab.empty()) NISE_HIP_CHECK(hipMemcpy(steps, tab.data(), tab.size() * sizeof(uint2), hipMemcpyHostToDevice));
   if (!ab.empty()) NISE_HIP_CHECK(hipMemcpy(abd, ab.data(), ab.size() * 4, hipMemcpyHostToDevice));
   // per-frame half-step phases and rotation tables (every entry written)
-  if ((rc = launch_frame_tables(src, N, sch, abd, trotter_factor(non->deltat, 1, m), f_lo, nfr, diag, cs, st, nullptr)))
-    return rc;
+  if ((rc = launch_frame_tables(src, N, sch, abd, fac, f_lo, nfr, diag, cs, st, nullptr))) return rc;
 
   NISE_HIP_CHECK(hipMemcpy(sysd, &r, sizeof(r), hipMemcpyHostToDevice));
   NISE_HIP_CHECK(hipMemcpy(wmapd, wmap.data(), wmap.size() * sizeof(int2), hipMemcpyHostToDevice));

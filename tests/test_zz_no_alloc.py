@@ -101,3 +101,26 @@ def test_noalloc_refuses_runs_beyond_its_scratch():
                                                    mu.shape[1], nfr, None, re, im)
     assert rc == abi.NISE_ERR_RANGE
     assert b"scratch" in abi.lib().nise_last_error()
+
+
+def test_many_windows_keep_the_conveyor():
+    """A run whose propagators would need a dozen windows of the array, one after
+    the other, takes the conveyor: bit for bit the plan's with the default row
+    count, whose own choice here is the propagators."""
+    import torch
+
+    from test_gpu_dense import lattice_case
+    non, H, mu = lattice_case(100, 256, 150, 10, seed=84)
+    Hd, mud = torch.from_numpy(H).cuda(), torch.from_numpy(mu).cuda()
+    torch.cuda.synchronize()
+    p = abi.AbsPlan(non, Hd, H.shape[1], mud, mu.shape[1], H.shape[0], where=abi.NISE_DEVICE)
+    dense = p.execute()
+    p.set_rows(0)
+    rows = p.execute()
+    p.close()
+    assert not np.array_equal(dense[0], rows[0])
+    re, im = np.zeros(256, np.float32), np.zeros(256, np.float32)
+    say("N=100 lattice, 150 samples of 256 steps")
+    abi.check(abi.lib().nise_absorption_batched_noalloc(C.byref(non), abi.ptr(Hd), H.shape[1], abi.ptr(mud), mu.shape[1],
+                                                        H.shape[0], None, re, im))
+    assert np.array_equal(re, rows[0]) and np.array_equal(im, rows[1])
