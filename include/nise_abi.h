@@ -284,16 +284,23 @@ int nise_abs_plan_create_onfly(nise_abs_plan **plan, const t_non *non,
  * (multi-wave), 64 (one wave) or -2 / -4 (one wave, 2 or 4 slots per lane). */
 int nise_abs_plan_set_shape(nise_abs_plan *plan, int vp, int samples_per_wg,
                             int block);
-/* Row conveyor (the default): one wave per workgroup holding 64/rows
- * vectors, rows rotations of a layer at a time (1, 2, 4, 8, 16, 32 or 64; 0
- * picks the count from the coupling structure). */
+/* Row conveyor: one wave per workgroup holding 64/rows vectors, rows
+ * rotations of a layer at a time (1, 2, 4, 8, 16, 32 or 64; 0 picks the count
+ * from the coupling structure).  A new plan takes it, or for nearest-neighbour
+ * chains kernels of their own (the same results bit for bit), or per-frame
+ * propagators where few vectors leave the chip idle (at most 256 sweeps, within
+ * 1.5e-5 of the reference's rounding); set_rows and set_shape leave those. */
 int nise_abs_plan_set_rows(nise_abs_plan *plan, int rows);
 /* Autotuner: times each candidate configuration (row conveyor with 1..64
- * rows, slot-conveyor shapes) on the plan's own workload and keeps the
- * fastest.  ms / codes (host, n entries each, optional) receive each timed
- * candidate's conveyor time and code (rows R as R; slot shapes as
- * -(10000 vp + 1000 spw + block), block -2/-4 as 902/904).  Returns the
- * number of candidates timed, or minus an error code. */
+ * rows, slot-conveyor shapes, the plan's chain kernels) on the plan's own
+ * workload and keeps the fastest.  All candidates agree within 1e-6: a plan's
+ * propagators are one of them only where their response does, so tuning a plan
+ * that runs through propagators usually puts it on a conveyor, with the
+ * reference's rounding and slower.  ms / codes (host, n entries each, optional)
+ * receive each timed candidate's conveyor time and code (rows R as R; slot
+ * shapes as -(10000 vp + 1000 spw + block), block -2/-4 as 902/904; the plan's
+ * own kernels on entry as 0).  Returns the number of candidates timed, or minus
+ * an error code. */
 int nise_abs_plan_autotune(nise_abs_plan *plan, float *ms, int *codes, int n);
 /* Run the plan; re_S / im_S (host, tmax1 each) may be NULL to leave the
  * result on the device.  flags bit 0: time the stages with HIP events;

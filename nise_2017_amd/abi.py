@@ -210,8 +210,8 @@ class AbsPlan:
 
     def autotune(self):
         """Time the candidate configurations and keep the fastest; returns
-        [(code, conveyor ms), ...] (code: rows R, or -(10000 vp + 1000 spw +
-        block))."""
+        [(code, conveyor ms), ...] (code: rows R, -(10000 vp + 1000 spw +
+        block), or 0 for the chain kernels or propagators on entry)."""
         ms = (C.c_float * 16)()
         codes = (C.c_int * 16)()
         k = lib().nise_abs_plan_autotune(self.h, ms, codes, 16)

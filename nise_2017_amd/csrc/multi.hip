@@ -722,15 +722,14 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
   // many couplings per layer take wide layers, which shortens the chain of
   // layers each of their workgroups walks)
   int R = 0, cap = kMultiRowCap;
-  bool own = R_force == 0 || R_force == -1;  // the default: systems that pay for it take the dense propagators
+  // with their own counts (whatever the cap), chains take their kernels and
+  // systems that pay for it the dense propagators
   std::vector<int64_t> sig;
   if (R_force == 0 && cache.tune_R != 0) batch_signature(systems, nsys, sig);
-  if (R_force > 0) R = R_force;
-  else if (R_force < -1) cap = -R_force;
-  else if (R_force == 0 && cache.tune_R != 0 && sig == cache.tune_sig) {
-    if (cache.tune_R > 0) R = cache.tune_R, own = false;
-    else if (cache.tune_R < -1) cap = -cache.tune_R, own = false;
-  }
+  const int pick = R_force == 0 && cache.tune_R != 0 && sig == cache.tune_sig ? cache.tune_R : R_force;
+  if (pick > 0) R = pick;
+  else if (pick < -1) cap = -pick;
+  const bool own = pick <= 0;
   // 4. tables of the Trotter systems.  The row schedules whose inputs changed
   //    are built first, on up to kSchedThreads host threads (they are
   //    independent; one after the other they took 40 ms for 16 systems up to
@@ -951,7 +950,7 @@ extern "C" int nise_absorption_multi(const nise_system *systems, int nsys, int w
   return multi_run(systems, nsys, where, re_S, im_S, done_ms, 0);
 }
 
-// Times the batch with each system's own row count (capped at 32, 16 and
+// Times the batch with each system's own choice (rows capped at 32, 16 and
 // 64: codes 0, -16, -64) and with every common row count of the row
 // conveyor (1, 2, ..., 64; the best of two runs each, after a warm run) and
 // keeps the fastest for later nise_absorption_multi calls on a batch of the
