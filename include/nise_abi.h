@@ -376,8 +376,9 @@ int nise_2dir_batched(const t_non *non, const float *H_rec, int64_t H_stride,
  * windows of at most window_samples start points (0: sized to a quarter of
  * the free device memory); a reader thread reads the next window's records
  * into pinned host memory and uploads them on a copy stream while the
- * current window runs as nise_absorption_batched; the windows' responses
- * are summed in FP64.  No counterpart in the reference, which reads one
+ * current window runs as nise_absorption_batched, with the kernels that the
+ * whole run would take in one pass; the windows' responses are summed in
+ * FP64.  No counterpart in the reference, which reads one
  * frame per step (src/read_trajectory.c:138-173); absorption() uses it when
  * the frame range exceeds a third of the free device memory.  re_S/im_S:
  * tmax1 floats (host), un-normalised as src/absorption.c:112-146 leaves

@@ -272,11 +272,12 @@ int onfly_scheme(const t_non *non) {
 
 // Plan set-up shared by nise_abs_plan_create, nise_abs_plan_create_onfly
 // (pos_rec: position records for on-the-fly couplings, else null) and
-// nise_absorption_batched (one_run).
+// absorption_part (one_run; whole: the samples and frames of the run that this
+// one is a window of, 0: itself).
 static int plan_create(nise_abs_plan **out, const t_non *non, const float *H_rec, int64_t H_stride,
                        const float *mu_rec, int64_t mu_stride, int64_t nframes, const float *coupling_rec,
                        const float *pos_rec, int64_t pos_stride, const float *box_rec, int where, int kernel,
-                       bool one_run = false) {
+                       bool one_run = false, int64_t S_whole = 0, int64_t F_whole = 0) {
   *out = nullptr;
   int rc = ensure_device();
   if (rc) return rc;
@@ -391,8 +392,8 @@ static int plan_create(nise_abs_plan **out, const t_non *non, const float *H_rec
     P->rows = rows_for(N, P->sch_asap.Kreal, P->sch_asap.nlayers());
     P->mask = mask;
     if (chain_mask(N, mask)) P->chain = chain_rows(N, P->tmax, P->m, 3 * (int64_t)(P->end - P->begin), nfr);
-    P->dense = !P->chain &&
-               dense_pays({N, P->tmax, P->m, P->end - P->begin, nfr, P->sch_asap.Kreal, P->sch_asap.nlayers()});
+    P->dense = !P->chain && dense_pays({N, P->tmax, P->m, S_whole ? S_whole : P->end - P->begin,
+                                        F_whole ? F_whole : nfr, P->sch_asap.Kreal, P->sch_asap.nlayers()});
     if (P->chain && (rc = P->rec.alloc((size_t)nfr * N * 2 * sizeof(float4)))) return rc;
     // a run made once does not pay for the list schedule
     if (P->dense && one_run) pack_schedule_rows(P->sch_asap, P->rows, P->sch_rows);
@@ -712,21 +713,30 @@ extern "C" int nise_abs_plan_adjoint(nise_abs_plan *P, const float *g_re, const 
 
 extern "C" void nise_abs_plan_destroy(nise_abs_plan *P) { delete P; }
 
-extern "C" int nise_absorption_batched(const t_non *non, const float *H_rec, int64_t H_stride,
-                                       const float *mu_rec, int64_t mu_stride, int64_t nframes,
-                                       const float *coupling_rec, int where, int kernel,
-                                       float *re_S, float *im_S) {
+// nise_absorption_batched for a window of a run of S_whole samples over F_whole
+// frames (0: the run itself): the kernels are chosen for the whole run, whose
+// one-pass result the windows then add up to.
+int nise::absorption_part(const t_non *non, const float *H_rec, int64_t H_stride, const float *mu_rec, int64_t mu_stride,
+                          int64_t nframes, const float *coupling_rec, int where, int kernel, int64_t S_whole,
+                          int64_t F_whole, float *re_S, float *im_S) {
   if (non && non->propagation == 0) {  // exact exponential: the dense propagators
     nise_system y{non, H_rec, H_stride, mu_rec, mu_stride, nframes, coupling_rec};
     return nise_absorption_multi(&y, 1, where, re_S, im_S, nullptr);
   }
   nise_abs_plan *P = nullptr;
   int rc = plan_create(&P, non, H_rec, H_stride, mu_rec, mu_stride, nframes, coupling_rec, nullptr, 0, nullptr, where,
-                       kernel, true);
+                       kernel, true, S_whole, F_whole);
   if (rc) return rc;
   rc = nise_abs_plan_execute(P, re_S, im_S, 0);
   nise_abs_plan_destroy(P);
   return rc;
+}
+
+extern "C" int nise_absorption_batched(const t_non *non, const float *H_rec, int64_t H_stride,
+                                       const float *mu_rec, int64_t mu_stride, int64_t nframes,
+                                       const float *coupling_rec, int where, int kernel,
+                                       float *re_S, float *im_S) {
+  return absorption_part(non, H_rec, H_stride, mu_rec, mu_stride, nframes, coupling_rec, where, kernel, 0, 0, re_S, im_S);
 }
 
 // ---------------------------------------------------------------------------

@@ -309,9 +309,9 @@ extern "C" int nise_absorption_stream(const t_non *non, int window_samples, floa
     const int i = (int)(k % 2);
     t_non loc = *non;  // the window's records start at its first frame
     loc.begin = 0, loc.end = w.e - w.b;
-    const int r = nise_absorption_batched(&loc, dH[i].as<float>(), hw, ctype ? dmu0.as<float>() : dmu[i].as<float>(),
-                                          mw, w.nfr, ctype ? dC.as<float>() : nullptr, NISE_DEVICE, 0, wr.data(),
-                                          wi.data());
+    const int r = absorption_part(&loc, dH[i].as<float>(), hw, ctype ? dmu0.as<float>() : dmu[i].as<float>(), mw, w.nfr,
+                                  ctype ? dC.as<float>() : nullptr, NISE_DEVICE, 0, end - begin,
+                                  window_frames(end - begin, sr, T), wr.data(), wi.data());
     if (reader.joinable()) reader.join();
     if (r) {
       (void)hipStreamDestroy(cp);

@@ -488,6 +488,9 @@ struct TrotterRun {
 };
 double rows_cost(const TrotterRun &run), dense_cost(const TrotterRun &run);  // cycles
 bool dense_pays(const TrotterRun &run);
+int absorption_part(const t_non *non, const float *H_rec, int64_t H_stride, const float *mu_rec, int64_t mu_stride,
+                    int64_t nframes, const float *coupling_rec, int where, int kernel, int64_t S_whole, int64_t F_whole,
+                    float *re_S, float *im_S);  // api_singles.hip
 bool dense_pays(const TrotterRun &run, double cost);  // cost: of the propagators, as the caller runs them
 void dense_choice(const std::vector<TrotterRun> &runs, std::vector<char> &dense);
 inline size_t dense_u_bytes(int N, int64_t F) { return (size_t)F * 2 * ((N + 1) / 2) * N * 8; }

@@ -81,6 +81,26 @@ def test_stream_matches_batched_and_oracle(orc, tmp_path, W, prop, ctype):
     assert e1 < 1e-6 and e2 < 1e-5
 
 
+def test_windows_take_the_kernels_of_the_whole_run(tmp_path):
+    """A lattice whose windows of 60 samples would go through per-frame
+    propagators, but not its 2,400 samples in one pass: the windows follow the
+    whole run and add up to its result within 1e-6 (the two kernels differ by the
+    reference's rounding, more than that)."""
+    from test_gpu_dense import lattice_case
+    non, H, mu = lattice_case(100, 48, 2400, 1, seed=710)
+    non.energyFName, non.dipoleFName, _ = files(str(tmp_path), H, mu)
+    say("N=100 lattice, 2,400 samples in windows of 60")
+    rc, re, im = run_stream(non, 60)
+    assert rc == 0, abi.lib().nise_last_error().decode()
+    p = abi.AbsPlan(non, H, H.shape[1], mu, mu.shape[1], H.shape[0])
+    one = p.execute()
+    p.set_rows(0)
+    rows = p.execute()
+    p.close()
+    assert np.array_equal(one[0], rows[0])
+    assert rel(re + 1j * im, one[0] + 1j * one[1]) < 1e-6
+
+
 def test_short_file_is_an_error(tmp_path):
     N, T, sr = 8, 16, 4
     H, mu = synth.chain_absorption(N=N, nframes=60, seed=9)
