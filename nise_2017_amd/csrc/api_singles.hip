@@ -93,7 +93,6 @@ int upload_dense(nise_abs_plan *P) {
   d.mu_rec = r.mu_rec, d.mu_stride = r.mu_stride, d.partial = r.partial;
   d.hist = r.hist, d.hist_every = r.hist_every, d.nck = r.nck;
   int rc;
-  if ((rc = P->U.alloc(dense_u_bytes(r.N, P->f_hi - P->f_lo)))) return rc;
   d.U = P->U.as<float2>();
   const int ns = P->end - P->begin;
   P->nwg = ns, P->npart = dense_parts(r.N, ns);
@@ -121,10 +120,26 @@ int upload_rows_desc(nise_abs_plan *P) {
   return upload(P->row_wmap, wmap.data(), wmap.size() * sizeof(int2), P->st);
 }
 
-// Row conveyor set-up: schedule, step table, tables and partials.
+// Per-frame tables of the current schedule.
+int alloc_tables(nise_abs_plan *P) {
+  const int64_t nfr = P->f_hi - P->f_lo, K = std::max(P->sch.K, 1);
+  int rc;
+  if ((rc = P->diag.alloc((size_t)nfr * P->N * sizeof(float2))) || (rc = P->cs.alloc((size_t)nfr * K * sizeof(float2))))
+    return rc;
+  return P->every ? P->jf.alloc((size_t)nfr * K * 4) : NISE_OK;
+}
+
+// Row conveyor set-up: schedule, step table, tables and partials.  The chain
+// kernels need only their records and the partials.
 int build_rows(nise_abs_plan *P) {
   int rc;
   P->sch = P->sch_rows;
+  P->npart = 3 * (P->end - P->begin);  // one row per vector
+  if ((rc = P->partial.alloc((size_t)std::max(P->npart, 1) * P->tmax * sizeof(double2)))) return rc;
+  if (P->chain) {
+    P->nwg = chain_groups(P->npart, P->chain);
+    return NISE_OK;
+  }
   std::vector<uint2> tab;
   rows_step_table(P->sch, P->rows, tab);
   if ((rc = upload(P->row_steps, tab.data(), tab.size() * sizeof(uint2), P->st))) return rc;
@@ -132,16 +147,10 @@ int build_rows(nise_abs_plan *P) {
   rows_device_order(P->sch, P->rows, ab);
   if ((rc = upload(P->ab, ab.data(), ab.size() * 4, P->st))) return rc;
   if ((rc = upload(P->layer_off, P->sch.layer_off.data(), P->sch.layer_off.size() * 4, P->st))) return rc;
-  const int64_t nfr = P->f_hi - P->f_lo;
-  if ((rc = P->cs.alloc((size_t)nfr * std::max(P->sch.K, 1) * sizeof(float2)))) return rc;
-  if (P->every && (rc = P->jf.alloc((size_t)nfr * std::max(P->sch.K, 1) * 4))) return rc;
+  if ((rc = alloc_tables(P))) return rc;
   const int G = 64 / P->rows;
-  P->nwg = (3 * (P->end - P->begin) + G - 1) / G;
-  P->npart = 3 * (P->end - P->begin);  // one row per vector
-  if ((rc = P->partial.alloc((size_t)std::max(P->npart, 1) * P->tmax * sizeof(double2)))) return rc;
-  if ((rc = upload_rows_desc(P))) return rc;
-  if (P->chain) P->nwg = chain_groups(P->npart, P->chain);
-  return NISE_OK;
+  P->nwg = (P->npart + G - 1) / G;
+  return upload_rows_desc(P);
 }
 
 // Slot assignment: consecutive samples, three polarisations each, spw
@@ -150,6 +159,7 @@ int build_slots(nise_abs_plan *P) {
   if (P->rows) return build_rows(P);
   int rc0;
   P->sch = P->sch_asap;
+  if ((rc0 = alloc_tables(P))) return rc0;
   if ((rc0 = upload(P->ab, P->sch.ab.data(), P->sch.ab.size() * 4, P->st))) return rc0;
   if ((rc0 = upload(P->layer_off, P->sch.layer_off.data(), P->sch.layer_off.size() * 4, P->st))) return rc0;
   std::vector<SlotDesc> sl;
@@ -384,8 +394,6 @@ static int plan_create(nise_abs_plan **out, const t_non *non, const float *H_rec
     if ((rc = P->resp_plain.alloc(P->tmax * sizeof(double2)))) return rc;
   } else {
     int64_t nfr = P->f_hi - P->f_lo;
-    if ((rc = P->diag.alloc((size_t)nfr * N * sizeof(float2)))) return rc;
-    if ((rc = P->cs.alloc((size_t)nfr * std::max(P->sch_asap.K, 1) * sizeof(float2)))) return rc;
     // default: the row conveyor with rows matched to the layer width; the
     // slot conveyor's shape (set_shape) stays available
     P->vp = 16, P->spw = 5;
@@ -394,11 +402,23 @@ static int plan_create(nise_abs_plan **out, const t_non *non, const float *H_rec
     if (chain_mask(N, mask)) P->chain = chain_rows(N, P->tmax, P->m, 3 * (int64_t)(P->end - P->begin), nfr);
     P->dense = !P->chain && dense_pays({N, P->tmax, P->m, S_whole ? S_whole : P->end - P->begin,
                                         F_whole ? F_whole : nfr, P->sch_asap.Kreal, P->sch_asap.nlayers()});
-    if (P->chain && (rc = P->rec.alloc((size_t)nfr * N * 2 * sizeof(float4)))) return rc;
-    // a run made once does not pay for the list schedule
-    if (P->dense && one_run) pack_schedule_rows(P->sch_asap, P->rows, P->sch_rows);
-    else build_schedule_rows(N, mask, P->rows, P->sch_rows);
-    if ((rc = build_slots(P))) return rc;
+    auto set_up = [&]() {
+      int r;
+      if ((P->chain && (r = P->rec.alloc((size_t)nfr * N * 2 * sizeof(float4)))) ||
+          (P->dense && (r = P->U.alloc(dense_u_bytes(N, nfr)))))
+        return r;
+      // a run made once does not pay for the list schedule
+      if (P->dense && one_run) pack_schedule_rows(P->sch_asap, P->rows, P->sch_rows);
+      else build_schedule_rows(N, mask, P->rows, P->sch_rows);
+      return build_slots(P);
+    };
+    rc = set_up();
+    if (rc == NISE_ERR_NOMEM && (P->chain || P->dense)) {  // the conveyor may still fit
+      P->chain = 0, P->dense = false;
+      P->rec.release(), P->U.release();
+      rc = set_up();
+    }
+    if (rc) return rc;
   }
   NISE_HIP_CHECK(hipStreamSynchronize(P->st));
   *out = guard.release();
@@ -623,7 +643,6 @@ extern "C" int nise_abs_plan_enable_adjoint(nise_abs_plan *P, int every) {
   if (nslot * nck > INT32_MAX) return set_error("too many checkpoints"), NISE_ERR_RANGE;
   int rc;
   if ((rc = P->ck.alloc((size_t)nslot * nck * N * sizeof(float2)))) return rc;
-  if ((rc = P->jf.alloc((size_t)(P->f_hi - P->f_lo) * std::max(P->sch.K, 1) * 4))) return rc;
   P->every = every, P->nck = nck;
   // backward grouping: consecutive slots, adj_vp per single-wave workgroup
   P->adj_vp = adjoint_vp(P->sch, N, T);

@@ -580,9 +580,10 @@ using namespace nise;
 // One batch; R_force > 0 runs every Trotter system with that row count,
 // R_force = -1 each with its own (capped at kMultiRowCap), R_force < -1 each
 // with its own capped at -R_force; R_force = 0 takes the tuned choice for a
-// batch of this shape, else each system's own count.
+// batch of this shape, else each system's own count.  conveyor: no chain
+// kernels or propagators, whose tables take more memory.
 static int multi_run(const nise_system *systems, int nsys, int where, float *re_S, float *im_S, double *done_ms,
-                     int R_force) {
+                     int R_force, bool conveyor = false) {
   int rc = ensure_device();
   if (rc) return rc;
   if (nsys < 1 || !systems || !re_S || !im_S) return set_error("multi: bad arguments"), NISE_ERR_ARG;
@@ -729,7 +730,7 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
   const int pick = R_force == 0 && cache.tune_R != 0 && sig == cache.tune_sig ? cache.tune_R : R_force;
   if (pick > 0) R = pick;
   else if (pick < -1) cap = -pick;
-  const bool own = pick <= 0;
+  const bool own = pick <= 0 && !conveyor;
   // 4. tables of the Trotter systems.  The row schedules whose inputs changed
   //    are built first, on up to kSchedThreads host threads (they are
   //    independent; one after the other they took 40 ms for 16 systems up to
@@ -947,7 +948,15 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
 
 extern "C" int nise_absorption_multi(const nise_system *systems, int nsys, int where, float *re_S,
                                      float *im_S, double *done_ms) {
-  return multi_run(systems, nsys, where, re_S, im_S, done_ms, 0);
+  int rc = multi_run(systems, nsys, where, re_S, im_S, done_ms, 0);
+  if (rc == NISE_ERR_NOMEM) {  // without the chains' records and the propagators the batch may still fit
+    NISE_HIP_CHECK(hipStreamSynchronize(default_stream()));
+    NISE_HIP_CHECK(hipStreamSynchronize(aux_stream()));
+    for (auto &s : g_multi.sys)
+      if (s) s->rec.release(), s->U.release();
+    rc = multi_run(systems, nsys, where, re_S, im_S, done_ms, 0, true);
+  }
+  return rc;
 }
 
 // Times the batch with each system's own choice (rows capped at 32, 16 and

@@ -28,6 +28,7 @@ int DevBuf::alloc(size_t n) {
   hipError_t e = hipMalloc(&p, n);
   if (e != hipSuccess) {
     p = nullptr;
+    (void)hipGetLastError();  // or the next launch check, of a run that did without, would report it
     set_error("hipMalloc(%zu) failed: %s", n, hipGetErrorString(e));
     return NISE_ERR_NOMEM;
   }

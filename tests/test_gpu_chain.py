@@ -120,3 +120,32 @@ def test_batch_of_uneven_chains_matches_plans():
         p.close()
         assert np.array_equal(re, r) and np.array_equal(im, i), non.singles
     assert np.all(done > 0)
+
+
+def test_chain_plan_holds_only_its_own_tables():
+    """A chain plan's device memory is its records (32 bytes per site and frame)
+    and the partial sums; the conveyor's tables come when the plan leaves the
+    chain kernels."""
+    import torch
+    N, T, ns, sr = 100, 64, 3000, 4
+    non, H, mu = chain_case(N, T, ns, sr)
+    Hd, mud = torch.from_numpy(H).cuda(), torch.from_numpy(mu).cuda()
+    torch.cuda.synchronize()
+    abi.AbsPlan(non, Hd, H.shape[1], mud, mu.shape[1], H.shape[0], where=abi.NISE_DEVICE).close()
+    free = torch.cuda.mem_get_info()[0]
+    p = abi.AbsPlan(non, Hd, H.shape[1], mud, mu.shape[1], H.shape[0], where=abi.NISE_DEVICE)
+    try:
+        chain = p.execute()
+        used = free - torch.cuda.mem_get_info()[0]
+        frames = (ns - 1) * sr + T
+        rec, partial, tables = 32 * N * frames, 3 * ns * T * 16, 16 * N * frames
+        print(f"[chain] plan of {rec >> 20} + {partial >> 20} MiB holds {used >> 20}", flush=True)
+        assert used < rec + partial + tables // 2
+        p.set_rows(0)
+        rows = p.execute()
+        assert np.array_equal(chain[0], rows[0]) and np.array_equal(chain[1], rows[1])
+        p.set_shape(16, 5)
+        slots = p.execute()
+        assert rel(slots[0] + 1j * slots[1], rows[0] + 1j * rows[1]) < 1e-6
+    finally:
+        p.close()
