@@ -364,7 +364,11 @@ int nise_row_schedule(int N, const uint8_t *mask, int R, uint32_t *ab_out,
  * the technique has the EA pathway.  R12 (host, 12 x tmax3 x tmax1, t1
  * fastest) receives the sums over samples and items of rrIpar, riIpar,
  * rrIIpar, riIIpar, then the per and cro planes in the same order,
- * un-normalised: what the reference reduces before print2D. */
+ * un-normalised: what the reference reduces before print2D.  tmax1 from 16
+ * on with no waiting time, N <= 61 and N + 3 <= 3 tmax1 goes through basis
+ * vectors: fused products and another order of the sums, as near to 64 bits as
+ * the reference's FP32 arithmetic; shorter windows propagate every vector in
+ * the reference's operation order. */
 int nise_2dir_batched(const t_non *non, const float *H_rec, int64_t H_stride,
                       const float *mu_rec, int64_t mu_stride, int64_t nframes,
                       const float *coupling_rec, const float *anh_rec,

@@ -6,8 +6,8 @@ t3 = 0 the three pathways of harmonic transitions sum to zero), Trotter substeps
 technique, per-frame anharmonicities, the Coupling type, samples that do not
 start at frame 0.  Large N and short t3 windows take the pathways apart: their
 sum there is a difference of about 1e-3 of its terms, in which the FP32
-oracle is itself 2e-4 to 1.4e-3 off the 64-bit result (as far as the path or
-further).  Tolerance as in test_gpu_2dir.py."""
+oracle is itself 2e-4 to 1.4e-3 off the 64-bit result (test_large_n_sum
+compares both with it).  Tolerance as in test_gpu_2dir.py."""
 import numpy as np
 import pytest
 
@@ -64,3 +64,21 @@ def test_dense_coupling_type_vs_oracle(orc):
     dev = [torch.from_numpy(x).cuda() for x in (Hc, mur, Cr)]
     torch.cuda.synchronize()
     assert np.array_equal(R, abi.twodir_batched(make(), dev[0], dev[1], coupling_rec=dev[2]))
+
+
+@pytest.mark.parametrize("N,T1,T3,S", [(33, 16, 3, 4), (45, 16, 2, 4), (61, 22, 2, 3), (40, 30, 20, 3)])
+def test_large_n_sum_vs_64_bits(orc, N, T1, T3, S):
+    """The sum of the three pathways above N = 32 against direct propagation in
+    64 bits: no further off than the reference's FP32 arithmetic (the oracle; 1.5
+    for the chance of two roundings of the same size)."""
+    from perf import cases
+    case = dict(kind="2dir", N=N, t1=T1, t3=T3, samples=S, every=9, anh=16.0)
+    print(f"[basis] 64 bits: N={N} T1={T1} T3={T3}", flush=True)
+    s = cases.prepare(case, 77)
+    R = cases.run(s)
+    exact = cases.exact(case, 77)
+    s = cases.inputs(case, 77)
+    ref = orc.twodir(s["non"], s["H"].cpu().numpy(), s["mu"].cpu().numpy(), acc64=True)
+    e, e_ref = rel(R, exact), rel(ref, exact)
+    print(f"[basis] {e:.1e}, oracle {e_ref:.1e}", flush=True)
+    assert e < 1.5 * e_ref
