@@ -243,9 +243,12 @@ int nise_absorption_batched(const t_non *non, const float *H_rec,
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): what nise_absorption_batched computes for device
- * records (where = NISE_DEVICE, kernel 0) with propagation 1, bit for bit,
- * using only a library-owned 32 MiB device array per GPU (held until the
- * process ends) for its mask, schedule, per-frame tables and partial sums.
+ * records (where = NISE_DEVICE, kernel 0) with propagation 1, using only a
+ * library-owned 32 MiB device array per GPU (held until the process ends) for
+ * its mask, schedule, per-frame tables and partial sums.  The result is
+ * bit for bit the same, except where nise_absorption_batched goes through
+ * per-frame propagators that here would take many windows of the array, one
+ * after the other: such a run takes the row conveyor (within 1.5e-5).
  * Runs needing more return NISE_ERR_RANGE with a message.  No hipMalloc /
  * hipFree, no stream or event is created (null stream, synchronous copies;
  * re_S / im_S are host arrays).  Calls on one GPU share the array: they are
@@ -417,9 +420,12 @@ typedef struct {
 
 /* Absorption of nsys independent systems of uneven size (no counterpart in
  * the reference; each system is what nise_absorption_batched computes).
- * Systems with propagation 1 share one row-conveyor launch; systems with
- * propagation 0 (exact exponential) and N <= 64 share one dense-propagator
- * launch fed by per-frame propagators from the batched Jacobi solver.
+ * Systems with propagation 1 share one row-conveyor launch, chains of nearest
+ * neighbours one of their own; those that the whole batch's time favours go
+ * through per-frame propagators (so a system's result may differ from its
+ * plan's by their rounding).  Systems with propagation 0 (exact exponential)
+ * and N <= 64 go through per-frame propagators from the FP64 matrix
+ * exponential, one launch per size class.
  * re_S / im_S (host) receive each system's tmax1 values, systems one after
  * another.  done_ms (host, nsys, optional) receives each system's
  * completion time in ms after the first workgroup of the run started
@@ -428,9 +434,9 @@ int nise_absorption_multi(const nise_system *systems, int nsys, int where,
                           float *re_S, float *im_S, double *done_ms);
 
 /* Autotuner of the multi-system batch: runs the batch once, then times it
- * with each system's own row count (the power of two nearest its mean layer
- * width, up to 32: code 0; up to 16 or 64: codes -16, -64) and with every
- * common row count of the row conveyor (1, 2, 4, ..., 64; best of two runs,
+ * with each system's own choice (its row count, where it takes the conveyor,
+ * the power of two nearest its mean layer width, up to 32: code 0; up to 16 or
+ * 64: codes -16, -64) and with every common row count of the row conveyor (1, 2, 4, ..., 64; best of two runs,
  * counts the batch cannot take skipped) and keeps the fastest for later
  * nise_absorption_multi calls of this thread on a batch of the same shape
  * (per system N, tmax, samples, spacing, scheme, Trotter steps); without it

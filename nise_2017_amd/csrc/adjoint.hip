@@ -143,9 +143,10 @@ __global__ void __launch_bounds__(64) adjoint_kernel(AdjArgs A) {
   if (t == 0) A.part_c[g] = cg;
 }
 
-// out[i] = sum over the workgroups of gradient i (i < N: offsets, N: scale),
-// one wave each in a fixed order; read across i by the lanes of 16 (a thread
-// per i walking all partials took 0.1 ms for a thousand workgroups).
+// out[i] = sum over the workgroups of gradient i (i < N: offsets, N: scale) in
+// a fixed order: 16 threads per i take every 16th workgroup, and 16 neighbouring
+// i are read together (a thread per i walking all partials took 0.1 ms for a
+// thousand workgroups).
 constexpr int kAdjRedX = 16, kAdjRedY = 16;
 __global__ void __launch_bounds__(kAdjRedX * kAdjRedY) adjoint_reduce_kernel(const double *pd, const double *pc, int nwg,
                                                                             int N, double *out) {

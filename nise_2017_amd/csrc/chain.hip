@@ -16,9 +16,9 @@
 // phase D_j, (cos, sin) and f J of the pair (j - 1, j), and the dipoles of j;
 // a lane reads its records in order, kAhead steps before their use, and the
 // lanes of a wave cover R frames, so the records' 128-byte lines are used from
-// L1.  What bounds it is the instruction issue of a lone wave (about 110
-// instructions a step forward, 190 backward) times tmax / R (N + 1) steps: a
-// thousand samples are one wave per SIMD.  Measured, with tables and sums
+// L1.  What bounds it is the instruction issue of a lone wave (about 100
+// instructions a step forward, 200 backward, 7 cycles each) times tmax / R (N + 1)
+// steps: a thousand samples are one wave per SIMD.  Measured, with tables and sums
 // (N = 128, 1,000 samples of 256 steps): forward 6.14 ms in the row conveyor,
 // 0.68 here; backward 14.4 and 0.84 ms.  N = 16, 200 samples of 128 steps: 0.45
 // and 0.145 ms (0.128 through propagators, dense.hip, whose rounding differs

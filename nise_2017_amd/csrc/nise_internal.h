@@ -450,8 +450,8 @@ int launch_rows_u(const RowsArgs &a, int R, int64_t nfr, float2 *U, hipStream_t 
 int launch_rows(const RowsArgs *sys, const int2 *wmap, int nwg, int R, bool pf, size_t smem, hipStream_t st,
                 unsigned long long *times = nullptr);
 
-// Dense-propagator vectors (dense.hip): one descriptor per system, one wave
-// per vector (vector v = 3 s + x as in RowsArgs).
+// Dense-propagator vectors (dense.hip): one descriptor per system (vector v =
+// 3 s + x as in RowsArgs).
 struct DiaSys {
   int N = 0, tmax = 0, begin = 0, sample = 1, nvec = 0;
   int64_t f_lo = 0;

@@ -2,8 +2,10 @@
 //
 // nise_absorption_batched_noalloc computes what nise_absorption_batched
 // computes for device-resident records and the Trotter scheme, with the same
-// schedule, tables and kernels (row conveyor of the default shape), so the
-// two agree bit for bit.  Every device buffer the run needs beyond its inputs
+// schedule, tables and kernels, so the two agree bit for bit; where chains or
+// propagators need windows of the array and those take longer, with the row
+// conveyor of the default shape (the chains' bits, not the propagators').  Every
+// device buffer the run needs beyond its inputs
 // and outputs (the coupling mask, the row schedule and its step table, the
 // per-frame phase and rotation tables, the system descriptor and workgroup
 // map, the per-vector partial responses and the reduced response) is carved

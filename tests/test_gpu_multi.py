@@ -1,6 +1,6 @@
 """GPU parity of the multi-system batch (nise_absorption_multi): systems of
 uneven N in one row-conveyor launch, exact-exponential (DIA) systems in the
-DIA-conveyor launch, each against the oracle on the same inputs.
+dense-propagator launches, each against the oracle on the same inputs.
 
 Tolerances: Trotter systems 1e-5 relative L2 against the FP32 oracle (the
 propagation is the reference's operation order; sums are FP64 here);
