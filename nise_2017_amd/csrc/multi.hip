@@ -868,15 +868,15 @@ static int multi_run(const nise_system *systems, int nsys, int where, float *re_
   // beside the row conveyor on the second stream, after their tables: the
   // chains, and the Trotter systems' propagators (without a conveyor these
   // stay on the first stream, beside the DIA systems)
-  const bool shared = !rmap.empty() && dend[1][3] > dend[0][3];
-  if (!cmap.empty() || shared) {
+  const bool shared = !rmap.empty() && (!cmap.empty() || dend[1][3] > dend[0][3]);
+  if (shared) {
     hipEvent_t ev;
     NISE_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     hipError_t e1 = hipEventRecord(ev, st), e2 = e1 == hipSuccess ? hipStreamWaitEvent(sd, ev, 0) : e1;
     (void)hipEventDestroy(ev);
     NISE_HIP_CHECK(e2);
   }
-  if ((rc = launch_chain_batch(chains, csys.as<ChainArgs>(), cwm.as<int2>(), (int)cmap.size(), sd,
+  if ((rc = launch_chain_batch(chains, csys.as<ChainArgs>(), cwm.as<int2>(), (int)cmap.size(), shared ? sd : st,
                                tm + 2 * (rmap.size() + dmap.size()))))
     return rc;
   if (!rmap.empty() && (rc = launch_rows(rsys.as<RowsArgs>(), rwm.as<int2>(), (int)rmap.size(), R, rpf, rsmem, st, tm)))
